@@ -75,7 +75,7 @@ struct ffs_plan {
   int32_t V[3] = {1, 1, 1};
   int64_t t = 0, t_tail = 0, nblocks = 0;
   int64_t tiles[3] = {1, 1, 1};
-  int64_t pairs = 0;
+  int64_t units = 0;  // work units of one block: tiles (32-point FP64 family) or tile pairs
   int32_t h_main[3] = {0, 0, 0}, h_tail[3] = {0, 0, 0};
   void* d_opsi = nullptr;  // 32-point family with V <= 16: inverse operands of the main and tail depths
   double* d_ops = nullptr;
@@ -87,7 +87,7 @@ struct ffs_plan {
   double* d_taps = nullptr;
   double* d_scratch = nullptr;  // ping-pong grid
   int64_t npoints = 0;
-  int64_t hlen = 0;
+  int64_t hlen = 0;    // complex spectrum values per depth (transform families)
   hipStream_t cap_stream = nullptr;
   // Captured block chains for the last few (d_in, d_out) pairs, least recently used replaced first.
   struct GraphSlot {
@@ -235,6 +235,12 @@ ffs_status choose_config_direct(ffs_plan* pl) {
   return FFS_OK;
 }
 
+// 32-point FP64 tiles run the real half-sample transforms: one real tile per work unit, operand and filter
+// tables of their own (ffsk::gen_operands_real, gen_spectrum_real).
+bool real_tiles(const ffs_plan* pl) {
+  return pl->kind == ffsk::KIND_2D32 && pl->prob.precision == FFS_PREC_FP64;
+}
+
 // Choose tile family, fused depth and valid widths.
 ffs_status choose_config(ffs_plan* pl) {
   const ffs_problem& p = pl->prob;
@@ -288,11 +294,12 @@ ffs_status choose_config(ffs_plan* pl) {
     if (tmax < 1 || (p.fuse > 0 && p.fuse > tmax)) return -1.0;
     double compute = p.precision == FFS_PREC_FP64 ? 4700.0 : (p.precision == FFS_PREC_MIXED_F32 ? 2600.0 : 2500.0);
     // 32-point pairs (full stages; SIMD cycles per pair from GRBM_GUI_ACTIVE of the reduced-stage kernels
-    // on Box2D25P 8192^2, divided by their factor below): FP16 5550 / 0.63, BF16 8000 / 0.70
+    // on Box2D25P 8192^2, divided by their factor below): FP16 5550 / 0.63, BF16 8000 / 0.70, FP64 (two real
+    // tiles) 10100 / 0.74
     if (kind == ffsk::KIND_2D32)
       compute = p.precision == FFS_PREC_MIXED_BF16 ? 12000.0
                 : p.precision == FFS_PREC_MIXED_F16 ? 8800.0
-                : p.precision == FFS_PREC_FP64     ? 31000.0  // 384 FP64 MFMAs per pair
+                : p.precision == FFS_PREC_FP64     ? 13700.0  // 128 FP64 MFMAs per two tiles
                                                    : 9000.0;
     // 32-point family with V <= 16: reduced inverse stages, measured at 0.63 (FP16), 0.70 (BF16) and
     // 0.74 (FP64) of a full tile pair on MI355X
@@ -353,7 +360,7 @@ ffs_status choose_config(ffs_plan* pl) {
     pl->h_main[1] = (int32_t)(hi * pl->t);
     pl->h_tail[1] = (int32_t)(hi * pl->t_tail);
     pl->tiles[1] = (p.sizes[0] + pl->V[1] - 1) / pl->V[1];
-    pl->pairs = (pl->tiles[1] + 1) / 2;
+    pl->units = (pl->tiles[1] + 1) / 2;
   } else {
     for (int d = 0; d < p.dims; d++) {
       pl->V[d] = (int32_t)(Pmain - 2 * r * pl->t);
@@ -361,8 +368,8 @@ ffs_status choose_config(ffs_plan* pl) {
       pl->h_tail[d] = (int32_t)(hi * pl->t_tail);
       pl->tiles[d] = (p.sizes[d] + pl->V[d] - 1) / pl->V[d];
     }
-    if (p.dims == 2) pl->pairs = pl->tiles[0] * ((pl->tiles[1] + 1) / 2);
-    if (p.dims == 3) pl->pairs = pl->tiles[0] * pl->tiles[1] * ((pl->tiles[2] + 1) / 2);
+    if (p.dims == 2) pl->units = pl->tiles[0] * (real_tiles(pl) ? pl->tiles[1] : (pl->tiles[1] + 1) / 2);
+    if (p.dims == 3) pl->units = pl->tiles[0] * pl->tiles[1] * ((pl->tiles[2] + 1) / 2);
   }
   return FFS_OK;
 }
@@ -412,7 +419,7 @@ ffsk::TileArgs make_args(const ffs_plan* pl, const double* src, double* dst, boo
   a.src = src;
   a.dst = dst;
   a.ops = pl->d_ops;
-  a.H = pl->d_H + (tail ? 2 * pl->hlen : 0);
+  a.H = pl->d_H + (tail ? (real_tiles(pl) ? ffsk::kSpecReal : 2 * pl->hlen) : 0);
   a.Hf = pl->d_Hf ? pl->d_Hf + (tail ? 2 * pl->hlen : 0) : nullptr;
   a.opsm = pl->d_opsm;
   a.unit = 1.0f;
@@ -430,7 +437,7 @@ ffsk::TileArgs make_args(const ffs_plan* pl, const double* src, double* dst, boo
   a.tiles0 = pl->tiles[0];
   a.tiles1 = pl->tiles[1];
   a.tiles2 = pl->tiles[2];
-  a.pairs = pl->pairs;
+  a.units = pl->units;
   a.V0 = pl->V[0];
   a.V1 = pl->V[1];
   a.V2 = pl->V[2];
@@ -442,11 +449,8 @@ ffsk::TileArgs make_args(const ffs_plan* pl, const double* src, double* dst, boo
   a.scale_exp = tail ? pl->scale_tail : pl->scale_main;
   a.linear_map = linear_map(pl) ? 1 : 0;
   a.out16 = out16_block(pl) ? 1 : 0;
-  if (a.out16) {
-    const size_t per = pl->prob.precision == FFS_PREC_FP64 ? sizeof(double) * ffsk::kInv32F64
-                                                            : sizeof(uint32_t) * ffsk::kInv32Words;
-    a.opsi = static_cast<const char*>(pl->d_opsi) + (tail ? per : 0);
-  }
+  if (a.out16 && pl->d_opsi)
+    a.opsi = static_cast<const char*>(pl->d_opsi) + (tail ? sizeof(uint32_t) * ffsk::kInv32Words : 0);
   return a;
 }
 
@@ -613,7 +617,8 @@ ffs_status plan_constants(ffs_plan* pl) {
 struct TableSizes {
   size_t ops, opsm, H, Hf, opsi, taps;
 };
-TableSizes table_sizes(const ffs_plan* pl) {
+// The DFT tables (complex operands and spectrum) of the plan's family and precision.
+TableSizes dft_table_sizes(const ffs_plan* pl) {
   TableSizes t{};
   if (pl->direct) return t;
   t.ops = sizeof(double) * std::max(ffsk::kOpsLen, ffsk::kOps32F64);
@@ -624,9 +629,31 @@ TableSizes table_sizes(const ffs_plan* pl) {
   t.taps = sizeof(double) * pl->weights.size();
   return t;
 }
+// The tables the plan's kernels read.
+TableSizes table_sizes(const ffs_plan* pl) {
+  TableSizes t = dft_table_sizes(pl);
+  if (!pl->direct && real_tiles(pl)) {
+    t.ops = sizeof(double) * ffsk::kOpsReal;
+    t.H = sizeof(double) * 2 * ffsk::kSpecReal;
+    t.opsi = 0;
+  }
+  return t;
+}
 
-// DFT operands and spectra into the plan's device tables, on stream s (the taps are already in d_taps).
-hipError_t plan_tables(ffs_plan* pl, hipStream_t s) {
+// Operands and spectra into the plan's device tables, on stream s (the taps are already in d_taps).
+hipError_t dft_tables(const ffs_plan* pl, hipStream_t s);
+hipError_t plan_tables(const ffs_plan* pl, hipStream_t s) {
+  if (!real_tiles(pl)) return dft_tables(pl, s);
+  const ffs_problem& p = pl->prob;
+  const int K = 2 * p.radius + 1;
+  hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
+  if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);
+  if (e == hipSuccess && pl->t_tail > 0)
+    e = ffsk::gen_spectrum_real(pl->d_H + ffsk::kSpecReal, 32, pl->d_taps, K, p.convention, pl->t_tail, s);
+  return e;
+}
+// The DFT tables of the plan's family (complex operands, spectrum of the cyclic DFT, inverse operands).
+hipError_t dft_tables(const ffs_plan* pl, hipStream_t s) {
   const ffs_problem& p = pl->prob;
   const int K = 2 * p.radius + 1;
   hipError_t e = hipSuccess;
@@ -913,14 +940,15 @@ ffs_status ffs_plan_get_info(const ffs_plan* pl, ffs_plan_info* info) {
   // 3D: the last inverse stage (phase 3) runs only the V0 slices of the valid block, not all 16
   if (pl->kind == ffsk::KIND_3D16) per_pair = (5.0 * 16.0 + std::min(16, pl->V[0])) * per_cplx;
   // 32-point family: output blocks over the 4 stages (4 + 4 + 4 + 4, or 4 + 4 + 2 + 1 for an out16 main
-  // block) x 4 real GEMMs x (6, 4 or 3) K=32 MFMAs
-  if (pl->kind == ffsk::KIND_2D32 && p.precision == FFS_PREC_FP64)  // x 3 Gauss GEMMs x 8 K=4 chunks
-    per_pair = (out16_block(pl) ? 11.0 : 16.0) * 3.0 * 8.0 * 2.0 * 16 * 16 * 4;
+  // block) x 4 real GEMMs x (6, 4 or 3) K=32 MFMAs; FP64: per real tile, 16 K=4 MFMAs a stage, 8 in the
+  // last one of an out16 block
+  if (real_tiles(pl))
+    per_pair = (out16_block(pl) ? 56.0 : 64.0) * 2.0 * 16 * 16 * 4;
   else if (pl->kind == ffsk::KIND_2D32)
     per_pair = (out16_block(pl) ? 11.0 : 16.0) * 4.0 *
                (p.precision == FFS_PREC_MIXED_BF16 ? 6.0 : (p.precision == FFS_PREC_MIXED_F16 ? 3.0 : 4.0)) *
                2.0 * 16 * 16 * 32;
-  info->flops_per_block = per_pair * (double)pl->pairs;
+  info->flops_per_block = per_pair * (double)pl->units;
   info->bytes_per_block = 16.0 * (double)pl->npoints;
   return FFS_OK;
 }
@@ -929,9 +957,11 @@ ffs_status ffs_plan_read_table(const ffs_plan* pl, int32_t which, void* host_out
                                int64_t* bytes) {
   if (!pl) return fail(FFS_ERR_INVALID_ARG, "plan is NULL");
   if (pl->direct) return fail(FFS_ERR_UNSUPPORTED, "the direct algorithm has no transform tables");
-  const TableSizes ts = table_sizes(pl);
+  const TableSizes ts = dft_table_sizes(pl);
   const void* src = nullptr;
   size_t n = 0;
+  // Real half-sample plans keep other tables: theirs is generated into temporary memory below.
+  const bool own = !real_tiles(pl);
   switch (which) {
     case FFS_TABLE_OPS: src = pl->d_ops; n = ts.ops; break;
     case FFS_TABLE_OPS_MIXED: src = pl->d_opsm; n = ts.opsm; break;
@@ -940,10 +970,35 @@ ffs_status ffs_plan_read_table(const ffs_plan* pl, int32_t which, void* host_out
     default: return fail(FFS_ERR_INVALID_ARG, "unknown table %d", which);
   }
   if (bytes) *bytes = (int64_t)n;
-  if (!src || n == 0) return fail(FFS_ERR_UNSUPPORTED, "this plan has no table %d", which);
+  if ((own && !src) || n == 0) return fail(FFS_ERR_UNSUPPORTED, "this plan has no table %d", which);
   if (!host_out) return FFS_OK;  // size query
   if (capacity < (int64_t)n) return fail(FFS_ERR_INVALID_ARG, "capacity %lld < %zu bytes", (long long)capacity, n);
   FFS_HIP(hipSetDevice(pl->dev));
+  if (!own) {
+    char* tmp = nullptr;
+    if (hipMalloc(&tmp, ts.ops + ts.H + ts.opsi) != hipSuccess)
+      return fail(FFS_ERR_OUT_OF_MEMORY, "device allocation failed");
+    ffs_plan dft;  // the same plan over temporary DFT tables; owns nothing
+    dft.prob = pl->prob;
+    dft.kind = pl->kind;
+    dft.t = pl->t;
+    dft.t_tail = pl->t_tail;
+    dft.hlen = pl->hlen;
+    std::memcpy(dft.L, pl->L, sizeof dft.L);
+    std::memcpy(dft.V, pl->V, sizeof dft.V);
+    std::memcpy(dft.h_main, pl->h_main, sizeof dft.h_main);
+    std::memcpy(dft.h_tail, pl->h_tail, sizeof dft.h_tail);
+    dft.d_taps = pl->d_taps;
+    dft.d_ops = reinterpret_cast<double*>(tmp);
+    dft.d_H = reinterpret_cast<double*>(tmp + ts.ops);
+    dft.d_opsi = ts.opsi ? tmp + ts.ops + ts.H : nullptr;
+    hipError_t e = dft_tables(&dft, nullptr);
+    const void* at = which == FFS_TABLE_OPS ? (void*)dft.d_ops : which == FFS_TABLE_SPECTRUM ? (void*)dft.d_H : dft.d_opsi;
+    if (e == hipSuccess) e = hipMemcpy(host_out, at, n, hipMemcpyDeviceToHost);
+    (void)hipFree(tmp);
+    if (e != hipSuccess) return fail(FFS_ERR_HIP, "table generation failed: %s", hipGetErrorString(e));
+    return FFS_OK;
+  }
   FFS_HIP(hipMemcpy(host_out, src, n, hipMemcpyDeviceToHost));
   return FFS_OK;
 }
@@ -1360,7 +1415,7 @@ ffs_status ffs_batch_run(ffs_batch* b, const double* const* d_in, double* const*
         const bool tail = (r == nb - 1) && pl->t_tail > 0;
         items[(size_t)(r * n + k)] = make_args(pl, src, dst, tail);
         prefix[(size_t)(r * (n + 1) + k)] = acc;
-        acc += pl->pairs;
+        acc += pl->units;
         k++;
       }
       prefix[(size_t)(r * (n + 1) + k)] = acc;

@@ -58,7 +58,7 @@ struct TileArgs {
   const uint32_t* opsm;  // mixed-form operand table (kOpsMixedLen words)
   int64_t n0, n1, n2;       // grid sides (unused axes = 1); 1D uses n1
   int64_t tiles0, tiles1, tiles2;
-  int64_t pairs;            // tile pairs in the block
+  int64_t units;            // work units of the block: tiles (32-point FP64 family) or tile pairs
   int32_t V0, V1, V2;       // valid widths
   int32_t h0, h1, h2;       // window start offset (valid region starts at h in the window)
   int32_t precision;
@@ -105,6 +105,13 @@ hipError_t launch_direct(const DirectArgs& a, int dims, int radius, bool star, h
 hipError_t gen_operands(double* ops, uint32_t* opsm, const int32_t* axis_len, hipStream_t s);
 hipError_t gen_operands32(uint32_t* ops32, bool f16, hipStream_t s);
 hipError_t gen_operands32_f64(double* ops, hipStream_t s);
+// Tables of the real half-sample transforms (the 32-point FP64 kernels): kOpsReal operand doubles, and the
+// filter of one depth, 4 doubles per (k0, k1) in kernel order.
+constexpr int kOpsReal = 2 * 4 * kLanes;
+constexpr int kSpecReal = 4 * 16 * 16;
+hipError_t gen_operands_real(double* ops, hipStream_t s);
+hipError_t gen_spectrum_real(double* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
+                             hipStream_t s);
 // Inverse operands of an out16 block, output column j <- window column (j + shift) mod 32:
 //   mixed forms: u4 per lane, [arr: R, I, NI][term 0..2][lane] (the kOps32Words entries of block Kb = 0);
 //   FP64: [R][chunk v][arr: Fr, -(Fr + Fi), Fi - Fr][lane] doubles (the kOps32F64 entries of block Kb = 0).

@@ -268,16 +268,16 @@ __global__ __launch_bounds__(256) void k_tile16_f64(TileArgs a) {
   };
 
   int64_t tp = gw;
-  if (tp >= a.pairs) return;
+  if (tp >= a.units) return;
   PairCoord pc = pair_coord<KIND>(a, tp);
   double xr[4], xi[4];
   gather_pair<KIND>(a, pc, q, j, xr, xi);
-  for (; tp < a.pairs; tp += W) {
+  for (; tp < a.units; tp += W) {
     // 2D: prefetch the next pair while this one computes
     const int64_t tn = tp + W;
     PairCoord pn = pc;
     double nr[4] = {0.0, 0.0, 0.0, 0.0}, ni[4] = {0.0, 0.0, 0.0, 0.0};
-    if (tn < a.pairs) {
+    if (tn < a.units) {
       pn = pair_coord<KIND>(a, tn);
       if (!ONE_D) gather_pair<KIND>(a, pn, q, j, nr, ni);
     }
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256) void k_tile16_f64(TileArgs a) {
 
     pc = pn;
     if (ONE_D) {
-      if (tn < a.pairs) gather_pair<KIND>(a, pc, q, j, xr, xi);
+      if (tn < a.units) gather_pair<KIND>(a, pc, q, j, xr, xi);
     } else {
 #pragma unroll
       for (int c = 0; c < 4; c++) {
@@ -318,56 +318,94 @@ __global__ __launch_bounds__(256) void k_tile16_f64(TileArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 2D 32x32 tiles, FP64.  A 32x32 matrix is held as 4 blocks (R, C) of 16x16 in FP64-accumulator order:
-//   block b = 2R + C, lane (j + 16q), reg v  <->  M[16R + q + 4v][16C + j],
-// so register v of block (R, I) is the A operand of contraction rows 16R + 4v .. + 3 (lane (i + 16k)
-// holds M[16R + 4v + k][16I + i]) and a stage Out = Z^T F is, per output block (I, Kb), 8 chunks x 3
-// Gauss GEMMs = 24 v_mfma_f64_16x16x4f64 into three accumulators, as in the 16-point kernel.  With OUT16
-// (V <= 16) the inverse stages compute only output block 0 from the inverse operands of window columns
-// h .. h + 15: blocks (I, 0), then (0, 0).  DFT operands (24 KB), the FP64 spectrum (16 KB) and the
-// out16 inverse operands (12 KB) are staged in LDS per workgroup.
+// 2D 32x32 tiles, FP64: real half-sample transforms.
+//
+// Overlap-save keeps only outputs that no wrap-around reaches, so the cyclic DFT of the window may be
+// replaced by a negacyclic one (x[n + 32] = -x[n]).  Its frequencies w_k = pi (2k + 1)/32, k = 0..15, have
+// no DC or Nyquist term, and about the window's centre a real window has 16 cosine and 16 sine
+// coefficients per axis that are exactly two symmetric 16 x 16 real matrices:
+//   C_k = sum_{n<16} (x[n] - x[31-n]) cos th_kn,  S_k = sum_{n<16} (x[n] + x[31-n]) sin th_kn,
+//   th_kn = pi (2k+1)(2n+1)/64;   16 x[n] = sum_k S_k sin + sum_k C_k cos,  16 x[31-n] = the difference.
+// Each stage therefore folds the window halves (register adds) and multiplies by 16 x 16 matrices: 16
+// v_mfma_f64_16x16x4f64 per real tile and stage, 8 in the last one when V <= 16 (OUT16: only the output
+// rows and columns 0..15), 56 per tile in all.  The complex Gauss form on 32-point DFTs took 132 per tile
+// (264 per tile pair), at 84% of the matrix peak that bounded it.
+//
+// Layout.  A tile is 2 x 2 blocks of 16x16 in FP64-accumulator order, lane (j + 16q), reg v <-> row q + 4v,
+// column j; block index 1 of a window axis counts from the far end (position 31 - i), so the two values of
+// every fold sit in the same lane and register, in every stage.  z[R][C] (window) -> y[C][type0]
+// -> x[type0][type1] (coefficients; type 0 cosine, 1 sine) -> u[type1][half0] -> out[half0][half1].
+//
+// The filter acts on the four coefficients (cc, cs, sc, ss) of one (k0, k1) as a 4 x 4 real matrix of four
+// numbers (k_gen_spectrum_real).  The spectrum is taken for correlation taps at offsets 0..2r per step, so
+// the valid region starts at window position 0 in both index conventions.
+//
+// DFT operands: 8 doubles per lane in registers (both matrices are symmetric, so all stages share them);
+// the spectrum (8 KB) in LDS.  A work unit is one tile: 128 VGPRs, 4 waves per SIMD (the complex form held a
+// pair in 237, 2 waves).  Box2D25P / Box2D9P 8192^2, one block: 1074 -> 541 us, 70% of the FP64 matrix rate
+// (262,144 tiles x 56 MFMAs x 64 cycles = 382 us; the adds and the filter on the same pipe 45 us more);
+// Box2D9P 128^2 x 16: 27.9 -> 11.4 us (one tile's chain instead of a pair's).
 // ---------------------------------------------------------------------------------------------
-struct Blk4d {
-  d4 b[4];
+struct OpsReal {
+  double c[4], s[4];
 };
-
-// Output blocks (I, Kb), I < NI, Kb < NK, from a table holding KBS column blocks per chunk: the full
-// operands (NI = NK = KBS = 2), or for the inverse stages of an out16 tile the shifted one-block table
-// (KBS = 1): NI = 2, NK = 1, then NI = NK = 1.  Gauss form with the tables r = Fr, n = -(Fr + Fi),
-// d = Fi - Fr: k1 = (zr + zi) r is accumulated first, and both outputs chain from it (the MFMA's C input
-// is k1, its result a new accumulator), so no output additions are needed:
-//   forward  Re = k1 + zi n, Im = k1 + zr d;   inverse  Re = k1 + zi d, Im = k1 + zr n.
-template <bool INV, int NI, int NK, int KBS>
-__device__ __forceinline__ void stage32_f64(const Blk4d& zr, const Blk4d& zi, const double* __restrict__ sF, int lane,
-                                            Blk4d& outr, Blk4d& outi) {
+__device__ __forceinline__ void load_ops_real(OpsReal& o, const double* __restrict__ ops, int lane) {
 #pragma unroll
-  for (int I = 0; I < NI; I++) {
-    double sum[2][4];
-#pragma unroll
-    for (int R = 0; R < 2; R++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) sum[R][v] = zr.b[2 * R + I][v] + zi.b[2 * R + I][v];
-#pragma unroll
-    for (int Kb = 0; Kb < NK; Kb++) {
-      d4 k1 = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int R = 0; R < 2; R++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) k1 = FFS_MFMA64(sum[R][v], sF[(((R * 4 + v) * KBS + Kb) * 3) * kLanes + lane], k1);
-      d4 re = k1, im = k1;
-#pragma unroll
-      for (int R = 0; R < 2; R++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const double* f = sF + (((R * 4 + v) * KBS + Kb) * 3) * kLanes + lane;
-          const double fn = f[kLanes], fd = f[2 * kLanes];
-          re = FFS_MFMA64(zi.b[2 * R + I][v], INV ? fd : fn, re);
-          im = FFS_MFMA64(zr.b[2 * R + I][v], INV ? fn : fd, im);
-        }
-      outr.b[2 * I + Kb] = re;
-      outi.b[2 * I + Kb] = im;
-    }
+  for (int v = 0; v < 4; v++) {
+    o.c[v] = ops[v * kLanes + lane];
+    o.s[v] = ops[(4 + v) * kLanes + lane];
   }
+}
+
+typedef d4 Tile4[2][2];
+
+// Window blocks z[half][col block] -> coefficients y[col block][type]; the rows are contracted.
+__device__ __forceinline__ void fold_fwd(const Tile4& z, const OpsReal& f, Tile4& y) {
+#pragma unroll
+  for (int C = 0; C < 2; C++) {
+    const d4 a = z[0][C] - z[1][C], b = z[0][C] + z[1][C];
+    d4 oc = {0.0, 0.0, 0.0, 0.0}, os = oc;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      oc = FFS_MFMA64(a[v], f.c[v], oc);
+      os = FFS_MFMA64(b[v], f.s[v], os);
+    }
+    y[C][0] = oc;
+    y[C][1] = os;
+  }
+}
+
+// Coefficients x[type][col block] -> y[col block][half], col blocks < NC, halves < NH (the sums are the
+// same whether or not the other blocks are computed: reduced and full stages agree bitwise).
+template <int NC, int NH>
+__device__ __forceinline__ void fold_inv(const Tile4& x, const OpsReal& f, Tile4& y) {
+#pragma unroll
+  for (int C = 0; C < NC; C++) {
+    d4 oc = {0.0, 0.0, 0.0, 0.0}, os = oc;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      oc = FFS_MFMA64(x[0][C][v], f.c[v], oc);
+      os = FFS_MFMA64(x[1][C][v], f.s[v], os);
+    }
+    y[C][0] = os + oc;
+    if (NH == 2) y[C][1] = os - oc;
+  }
+}
+
+// The filter on the coefficients of one (k0, k1), h = (alpha, beta, gamma, delta) of k_gen_spectrum_real;
+// explicit FMAs, so every kernel rounds alike.
+template <typename T>
+__device__ __forceinline__ T fma_t(T a, T b, T c) {
+  if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
+  else return __builtin_fmaf(a, b, c);
+}
+template <typename T>
+__device__ __forceinline__ void filter4(T& cc, T& cs, T& sc, T& ss, T ha, T hb, T hg, T hd) {
+  const T a = cc, b = cs, c = sc, d = ss;
+  cc = fma_t(ha, a, fma_t(hb, d, fma_t(hg, c, hd * b)));
+  ss = fma_t(ha, d, fma_t(hb, a, -fma_t(hd, c, hg * b)));
+  sc = fma_t(ha, c, fma_t(hd, d, -fma_t(hb, b, hg * a)));
+  cs = fma_t(ha, b, fma_t(hg, d, -fma_t(hb, c, hd * a)));
 }
 
 // Interior windows are read through a raw buffer view based at the window's first element: one 32-bit
@@ -382,88 +420,118 @@ __device__ __forceinline__ double window_load(__amdgpu_buffer_rsrc_t r, uint32_t
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
 }
 
-// Window values of the pair in block order: x.b[2R + C][v] = window[16R + q + 4v][16C + j].
-__device__ __forceinline__ void gather32_f64(const TileArgs& a, const PairCoord& pc, int q, int j, Blk4d& xa,
-                                             Blk4d& xb) {
-  const double* __restrict__ src = a.src;
-  const int64_t rw = pc.r0 - a.h0, cwA = pc.orgA - a.h1, cwB = pc.orgB - a.h1;
-  const bool interior = rw >= 0 && rw + 32 <= a.n0 && cwA >= 0 && (pc.hasB ? cwB : cwA) + 32 <= a.n1 &&
-                        a.n1 <= (1 << 22);
-  if (interior) {
-    const double* baseA = src + rw * a.n1 + cwA;
-    const __amdgpu_buffer_rsrc_t ra = window_rsrc(baseA, true), rb = window_rsrc(baseA + a.V1, pc.hasB);
-    const uint32_t voff = ((uint32_t)q * (uint32_t)a.n1 + (uint32_t)j) * 8u;
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const uint32_t soff = ((uint32_t)(16 * (b >> 1) + 4 * v) * (uint32_t)a.n1 + 16 * (b & 1)) * 8u;
-        xa.b[b][v] = window_load(ra, voff, soff);
-        xb.b[b][v] = window_load(rb, voff, soff);
-      }
-  } else {
-#pragma unroll
-    for (int C = 0; C < 2; C++) {
-      const int64_t cA = wrap_near(cwA + 16 * C + j, a.n1);
-      const int64_t cB = wrap_near(cwB + 16 * C + j, a.n1);
-#pragma unroll
-      for (int R = 0; R < 2; R++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int64_t row = wrap_near(rw + 16 * R + q + 4 * v, a.n0) * a.n1;
-          xa.b[2 * R + C][v] = src[row + cA];
-          xb.b[2 * R + C][v] = pc.hasB ? src[row + cB] : 0.0;
-        }
-    }
+// Tile t of a 2D grid of tiles (units of the single-tile kernels): window and output origins.
+struct TilePos {
+  int64_t t0, t1;
+};
+__device__ __forceinline__ TilePos tile_pos(int64_t u, int64_t tiles1) {
+  const int64_t t0 = u / tiles1;
+  return {t0, u - t0 * tiles1};
+}
+// Advance by the same stride each time: its quotient and remainder are taken once, outside the loop.
+__device__ __forceinline__ void tile_step(TilePos& p, const TilePos& stride, int64_t tiles1) {
+  p.t0 += stride.t0;
+  p.t1 += stride.t1;
+  if (p.t1 >= tiles1) {
+    p.t1 -= tiles1;
+    p.t0++;
   }
 }
 
-// Store the valid outputs of all four blocks (window rows 16R + q + 4v, columns 16C + j).
-__device__ __forceinline__ void store32_f64(const TileArgs& a, const PairCoord& pc, int q, int j, const Blk4d& yr,
-                                            const Blk4d& yi) {
+// Window of a tile in fold order: z[R][C] holds rows q + 4v (R = 0) or 31 - (q + 4v) (R = 1), columns j or
+// 31 - j.
+__device__ __forceinline__ void gather32_f64(const TileArgs& a, const TilePos& p, int q, int j, Tile4& z) {
+  const int64_t rw = p.t0 * a.V0 - a.h0, cw = p.t1 * a.V1 - a.h1;
+  const bool interior = rw >= 0 && rw + 32 <= a.n0 && cw >= 0 && cw + 32 <= a.n1 && a.n1 <= (1 << 22);
+  if (interior) {
+    const __amdgpu_buffer_rsrc_t rs = window_rsrc(a.src + rw * a.n1 + cw, true);
+    const uint32_t n1 = (uint32_t)a.n1;
 #pragma unroll
-  for (int C = 0; C < 2; C++) {
-    const int wc = 16 * C + j;
-    const int64_t cA = pc.orgA + wc - a.h1, cB = pc.orgB + wc - a.h1;
-    const bool colok = wc >= a.h1 && wc < a.h1 + a.V1;
-    const bool okA = colok && cA < a.n1;
-    const bool okB = colok && pc.hasB && cB < a.n1;
+    for (int R = 0; R < 2; R++)
+#pragma unroll
+      for (int C = 0; C < 2; C++) {
+        const uint32_t voff = ((uint32_t)(R ? 3 - q : q) * n1 + (uint32_t)(C ? 31 - j : j)) * 8u;
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          z[R][C][v] = window_load(rs, voff, (uint32_t)(R ? 28 - 4 * v : 4 * v) * n1 * 8u);
+      }
+  } else {
 #pragma unroll
     for (int R = 0; R < 2; R++)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const int row = 16 * R + q + 4 * v;
-        const int64_t y = pc.r0 + row - a.h0;
-        if (row >= a.h0 && row < a.h0 + a.V0 && y < a.n0) {
-          double* drow = a.dst + y * a.n1;
-          if (okA) put_out(drow + cA, yr.b[2 * R + C][v]);
-          if (okB) put_out(drow + cB, yi.b[2 * R + C][v]);
-        }
+        const int i = q + 4 * v;
+        const double* row = a.src + wrap_near(rw + (R ? 31 - i : i), a.n0) * a.n1;
+#pragma unroll
+        for (int C = 0; C < 2; C++) z[R][C][v] = row[wrap_near(cw + (C ? 31 - j : j), a.n1)];
       }
   }
 }
 
-// Store of an out16 tile pair: output block 0, lane (j + 16q), reg v = valid point (q + 4v, j) (window
-// position (h0 + q + 4v, h1 + j)).
-__device__ __forceinline__ void store16_f64(const TileArgs& a, const PairCoord& pc, int q, int j, const d4& yr,
-                                            const d4& yi) {
-  const int64_t cA = pc.orgA + j, cB = pc.orgB + j;
-  const bool okA = j < a.V1 && cA < a.n1;
-  const bool okB = j < a.V1 && pc.hasB && cB < a.n1;
+// Valid outputs of the blocks out[half0][half1], half0 and half1 < NH.
+template <int NH>
+__device__ __forceinline__ void store32_f64(const TileArgs& a, const TilePos& p, int q, int j, const Tile4& out) {
+  const int64_t r0 = p.t0 * a.V0, c0 = p.t1 * a.V1;
+  const int64_t rows = min((int64_t)a.V0, a.n0 - r0), cols = min((int64_t)a.V1, a.n1 - c0);
 #pragma unroll
-  for (int v = 0; v < 4; v++) {
-    const int row = q + 4 * v;
-    const int64_t y = pc.r0 + row;
-    if (row < a.V0 && y < a.n0) {
-      double* drow = a.dst + y * a.n1;
-      if (okA) put_out(drow + cA, yr[v]);
-      if (okB) put_out(drow + cB, yi[v]);
+  for (int R = 0; R < NH; R++)
+#pragma unroll
+    for (int C = 0; C < NH; C++) {
+      const int wc = C ? 31 - j : j;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int wr = R ? 31 - (q + 4 * v) : q + 4 * v;
+        if (wr < rows && wc < cols) put_out(a.dst + (r0 + wr) * a.n1 + c0 + wc, out[R][C][v]);
+      }
     }
-  }
 }
 
-// One tile pair of the 32-point FP64 family; the spectrum comes from LDS (single-grid launch) or from
-// the item's FP64 table in global memory (batch launch).
+// One tile: the spectrum comes from LDS (single-grid launch) or from the item's table in global memory
+// (batch launch), entry v * 64 + lane = (alpha, beta, gamma, delta) of (k0 = q + 4v, k1 = j).
+template <bool OUT16>
+__device__ __forceinline__ void tile32_f64(const TileArgs& a, const TilePos& p, const d4* __restrict__ H,
+                                           const OpsReal& f, int lane, int q, int j) {
+  constexpr int NH = OUT16 ? 1 : 2;
+  Tile4 z, y;
+  __builtin_amdgcn_s_setprio(1);  // a wave that starts a tile issues its loads ahead of the others' stages (0.5-1%)
+  gather32_f64(a, p, q, j, z);
+  __builtin_amdgcn_s_setprio(0);
+  fold_fwd(z, f, y);
+  fold_fwd(y, f, z);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    const d4 h = H[v * kLanes + lane];
+    double cc = z[0][0][v], cs = z[0][1][v], sc = z[1][0][v], ss = z[1][1][v];
+    filter4(cc, cs, sc, ss, h[0], h[1], h[2], h[3]);
+    z[0][0][v] = cc;
+    z[0][1][v] = cs;
+    z[1][0][v] = sc;
+    z[1][1][v] = ss;
+  }
+  fold_inv<2, NH>(z, f, y);
+  fold_inv<NH, NH>(y, f, z);
+  store32_f64<NH>(a, p, q, j, z);
+}
+
+template <bool OUT16>
+__global__ __launch_bounds__(256, OUT16 ? 4 : 3) void k_tile32_f64(TileArgs a) {
+  __shared__ d4 sH[4 * kLanes];  // spectrum, 8 KB
+  const d4* H = reinterpret_cast<const d4*>(a.H);
+  for (int i = threadIdx.x; i < 4 * kLanes; i += blockDim.x) sH[i] = H[i];
+  const int lane = threadIdx.x & 63;
+  const int q = lane >> 4, j = lane & 15;
+  OpsReal f;
+  load_ops_real(f, a.ops, lane);
+  __syncthreads();
+  const int64_t W = (int64_t)gridDim.x * 4;
+  const int64_t gw = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  TilePos p = tile_pos(gw, a.tiles1);
+  const TilePos stride = tile_pos(W, a.tiles1);
+  for (int64_t u = gw; u < a.units; u += W, tile_step(p, stride, a.tiles1))
+    tile32_f64<OUT16>(a, p, sH, f, lane, q, j);
+}
+
 // The inverse operands of shift h (output column m <- window column (m + h) mod 32) are columns of the
 // forward operand table: lane j + 16q of column block 0 of the shifted table holds what lane
 // (c & 15) + 16q of column block c >> 4 holds in the forward one, c = (j + h) mod 32.  ShiftedView
@@ -479,61 +547,6 @@ __device__ __forceinline__ ShiftedView<T> shifted_view(const T* table, int h, in
   return {table + (c >> 4) * 3 * kLanes, (lane & 48) | (c & 15)};
 }
 
-// IKBS: column blocks per chunk of the inverse-operand table sG (1: the shifted one-block table; 2: the
-// forward operand table, read through a shifted_view whose lane is `ilane`).
-template <bool H_FROM_LDS, bool OUT16, int IKBS = 1>
-__device__ __forceinline__ void tile32_pair_f64(const TileArgs& a, int64_t tp, const double* __restrict__ sF,
-                                                const double2* __restrict__ sH, const double* __restrict__ sG,
-                                                int lane, int q, int j, int ilane = -1) {
-  const PairCoord pc = pair_coord<KIND_2D16>(a, tp);
-  Blk4d zr, zi, orr, oi;
-  gather32_f64(a, pc, q, j, zr, zi);
-  stage32_f64<false, 2, 2, 2>(zr, zi, sF, lane, orr, oi);
-  stage32_f64<false, 2, 2, 2>(orr, oi, sF, lane, zr, zi);  // Y[k0][k1], block order
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int b = 0; b < 4; b++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int e = (b * 4 + v) * kLanes + lane;
-      const double hr = H_FROM_LDS ? sH[e].x : a.H[e];
-      const double hi = H_FROM_LDS ? sH[e].y : a.H[1024 + e];
-      double yr = zr.b[b][v], yi = zi.b[b][v];
-      cmul(yr, yi, hr, hi);
-      zr.b[b][v] = yr;
-      zi.b[b][v] = yi;
-    }
-  if (OUT16) {
-    const int il = ilane < 0 ? lane : ilane;  // the lane whose inverse operands this lane reads
-    stage32_f64<true, 2, 1, IKBS>(zr, zi, sG, il, orr, oi);  // blocks 0 and 2: window rows h0 ..
-    stage32_f64<true, 1, 1, IKBS>(orr, oi, sG, il, zr, zi);  // block 0 = the valid region
-    store16_f64(a, pc, q, j, zr.b[0], zi.b[0]);
-  } else {
-    stage32_f64<true, 2, 2, 2>(zr, zi, sF, lane, orr, oi);
-    stage32_f64<true, 2, 2, 2>(orr, oi, sF, lane, zr, zi);  // X'[n0][n1], block order
-    store32_f64(a, pc, q, j, zr, zi);
-  }
-}
-
-template <bool OUT16>
-__global__ __launch_bounds__(256, 2) void k_tile32_f64(TileArgs a) {
-  __shared__ double sF[kOps32F64];           // 24 KB
-  __shared__ double2 sH[4 * 4 * kLanes];     // spectrum [block][reg][lane] (re, im), 16 KB
-  __shared__ double sG[OUT16 ? kInv32F64 : 1];  // out16 inverse operands, 12 KB
-  for (int i = threadIdx.x; i < kOps32F64; i += blockDim.x) sF[i] = a.ops[i];
-  if (OUT16)
-    for (int i = threadIdx.x; i < kInv32F64; i += blockDim.x) sG[i] = static_cast<const double*>(a.opsi)[i];
-  for (int i = threadIdx.x; i < 1024; i += blockDim.x) sH[i] = double2{a.H[i], a.H[1024 + i]};
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int q = lane >> 4, j = lane & 15;
-  const int64_t W = (int64_t)gridDim.x * 4;
-  const int64_t gw = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int64_t tp = gw; tp < a.pairs; tp += W) tile32_pair_f64<true, OUT16>(a, tp, sF, sH, sG, lane, q, j);
-}
-
-// Multi-grid launch of the FP64 form (the k_batch32_* structure): the DFT operands, the same for every
-// item, in LDS; each item's spectrum read per tile pair from its FP64 table (L2-resident).
 // Work item idx of a batch round -> grid g with prefix[g] <= idx < prefix[g + 1].  A wave takes its items in
 // increasing order, so the search starts after the grid of its previous item and most items stay in that
 // grid (no dependent scalar loads); a change costs one binary search over the later grids.  g = -1 and
@@ -550,13 +563,14 @@ __device__ __forceinline__ int batch_grid(const int64_t* __restrict__ prefix, in
   return lo;
 }
 
-__global__ __launch_bounds__(256, 2) void k_batch32_f64(const TileArgs* __restrict__ items,
+// Multi-grid launch of the FP64 form: the operands, the same for every item, in registers; each item's
+// spectrum is read per tile from its table (L2-resident).
+__global__ __launch_bounds__(256, 4) void k_batch32_f64(const TileArgs* __restrict__ items,
                                                         const int64_t* __restrict__ prefix, int32_t n) {
-  __shared__ double sF[kOps32F64];
-  for (int i = threadIdx.x; i < kOps32F64; i += blockDim.x) sF[i] = items[0].ops[i];
-  __syncthreads();
   const int lane = threadIdx.x & 63;
   const int q = lane >> 4, j = lane & 15;
+  OpsReal f;
+  load_ops_real(f, items[0].ops, lane);
   const int64_t W = (int64_t)gridDim.x * 4;
   const int64_t gw = block_order(items[0].linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t total = prefix[n];
@@ -565,12 +579,12 @@ __global__ __launch_bounds__(256, 2) void k_batch32_f64(const TileArgs* __restri
   for (int64_t idx = gw; idx < total; idx += W) {
     lo = batch_grid(prefix, n, idx, lo, next);
     const TileArgs a = items[lo];  // independent scalar loads, from the scalar cache while lo is unchanged
-    if (a.out16) {
-      const ShiftedView<double> v = shifted_view(sF, a.h1, lane);
-      tile32_pair_f64<false, true, 2>(a, idx - prefix[lo], sF, nullptr, v.base, lane, q, j, v.lane);
-    } else {
-      tile32_pair_f64<false, false>(a, idx - prefix[lo], sF, nullptr, nullptr, lane, q, j);
-    }
+    const TilePos p = tile_pos(idx - prefix[lo], a.tiles1);
+    const d4* H = reinterpret_cast<const d4*>(a.H);
+    if (a.out16)
+      tile32_f64<true>(a, p, H, f, lane, q, j);
+    else
+      tile32_f64<false>(a, p, H, f, lane, q, j);
   }
 }
 
@@ -906,25 +920,25 @@ __global__ __launch_bounds__(256) void k_tile16_mixed(TileArgs a) {
 
   // Two register sets alternate (unrolled by 2): the next pair's window loads while this one computes.
   int64_t tp = gw;
-  if (tp >= a.pairs) return;
+  if (tp >= a.units) return;
   PairCoord pa = pair_coord<KIND>(a, tp), pb = pa;
   double ar[4], ai[4], br[4] = {0.0, 0.0, 0.0, 0.0}, bi[4] = {0.0, 0.0, 0.0, 0.0};
   gather_pair_m<KIND>(a, pa, q, j, ar, ai);
   while (true) {
-    if (tp + W < a.pairs) {
+    if (tp + W < a.units) {
       pb = pair_coord<KIND>(a, tp + W);
       gather_pair_m<KIND>(a, pb, q, j, br, bi);
     }
     mixed_pair<KIND, NTERMS>(a, pa, q, j, ar, ai, f0, g1, hr, hi);
     tp += W;
-    if (tp >= a.pairs) break;
-    if (tp + W < a.pairs) {
+    if (tp >= a.units) break;
+    if (tp + W < a.units) {
       pa = pair_coord<KIND>(a, tp + W);
       gather_pair_m<KIND>(a, pa, q, j, ar, ai);
     }
     mixed_pair<KIND, NTERMS>(a, pb, q, j, br, bi, f0, g1, hr, hi);
     tp += W;
-    if (tp >= a.pairs) break;
+    if (tp >= a.units) break;
   }
 }
 
@@ -1370,7 +1384,7 @@ __global__ __launch_bounds__(256, 3) void k_tile32_bf16(TileArgs a) {
   const int q = lane >> 4, j = lane & 15;
   const int64_t W = (int64_t)gridDim.x * 4;
   const int64_t gw = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int64_t tp = gw; tp < a.pairs; tp += W) tile32_pair<NTERMS, true, OUT16>(a, tp, sF, sH, sG, lane, q, j);
+  for (int64_t tp = gw; tp < a.units; tp += W) tile32_pair<NTERMS, true, OUT16>(a, tp, sF, sH, sG, lane, q, j);
 }
 
 // Multi-grid launch: one fused block of every grid still running, as one persistent launch over the
@@ -1453,7 +1467,7 @@ __global__ __launch_bounds__(256, OUT16 ? 4 : 3) void k_tile32_f16(TileArgs a) {
   const int q = lane >> 4, j = lane & 15;
   const int64_t W = (int64_t)gridDim.x * 4;
   const int64_t gw = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int64_t tp = gw; tp < a.pairs; tp += W) tile32_pair_f16<true, OUT16>(a, tp, sF, sH, sG, lane, q, j);
+  for (int64_t tp = gw; tp < a.units; tp += W) tile32_pair_f16<true, OUT16>(a, tp, sF, sH, sG, lane, q, j);
 }
 
 __global__ __launch_bounds__(256, 3) void k_batch32_f16(const TileArgs* __restrict__ items,
@@ -1478,7 +1492,7 @@ __global__ __launch_bounds__(256, 3) void k_batch32_f16(const TileArgs* __restri
 
 hipError_t launch_batch(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision, hipStream_t s,
                         int num_cus) {
-  const dim3 g((unsigned)num_cus * (precision == 0 ? 2 : 3)), b(256);
+  const dim3 g((unsigned)num_cus * (precision == 0 ? 4 : 3)), b(256);
   if (precision == 0)
     hipLaunchKernelGGL(k_batch32_f64, g, b, 0, s, d_items, d_prefix, n);
   else if (precision == PREC_BF16)
@@ -1637,8 +1651,8 @@ __global__ __launch_bounds__(256) void k_tile3d(TileArgs a) {
   double va[16], vb[16];
   int64_t tp = block_order(a.linear_map, blockIdx.x, gridDim.x);
   Win3 g = win3(a, tp);
-  if (tp < a.pairs) load3(a, g, fy, fz, va, vb);
-  for (; tp < a.pairs; tp += gridDim.x) {
+  if (tp < a.units) load3(a, g, fy, fz, va, vb);
+  for (; tp < a.units; tp += gridDim.x) {
     if (!PREFETCH) load3(a, g, fy, fz, va, vb);
     const Win3 cur = g;
     const int64_t o0 = cur.o0, o1 = cur.o1, o2A = cur.o2A, o2B = cur.o2B;
@@ -1659,7 +1673,7 @@ __global__ __launch_bounds__(256) void k_tile3d(TileArgs a) {
     }
     __syncthreads();
     const int64_t tn = tp + gridDim.x;
-    if (tn < a.pairs) {
+    if (tn < a.units) {
       g = win3(a, tn);
       if (PREFETCH) load3(a, g, fy, fz, va, vb);
     }
@@ -2043,6 +2057,85 @@ __global__ void k_gen_spectrum(double* H, int kind, int layout, int32_t L0, int3
   H[len + e] = zero ? 0.0 : ki;
 }
 
+// Operands of the real half-sample transforms: [cos, sin][chunk v][lane], lane (j + 16k) holding entry
+// (4 v + k, j) of cos / sin (pi (2a + 1)(2b + 1)/64).
+__global__ void k_gen_operands_real(double* t) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= kOpsReal) return;
+  const int lane = idx % kLanes, v = (idx / kLanes) % 4, sine = idx / (4 * kLanes);
+  const int m = ((2 * (4 * v + (lane >> 4)) + 1) * (2 * (lane & 15) + 1)) % 128;
+  double s, c;
+  sincospi((double)m / 64.0, &s, &c);
+  t[idx] = sine ? s : c;
+}
+
+// Filter of the real half-sample transforms on a 2D window of P points per axis.  With correlation taps
+// g[e], e in [0, 2r]^2 (ref: e = 2r - a; centred: e = a), the complex coefficient F = C - i S of one
+// frequency pair is multiplied by L = (sum g[e] exp(i (w0 e0 + w1 e1)))^t, w_k = pi (2k + 1)/P.  With
+// L1 = L(w0, w1), L2 = L(w0, -w1): alpha = Re(L1 + L2)/2, beta = Re(L2 - L1)/2, gamma = Im(L1 + L2)/2,
+// delta = Im(L1 - L2)/2 give
+//   cc' =  alpha cc + beta ss + gamma sc + delta cs,   ss' =  alpha ss + beta cc - delta sc - gamma cs,
+//   sc' =  alpha sc - beta cs - gamma cc + delta ss,   cs' =  alpha cs - beta sc + gamma ss - delta cc
+// (c and s: cosine and sine along axis 0, then axis 1).  The transforms' 4/P^2 is folded in.
+// The entry order is the family's: FP64 32-point, entry v * 64 + lane <-> (q + 4v, j).
+__device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
+  double pr = 1.0, pi = 0.0, br = kr, bi = ki;
+  for (int64_t n = t; n > 0; n >>= 1) {
+    if (n & 1) {
+      const double tr = pr * br - pi * bi;
+      pi = pr * bi + pi * br;
+      pr = tr;
+    }
+    const double tr = br * br - bi * bi;
+    bi = 2.0 * br * bi;
+    br = tr;
+  }
+  kr = pr;
+  ki = pi;
+}
+__global__ void k_gen_spectrum_real(double* H, int32_t P, const double* taps, int32_t K, int32_t convention,
+                                    int64_t t) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= 4 * kLanes) return;
+  const int lane = e % kLanes, v = e / kLanes;
+  const int k0 = (lane >> 4) + 4 * v, k1 = lane & 15;
+  double L1r = 0.0, L1i = 0.0, L2r = 0.0, L2i = 0.0;
+  for (int a0 = 0; a0 < K; a0++)
+    for (int a1 = 0; a1 < K; a1++) {
+      const double w = taps[a0 * K + a1];
+      if (w == 0.0) continue;
+      const int e0 = convention == 0 ? K - 1 - a0 : a0, e1 = convention == 0 ? K - 1 - a1 : a1;
+      const int64_t x0 = (int64_t)(2 * k0 + 1) * e0, x1 = (int64_t)(2 * k1 + 1) * e1;
+      const int64_t m1 = (x0 + x1) % (2 * P);
+      const int64_t m2 = (((x0 - x1) % (2 * P)) + 2 * P) % (2 * P);
+      double s, c;
+      sincospi((double)m1 / (double)P, &s, &c);
+      L1r += w * c;
+      L1i += w * s;
+      sincospi((double)m2 / (double)P, &s, &c);
+      L2r += w * c;
+      L2i += w * s;
+    }
+  cpow_t(L1r, L1i, t);
+  cpow_t(L2r, L2i, t);
+  const double norm = 0.5 * 4.0 / ((double)P * (double)P);
+  H[4 * e + 0] = (L1r + L2r) * norm;
+  H[4 * e + 1] = (L2r - L1r) * norm;
+  H[4 * e + 2] = (L1i + L2i) * norm;
+  H[4 * e + 3] = (L1i - L2i) * norm;
+}
+
+hipError_t gen_operands_real(double* ops, hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_operands_real, dim3(kOpsReal / 256), dim3(256), 0, s, ops);
+  return hipGetLastError();
+}
+
+hipError_t gen_spectrum_real(double* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_spectrum_real, dim3(4), dim3(64), 0, s, H, P, d_taps, K, convention, t);
+  return hipGetLastError();
+}
+
 struct TapChunk {
   double w[kTapsPerLaunch];
   int32_t n;
@@ -2144,9 +2237,9 @@ void launch16(const TileArgs& a, int64_t blocks, int num_cus, hipStream_t s) {
 }
 
 hipError_t launch_block(const TileArgs& a, int kind, hipStream_t s, int num_cus) {
-  if (a.pairs <= 0) return hipSuccess;
+  if (a.units <= 0) return hipSuccess;
   if (kind == KIND_3D16) {  // one workgroup per tile pair, two resident per CU (68 KB LDS each for FP64)
-    const int64_t blocks3 = std::min<int64_t>(a.pairs, (int64_t)num_cus * (a.precision == 0 ? 2 : 3));
+    const int64_t blocks3 = std::min<int64_t>(a.units, (int64_t)num_cus * (a.precision == 0 ? 2 : 3));
     const dim3 g3((unsigned)blocks3), b3(256);
     if (a.precision == PREC_BF16)
       hipLaunchKernelGGL((k_tile3d<PREC_BF16, 3>), g3, b3, 0, s, a);
@@ -2158,12 +2251,12 @@ hipError_t launch_block(const TileArgs& a, int kind, hipStream_t s, int num_cus)
       return hipErrorInvalidValue;
     return hipGetLastError();
   }
-  const int64_t waves_needed = a.pairs;
+  const int64_t waves_needed = a.units;
   int64_t blocks = (waves_needed + 3) / 4;
   // 8 workgroups (32 waves) per CU at most, grid-stride beyond; the 32-point kernels stage their tables
   // in LDS per workgroup and run 3 waves per SIMD (4 for the FP16 out16 kernel), so they launch exactly
   // the resident workgroups.
-  const int64_t per_cu32 = (a.precision == PREC_F16 && a.out16) ? 4 : (a.precision == 0 ? 2 : 3);
+  const int64_t per_cu32 = a.out16 && (a.precision == PREC_F16 || a.precision == 0) ? 4 : 3;
   const int64_t cap = (int64_t)num_cus * (kind == KIND_2D32 ? per_cu32 : 8);
   if (blocks > cap) blocks = cap;
   const dim3 g((unsigned)blocks), b(256);

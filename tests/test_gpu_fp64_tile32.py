@@ -81,3 +81,22 @@ def test_2d_tile32_long_rows(ffs, oracle, torch_cuda, n1, precision):
     ref = oracle.sweep(x, r, w, 3)
     tol = TOL_FP64 if precision == "fp64" else 1e-6
     assert oracle.errors(got, ref)[1] <= tol, (precision, n1, info)
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,fuse,size", [(0, 3, (65, 31)), (15, 1, (9, 40)), (7, 1, (35, 37)), (5, 2, (25, 24)),
+                                              (1, 15, (3, 130)), (2, 4, (17, 15)), (2, 4, (16, 272)), (1, 1, (31, 61))])
+def test_2d_fp64_tile32_edges(ffs, oracle, torch_cuda, convention, radius, fuse, size):
+    # The real half-sample transforms at the ends of their range: every position valid (V = 32), V = 2, V = 18
+    # (one column past the reduced block), the widest shift of the filter (radius 15), signed taps, and
+    # grids one short of, equal to and one past a tile.
+    rng = np.random.default_rng(31 * radius + fuse)
+    w = rng.standard_normal((2 * radius + 1) ** 2)
+    w /= np.abs(w).sum()
+    x = oracle.uniform(9 + radius, size)
+    got, info = _run(ffs, torch_cuda, x, radius, w, fuse, tile=32, fuse=fuse, convention=convention)
+    assert info["tile"][:2] == [32, 32] and info["valid"][0] == 32 - 2 * radius * fuse
+    ref = oracle.sweep(x, radius, w, fuse, convention=0 if convention == "ref" else 1)
+    # against the input's size: taps of |sum| 1 in absolute value keep |out| <= max |in|, and a few hundred FP64
+    # roundings of values that large stay far below 1e-13
+    assert np.abs(got - ref).max() <= 1e-13 * np.abs(x).max(), (convention, radius, fuse, info)
