@@ -82,6 +82,13 @@ struct ffs_plan {
   uint32_t* d_opsm = nullptr;  // mixed-form operand table
   double* d_H = nullptr;       // [main | tail], each 2*len doubles
   float* d_Hf = nullptr;       // mixed forms: [main | tail] FP32 copies, each len (re, im) pairs
+  // Mixed 32-point plans with V <= 16 and two or more blocks: a run takes two blocks per launch on 64-point
+  // windows of valid width 2V (wide_launches(pl) launches of depth 2t, the last one of depth t_wide_tail).
+  bool wide = false;
+  int64_t t_wide_tail = 0;             // depth of the last launch when it is below 2t, else 0
+  uint32_t* d_wide = nullptr;          // kOpsWide operand words, then kSpecWide floats for depth 2t and the tail
+  double dc_wide = 1.0, dc_wide_tail = 1.0;
+  int32_t scale_wide = 0, scale_wide_tail = 0;
   double dc_main = 1.0, dc_tail = 1.0;  // K(0)^t and K(0)^t_tail
   int32_t scale_main = 0, scale_tail = 0;  // FP16 form: scale exponents of the main and tail depths
   double* d_taps = nullptr;
@@ -108,9 +115,9 @@ struct ffs_batch {
   int dev = 0;
   int num_cus = 256;
   int64_t rounds = 0;
-  ffsk::TileArgs* d_items = nullptr;  // [round][grid]
-  int64_t* d_prefix = nullptr;        // [round][grid + 1]
-  std::vector<int32_t> active;        // grids with a block in each round
+  ffsk::TileArgs* d_items = nullptr;  // [round][grid]: the round's 64-point items, then its 32-point items
+  int64_t* d_prefix = nullptr;        // [round][2][grid + 1]: prefix sums of their work units
+  std::vector<int32_t> active[2];     // per round, grids with a 64-point (0) and a 32-point (1) launch
   std::vector<const double*> g_in;
   std::vector<double*> g_out;
   hipStream_t cap_stream = nullptr;
@@ -239,6 +246,11 @@ ffs_status choose_config_direct(ffs_plan* pl) {
 // tables of their own (ffsk::gen_operands_real, gen_spectrum_real).
 bool real_tiles(const ffs_plan* pl) {
   return pl->kind == ffsk::KIND_2D32 && pl->prob.precision == FFS_PREC_FP64;
+}
+
+// Launches of one run.
+int64_t run_launches(const ffs_plan* pl) {
+  return pl->wide ? (pl->prob.steps + 2 * pl->t - 1) / (2 * pl->t) : pl->nblocks;
 }
 
 // Choose tile family, fused depth and valid widths.
@@ -371,6 +383,11 @@ ffs_status choose_config(ffs_plan* pl) {
     if (p.dims == 2) pl->units = pl->tiles[0] * (real_tiles(pl) ? pl->tiles[1] : (pl->tiles[1] + 1) / 2);
     if (p.dims == 3) pl->units = pl->tiles[0] * pl->tiles[1] * ((pl->tiles[2] + 1) / 2);
   }
+  // Two blocks per launch on 64-point windows wherever the valid region of the doubled tile still fits the
+  // near half of the window (2V <= 32; beyond it the inverse stages would need both halves) and there are
+  // two blocks to take: Box2D25P 8192^2, two t = 4 blocks 684 us, one 64-point launch 337 us (FP16; BF16 1000 and 445).
+  pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2;
+  if (pl->wide) pl->t_wide_tail = p.steps % (2 * pl->t);
   return FFS_OK;
 }
 
@@ -389,6 +406,7 @@ void release(ffs_plan* pl) {
   if (pl->d_opsi) (void)hipFree(pl->d_opsi);
   if (pl->d_H) (void)hipFree(pl->d_H);
   if (pl->d_Hf) (void)hipFree(pl->d_Hf);
+  if (pl->d_wide) (void)hipFree(pl->d_wide);
   if (pl->d_taps) (void)hipFree(pl->d_taps);
   if (pl->d_scratch) (void)hipFree(pl->d_scratch);
   delete pl;
@@ -451,6 +469,24 @@ ffsk::TileArgs make_args(const ffs_plan* pl, const double* src, double* dst, boo
   a.out16 = out16_block(pl) ? 1 : 0;
   if (a.out16 && pl->d_opsi)
     a.opsi = static_cast<const char*>(pl->d_opsi) + (tail ? sizeof(uint32_t) * ffsk::kInv32Words : 0);
+  return a;
+}
+
+// One launch of a run on 64-point windows: the tile of valid width 2V at depth 2t (or the tail's depth).
+ffsk::TileArgs make_wide_args(const ffs_plan* pl, const double* src, double* dst, bool tail) {
+  ffsk::TileArgs a = make_args(pl, src, dst, false);
+  const ffs_problem& p = pl->prob;
+  const int64_t t = tail ? pl->t_wide_tail : 2 * pl->t;
+  const int hi = p.convention == FFS_CONV_REF ? 2 * p.radius : p.radius;
+  a.V0 = a.V1 = 2 * pl->V[0];
+  a.h0 = a.h1 = (int32_t)(hi * t);
+  a.tiles0 = (a.n0 + a.V0 - 1) / a.V0;
+  a.tiles1 = (a.n1 + a.V1 - 1) / a.V1;
+  a.units = a.tiles0 * a.tiles1;
+  a.opsm = pl->d_wide;
+  a.Hf = reinterpret_cast<const float*>(pl->d_wide + ffsk::kOpsWide) + (tail ? ffsk::kSpecWide : 0);
+  a.scale_exp = tail ? pl->scale_wide_tail : pl->scale_wide;
+  a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
   return a;
 }
 
@@ -518,12 +554,13 @@ hipError_t launch_one_block(ffs_plan* pl, const double* src, double* dst, bool t
 
 // Enqueue the whole block chain d_in -> ... -> d_out on stream s.
 ffs_status enqueue_chain(ffs_plan* pl, const double* d_in, double* d_out, hipStream_t s) {
-  const int64_t nb = pl->nblocks;
+  const int64_t nb = run_launches(pl);
   const double* src = d_in;
   for (int64_t b = 0; b < nb; b++) {
     double* dst = ((nb - 1 - b) % 2 == 0) ? d_out : pl->d_scratch;
-    const bool tail = (b == nb - 1) && pl->t_tail > 0;
-    hipError_t e = launch_one_block(pl, src, dst, tail, s);
+    const bool last = b == nb - 1;
+    hipError_t e = pl->wide ? ffsk::launch_wide(make_wide_args(pl, src, dst, last && pl->t_wide_tail > 0), s, pl->num_cus)
+                            : launch_one_block(pl, src, dst, last && pl->t_tail > 0, s);
     if (e != hipSuccess) return fail(FFS_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     src = dst;
   }
@@ -582,6 +619,8 @@ ffs_status plan_constants(ffs_plan* pl) {
     };
     pl->dc_main = ipow(sw, pl->t);
     pl->dc_tail = ipow(sw, pl->t_tail > 0 ? pl->t_tail : pl->t);
+    pl->dc_wide = ipow(sw, 2 * pl->t);
+    pl->dc_wide_tail = ipow(sw, pl->t_wide_tail);
   }
   if (p.precision == FFS_PREC_MIXED_F16) {
     // largest |K(k)| over the 32 x 32 frequencies (direct DFT of the taps; |K| does not depend on the
@@ -609,13 +648,24 @@ ffs_status plan_constants(ffs_plan* pl) {
                   10.0 - std::min(em, et));
     pl->scale_main = (int32_t)em;
     pl->scale_tail = (int32_t)et;
+    if (pl->wide) {
+      // 64-point windows scale their folded inputs below 2^9 (one bit for the fold of stage 2).  A doubled
+      // depth beyond the FP16 range keeps the plan's single blocks.
+      const double ew = expo(2 * pl->t) - 1.0, ewt = expo(pl->t_wide_tail) - 1.0;
+      if (ew < -100.0 || ewt < -100.0) {
+        pl->wide = false;
+      } else {
+        pl->scale_wide = (int32_t)ew;
+        pl->scale_wide_tail = (int32_t)ewt;
+      }
+    }
   }
   return FFS_OK;
 }
 
 // Bytes of each device table of a transform plan (0 = not used).
 struct TableSizes {
-  size_t ops, opsm, H, Hf, opsi, taps;
+  size_t ops, opsm, H, Hf, opsi, taps, wide;
 };
 // The DFT tables (complex operands and spectrum) of the plan's family and precision.
 TableSizes dft_table_sizes(const ffs_plan* pl) {
@@ -637,15 +687,24 @@ TableSizes table_sizes(const ffs_plan* pl) {
     t.H = sizeof(double) * 2 * ffsk::kSpecReal;
     t.opsi = 0;
   }
+  if (pl->wide) t.wide = sizeof(uint32_t) * ffsk::kOpsWide + sizeof(float) * 2 * ffsk::kSpecWide;
   return t;
 }
 
 // Operands and spectra into the plan's device tables, on stream s (the taps are already in d_taps).
 hipError_t dft_tables(const ffs_plan* pl, hipStream_t s);
 hipError_t plan_tables(const ffs_plan* pl, hipStream_t s) {
-  if (!real_tiles(pl)) return dft_tables(pl, s);
   const ffs_problem& p = pl->prob;
   const int K = 2 * p.radius + 1;
+  if (pl->wide) {
+    float* H = reinterpret_cast<float*>(pl->d_wide + ffsk::kOpsWide);
+    hipError_t e = ffsk::gen_operands_wide(pl->d_wide, p.precision == FFS_PREC_MIXED_F16, s);
+    if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, s);
+    if (e == hipSuccess && pl->t_wide_tail > 0)
+      e = ffsk::gen_spectrum_real(H + ffsk::kSpecWide, 64, pl->d_taps, K, p.convention, pl->t_wide_tail, s);
+    if (e != hipSuccess) return e;
+  }
+  if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
   if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);
   if (e == hipSuccess && pl->t_tail > 0)
@@ -835,9 +894,10 @@ ffs_status ffs_plan_create(const ffs_problem* p, ffs_plan** out) {
     chk(hipMalloc(&pl->d_H, ts.H));
     if (ts.Hf) chk(hipMalloc(&pl->d_Hf, ts.Hf));
     if (ts.opsi) chk(hipMalloc(&pl->d_opsi, ts.opsi));
+    if (ts.wide) chk(hipMalloc(&pl->d_wide, ts.wide));
     chk(hipMalloc(&pl->d_taps, ts.taps));
   }
-  if (pl->nblocks >= 2) chk(hipMalloc(&pl->d_scratch, sizeof(double) * pl->npoints));
+  if (run_launches(pl) >= 2) chk(hipMalloc(&pl->d_scratch, sizeof(double) * pl->npoints));
   if (e != hipSuccess) {
     release(pl);
     return fail(e == hipErrorOutOfMemory ? FFS_ERR_OUT_OF_MEMORY : FFS_ERR_HIP, "device allocation failed: %s",
@@ -924,7 +984,7 @@ ffs_status ffs_plan_get_info(const ffs_plan* pl, ffs_plan_info* info) {
   info->fuse = (int32_t)pl->t;
   info->fuse_tail = (int32_t)pl->t_tail;
   info->blocks = pl->nblocks;
-  info->launches = pl->nblocks;
+  info->launches = run_launches(pl);
   // Matrix-core flops executed per tile pair: stages (2 per axis) x 16^(d-2) slices x real 16x16x16
   // GEMMs per complex product x MFMA flops per real GEMM.
   //   FP64: Gauss form, 3 GEMMs of 4 x v_mfma_f64_16x16x4f64 (2*16^3 flops each GEMM)
@@ -1022,7 +1082,7 @@ ffs_status ffs_run(ffs_plan* pl, const double* d_in, double* d_out, void* stream
   }
   // Chains of a few launches go out as plain launches: replaying a graph costs ~9 us more per run on
   // MI355X than launching up to four kernels directly (measured on 1 to 4 block chains).
-  if (!pl->prob.use_graph || pl->nblocks <= kGraphMinLaunches) return enqueue_chain(pl, d_in, d_out, s);
+  if (!pl->prob.use_graph || run_launches(pl) <= kGraphMinLaunches) return enqueue_chain(pl, d_in, d_out, s);
   ffs_plan::GraphSlot* slot = nullptr;
   for (ffs_plan::GraphSlot& g : pl->graphs)
     if (g.gexec && g.in == d_in && g.out == d_out) slot = &g;
@@ -1083,7 +1143,7 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
     return at;
   };
   const size_t o_ops = carve(ts.ops), o_opsm = carve(ts.opsm), o_H = carve(ts.H), o_Hf = carve(ts.Hf),
-               o_opsi = carve(ts.opsi), o_taps = carve(ts.taps);
+               o_opsi = carve(ts.opsi), o_taps = carve(ts.taps), o_wide = carve(ts.wide);
   if (off > FFS_STATIC_TABLE_BYTES)
     return fail(FFS_ERR_INTERNAL, "plan tables need %zu bytes of the %llu reserved", off, FFS_STATIC_TABLE_BYTES);
   const size_t grid_bytes = pl.nblocks >= 2 ? sizeof(double) * (size_t)pl.npoints : 0;
@@ -1104,6 +1164,7 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
     pl.d_Hf = ts.Hf ? reinterpret_cast<float*>(b + o_Hf) : nullptr;
     pl.d_opsi = ts.opsi ? static_cast<void*>(b + o_opsi) : nullptr;
     pl.d_taps = reinterpret_cast<double*>(b + o_taps);
+    pl.d_wide = ts.wide ? reinterpret_cast<uint32_t*>(b + o_wide) : nullptr;
   }
   pl.d_scratch = grid_bytes ? reinterpret_cast<double*>(b + FFS_STATIC_TABLE_BYTES) : nullptr;
   hipStream_t s = (hipStream_t)stream;
@@ -1359,15 +1420,15 @@ ffs_status ffs_batch_create(const ffs_problem* problems, int32_t count, ffs_batc
     ffs_status st = ffs_plan_create(&p, &pl);
     if (st != FFS_OK) return bail(st);
     b->plans.push_back(pl);
-    b->rounds = std::max(b->rounds, pl->nblocks);
+    b->rounds = std::max(b->rounds, run_launches(pl));
   }
   b->dev = b->plans[0]->dev;
   b->num_cus = b->plans[0]->num_cus;
-  b->active.assign((size_t)b->rounds, 0);
+  for (auto& a : b->active) a.assign((size_t)b->rounds, 0);
   hipError_t e = hipSuccess;
   if (b->rounds > 0) {
     e = hipMalloc(&b->d_items, sizeof(ffsk::TileArgs) * b->rounds * count);
-    if (e == hipSuccess) e = hipMalloc(&b->d_prefix, sizeof(int64_t) * b->rounds * (count + 1));
+    if (e == hipSuccess) e = hipMalloc(&b->d_prefix, sizeof(int64_t) * b->rounds * 2 * (count + 1));
   }
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -1398,28 +1459,35 @@ ffs_status ffs_batch_run(ffs_batch* b, const double* const* d_in, double* const*
     // per-round work lists: grid g's block r reads its previous output and writes d_out or the plan's
     // ping-pong grid so that its last block lands in d_out
     std::vector<ffsk::TileArgs> items((size_t)(b->rounds * n));
-    std::vector<int64_t> prefix((size_t)(b->rounds * (n + 1)));
+    std::vector<int64_t> prefix((size_t)(b->rounds * 2 * (n + 1)));
     for (int64_t r = 0; r < b->rounds; r++) {
-      int32_t k = 0;
-      int64_t acc = 0;
-      for (int32_t g = 0; g < n; g++) {
-        ffs_plan* pl = b->plans[g];
-        const int64_t nb = pl->nblocks;
-        if (r >= nb) continue;
-        const double* src = d_in[g];
-        double* dst = nullptr;
-        for (int64_t q = 0; q <= r; q++) {
-          dst = ((nb - 1 - q) % 2 == 0) ? d_out[g] : pl->d_scratch;
-          if (q < r) src = dst;
+      int32_t at = 0;
+      for (int kind = 0; kind < 2; kind++) {  // 64-point items first
+        int32_t k = 0;
+        int64_t acc = 0;
+        int64_t* pre = &prefix[(size_t)((r * 2 + kind) * (n + 1))];
+        for (int32_t g = 0; g < n; g++) {
+          ffs_plan* pl = b->plans[g];
+          const int64_t nb = run_launches(pl);
+          if (r >= nb || pl->wide != (kind == 0)) continue;
+          const double* src = d_in[g];
+          double* dst = nullptr;
+          for (int64_t q = 0; q <= r; q++) {
+            dst = ((nb - 1 - q) % 2 == 0) ? d_out[g] : pl->d_scratch;
+            if (q < r) src = dst;
+          }
+          const bool last = r == nb - 1;
+          const ffsk::TileArgs item = pl->wide ? make_wide_args(pl, src, dst, last && pl->t_wide_tail > 0)
+                                               : make_args(pl, src, dst, last && pl->t_tail > 0);
+          items[(size_t)(r * n + at)] = item;
+          pre[k] = acc;
+          acc += item.units;
+          k++;
+          at++;
         }
-        const bool tail = (r == nb - 1) && pl->t_tail > 0;
-        items[(size_t)(r * n + k)] = make_args(pl, src, dst, tail);
-        prefix[(size_t)(r * (n + 1) + k)] = acc;
-        acc += pl->units;
-        k++;
+        pre[k] = acc;
+        b->active[kind][(size_t)r] = k;
       }
-      prefix[(size_t)(r * (n + 1) + k)] = acc;
-      b->active[(size_t)r] = k;
     }
     // a replay of the previous graph may still be reading the work lists (on any stream): let it finish
     FFS_HIP(hipDeviceSynchronize());
@@ -1435,9 +1503,14 @@ ffs_status ffs_batch_run(ffs_batch* b, const double* const* d_in, double* const*
     }
     FFS_HIP(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
     hipError_t le = hipSuccess;
-    for (int64_t r = 0; r < b->rounds && le == hipSuccess; r++)
-      le = ffsk::launch_batch(b->d_items + r * n, b->d_prefix + r * (n + 1), b->active[(size_t)r], b->precision,
-                              b->cap_stream, b->num_cus);
+    for (int64_t r = 0; r < b->rounds && le == hipSuccess; r++) {
+      const int32_t wide = b->active[0][(size_t)r], narrow = b->active[1][(size_t)r];
+      const int64_t* pre = b->d_prefix + r * 2 * (n + 1);
+      if (wide > 0)
+        le = ffsk::launch_batch_wide(b->d_items + r * n, pre, wide, b->precision, b->cap_stream, b->num_cus);
+      if (narrow > 0 && le == hipSuccess)
+        le = ffsk::launch_batch(b->d_items + r * n + wide, pre + n + 1, narrow, b->precision, b->cap_stream, b->num_cus);
+    }
     hipGraph_t g = nullptr;
     const hipError_t ee = hipStreamEndCapture(b->cap_stream, &g);
     if (le != hipSuccess || ee != hipSuccess) {

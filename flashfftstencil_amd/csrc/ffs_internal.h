@@ -105,12 +105,16 @@ hipError_t launch_direct(const DirectArgs& a, int dims, int radius, bool star, h
 hipError_t gen_operands(double* ops, uint32_t* opsm, const int32_t* axis_len, hipStream_t s);
 hipError_t gen_operands32(uint32_t* ops32, bool f16, hipStream_t s);
 hipError_t gen_operands32_f64(double* ops, hipStream_t s);
-// Tables of the real half-sample transforms (the 32-point FP64 kernels): kOpsReal operand doubles, and the
-// filter of one depth, 4 doubles per (k0, k1) in kernel order.
+// Tables of the real half-sample transforms.  32-point FP64 kernels: kOpsReal operand doubles, and the filter
+// of one depth, 4 doubles per (k0, k1) in kernel order.  64-point mixed kernels: kOpsWide operand words (the
+// BF16 form's size; FP16 uses two thirds), and kSpecWide floats per depth.
 constexpr int kOpsReal = 2 * 4 * kLanes;
 constexpr int kSpecReal = 4 * 16 * 16;
+constexpr int kOpsWide = 4 * 3 * 4 * kLanes;
+constexpr int kSpecWide = 4 * 32 * 32;
 hipError_t gen_operands_real(double* ops, hipStream_t s);
-hipError_t gen_spectrum_real(double* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
+hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s);
+hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
                              hipStream_t s);
 // Inverse operands of an out16 block, output column j <- window column (j + shift) mod 32:
 //   mixed forms: u4 per lane, [arr: R, I, NI][term 0..2][lane] (the kOps32Words entries of block Kb = 0);
@@ -132,6 +136,10 @@ hipError_t gen_spectrum(double* H, int kind, int layout, const int32_t* axis_len
 // Hf[2e], Hf[2e + 1] = (float)H[e], (float)H[len + e] for e < len: the FP32 copy of one depth's spectrum
 // that the mixed-form kernels read from global memory (the batch kernels and the 3D kernel).
 hipError_t spectrum_to_f32(const double* H, float* Hf, int64_t len, hipStream_t s);
+// Two fused blocks of a 32-point mixed plan on 64-point windows (FP16, BF16), for one grid or a batch's items.
+hipError_t launch_wide(const TileArgs& a, hipStream_t s, int num_cus);
+hipError_t launch_batch_wide(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision,
+                             hipStream_t s, int num_cus);
 hipError_t launch_block(const TileArgs& a, int kind, hipStream_t s, int num_cus);
 // One fused block of every grid of a batch (32-point family: FP64, BF16, FP16), items/prefix in device memory.
 hipError_t launch_batch(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision, hipStream_t s,

@@ -1490,6 +1490,430 @@ __global__ __launch_bounds__(256, 3) void k_batch32_f16(const TileArgs* __restri
              });
 }
 
+// ---------------------------------------------------------------------------------------------
+// 2D 64x64 windows, mixed FP16 and BF16 forms: two fused blocks of a 32-point plan in one launch.
+//
+// A 32-point plan of valid width V <= 16 and depth t has the same proportions as a 64-point window of
+// valid width 2V and depth 2t, with half the HBM passes, half the gather, store, split and filter work and
+// 5/8 of the MFMAs per point-step.  One wave takes one real window (no pairing) through the real
+// half-sample transforms of the FP64 32-point kernels, here with 32 x 32 cosine and sine matrices
+// (th_kn = pi (2k+1)(2n+1)/128), whose contraction fills the K = 32 of one MFMA.
+//
+// Layout.  A window axis has 4 blocks of 16: block 2 h + b holds positions 2i + b, counted from the near
+// (h = 0) or the far end (h = 1: position 63 - (2i + b)); a coefficient axis likewise: block 2 T + b holds
+// frequencies 2i + b of type T (0 cosine, 1 sine).  Interleaving the two blocks (2i + b) lets a lane load and
+// store two neighbouring columns at once (16 bytes).  Inside a block: FP32-accumulator order, lane
+// (j + 16q), reg v <-> row i = 4q + v, column i = j.  The A operand of a contraction over blocks (x0, x1) of
+// one half or type is (x0 | x1): element e <-> block e >> 2, row 4q + (e & 3).
+//   gather + fold  z[a_b | b_b][col block]     a = near - far, b = near + far rows, folded in FP64
+//   stage 1 y[col block][type0 block]; fold; stage 2 x[type0 block][type1 block]; filter
+//   stage 3 u[type1 block][near row block]; stage 4 out[near row block][near col block]
+// The near halves alone hold the valid region (positions 0 .. 2V - 1 < 32).
+//
+// FP16 range: the folded inputs are scaled below 2^s, s <= 9.  The absolute row sums of both matrices are
+// 1/(2 sin(pi/128)) = 20.4, so stage 1 stays below 20.4 * 2^9, its folds below 41 * 2^9 = 20,900; stage 2 is not
+// split before the filter, which carries the transforms' 1/1024; the stage 3 outputs are 1/32 of the column
+// transforms of the filtered window, below 1.3 max |out|.
+// ---------------------------------------------------------------------------------------------
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// LDS reads below this point are not moved above it (no instruction: one wave's LDS accesses are in order).
+// Without it the compiler hoists the operand and filter reads, which are the same for every window, out of
+// the loop and spills the registers it keeps them in.
+__device__ __forceinline__ void lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); }
+
+// Split operands of one contraction: NT terms (FP16: h, l; BF16: h, m, l).
+template <int PREC>
+struct Split;
+template <>
+struct Split<PREC_F16> {
+  static constexpr int NT = 2;
+  h8 t[2];
+  __device__ __forceinline__ void make(const f4& x0, const f4& x1, float unit) { split8_f16(x0, x1, unit, t[0], t[1]); }
+  __device__ __forceinline__ void make_scaled(const f4& x0, const f4& x1, float sc, float) {
+    split8_f16_scaled(x0, x1, sc, t[0], t[1]);
+  }
+  // acc += x F without the dominant product h Fh
+  __device__ __forceinline__ f4 small(const u4 (&F)[2], f4 acc) const {
+    acc = FFS_MFMA_F16(t[0], as_h8(F[1]), acc);
+    return FFS_MFMA_F16(t[1], as_h8(F[0]), acc);
+  }
+  __device__ __forceinline__ f4 main(const u4 (&F)[2], f4 acc) const { return FFS_MFMA_F16(t[0], as_h8(F[0]), acc); }
+};
+template <>
+struct Split<PREC_BF16> {
+  static constexpr int NT = 3;
+  bf8 t[3];
+  __device__ __forceinline__ void make(const f4& x0, const f4& x1, float) { split8<3>(x0, x1, t[0], t[1], t[2]); }
+  __device__ __forceinline__ void make_scaled(const f4& x0, const f4& x1, float, float unit) { make(x0, x1, unit); }
+  __device__ __forceinline__ f4 small(const u4 (&F)[3], f4 acc) const {
+    const bf8 G[3] = {as_bf8(F[0]), as_bf8(F[1]), as_bf8(F[2])};
+    return prod32_small<3>(t[0], t[1], t[2], G, acc);
+  }
+  __device__ __forceinline__ f4 main(const u4 (&F)[3], f4 acc) const { return FFS_MFMA_BF16(t[0], as_bf8(F[0]), acc); }
+};
+
+constexpr int kAhead = 4;  // row groups of the next window in flight (0: 405, 1: 346, 2: 343, 4: 336, 5: 340 us)
+typedef f4 Tile16[4][4];
+
+// The two contractions of one column block: cosine matrix on `c`, sine matrix on `s`, both output blocks.
+// sW: [type][block][term][lane].  The small split products of an output come first, the dominant one last.
+template <int PREC>
+__device__ __forceinline__ void contract(const Split<PREC>& c, const Split<PREC>& s, const u4* __restrict__ sW, int lane,
+                                         f4 (&oc)[2], f4 (&os)[2]) {
+  constexpr int NT = Split<PREC>::NT;
+  const f4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    u4 Fc[NT], Fs[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      Fc[t] = sW[(b * NT + t) * kLanes + lane];
+      Fs[t] = sW[((2 + b) * NT + t) * kLanes + lane];
+    }
+    oc[b] = c.small(Fc, z);
+    os[b] = s.small(Fs, z);
+    oc[b] = c.main(Fc, oc[b]);
+    os[b] = s.main(Fs, os[b]);
+  }
+}
+// Sum of the two contractions (the near half of an inverse stage), both output blocks.  The MFMA truncates an
+// accumulator that is smaller than its products toward zero, so the small split products of both types
+// are summed on their own and the two dominant products each start from zero: mean error on Box2D25P
+// 8192^2 x 32 -2.9e-9 -> -2e-10 for 1.8% of the time.  The same in the forward stages changed nothing
+// measurable (their errors pass the filter) and spilled.
+template <int PREC>
+__device__ __forceinline__ void contract_sum(const Split<PREC>& c, const Split<PREC>& s, const u4* __restrict__ sW,
+                                             int lane, f4 (&o)[2]) {
+  constexpr int NT = Split<PREC>::NT;
+  const f4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    u4 Fc[NT], Fs[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      Fc[t] = sW[(b * NT + t) * kLanes + lane];
+      Fs[t] = sW[((2 + b) * NT + t) * kLanes + lane];
+    }
+    const f4 e = s.small(Fs, c.small(Fc, z));
+    const f4 mc = c.main(Fc, z), ms = s.main(Fs, z);
+    o[b] = (ms + mc) + e;
+  }
+}
+
+// Sum over the wave, in every lane (DPP exchanges inside each row of 16 lanes, then the four row sums).
+__device__ __forceinline__ double dpp_add(double x, int sel) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, x);
+  int lo = (int)w, hi = (int)(w >> 32);
+  switch (sel) {  // the DPP control must be a constant
+    case 0: lo = __builtin_amdgcn_update_dpp(lo, lo, 0xB1, 0xF, 0xF, false);
+            hi = __builtin_amdgcn_update_dpp(hi, hi, 0xB1, 0xF, 0xF, false); break;  // quad_perm [1,0,3,2]
+    case 1: lo = __builtin_amdgcn_update_dpp(lo, lo, 0x4E, 0xF, 0xF, false);
+            hi = __builtin_amdgcn_update_dpp(hi, hi, 0x4E, 0xF, 0xF, false); break;  // quad_perm [2,3,0,1]
+    case 2: lo = __builtin_amdgcn_update_dpp(lo, lo, 0x141, 0xF, 0xF, false);
+            hi = __builtin_amdgcn_update_dpp(hi, hi, 0x141, 0xF, 0xF, false); break;  // row_half_mirror
+    default: lo = __builtin_amdgcn_update_dpp(lo, lo, 0x140, 0xF, 0xF, false);
+             hi = __builtin_amdgcn_update_dpp(hi, hi, 0x140, 0xF, 0xF, false); break;  // row_mirror
+  }
+  return x + __builtin_bit_cast(double, (uint64_t)(uint32_t)lo | ((uint64_t)(uint32_t)hi << 32));
+}
+__device__ __forceinline__ double wave_sum(double x) {
+  x = dpp_add(x, 0);
+  x = dpp_add(x, 1);
+  x = dpp_add(x, 2);
+  x = dpp_add(x, 3);
+  return (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
+}
+
+// A window's raw values as loaded: group g = 4 b + v holds row 2 (4q + v) + b (near) and 63 minus that (far),
+// each as the column pairs (2j, 2j + 1) and (62 - 2j, 63 - 2j): [near/near, near/far, far/near, far/far].
+struct Raw64 {
+  d2u g[8][4];
+};
+// Where a window lies: its grid and its first row and column (before the periodic wrap).
+struct Win64 {
+  const double* src;
+  int64_t n0, n1, rw, cw;
+};
+__device__ __forceinline__ Win64 win64(const TileArgs& a, const TilePos& p) {
+  return {a.src, a.n0, a.n1, p.t0 * a.V0 - a.h0, p.t1 * a.V1 - a.h1};
+}
+template <int G0, int G1>
+__device__ __forceinline__ void load64(const Win64& w, int q, int j, Raw64& r) {
+  const bool interior = w.rw >= 0 && w.rw + 64 <= w.n0 && w.cw >= 0 && w.cw + 64 <= w.n1 && w.n1 <= (1 << 22);
+  if (interior) {
+    const __amdgpu_buffer_rsrc_t rs = window_rsrc(w.src + w.rw * w.n1 + w.cw, true);
+    const uint32_t n1 = (uint32_t)w.n1;
+    // near rows 8q + (2v + b), far rows 63 - (8q + 2v + b) = 8 (3 - q) + (39 - 2v - b)
+    const uint32_t vn = (uint32_t)(8 * q) * n1 * 8u, vf = (uint32_t)(8 * (3 - q)) * n1 * 8u;
+    const uint32_t cn = (uint32_t)(2 * j) * 8u, cf = (uint32_t)(62 - 2 * j) * 8u;
+#pragma unroll
+    for (int g = G0; g < G1; g++) {
+      const int b = g >> 2, v = g & 3;
+      const uint32_t sn = (uint32_t)(2 * v + b) * n1 * 8u, sf = (uint32_t)(39 - 2 * v - b) * n1 * 8u;
+      r.g[g][0] = __builtin_bit_cast(d2u, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(vn + cn), (int)sn, 0));
+      r.g[g][1] = __builtin_bit_cast(d2u, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(vn + cf), (int)sn, 0));
+      r.g[g][2] = __builtin_bit_cast(d2u, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(vf + cn), (int)sf, 0));
+      r.g[g][3] = __builtin_bit_cast(d2u, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(vf + cf), (int)sf, 0));
+    }
+  } else {
+    const int64_t c0 = wrap_near(w.cw + 2 * j, w.n1), c1 = wrap_near(w.cw + 2 * j + 1, w.n1);
+    const int64_t c2 = wrap_near(w.cw + 62 - 2 * j, w.n1), c3 = wrap_near(w.cw + 63 - 2 * j, w.n1);
+#pragma unroll
+    for (int g = G0; g < G1; g++) {
+      const int i = 2 * (4 * q + (g & 3)) + (g >> 2);
+      const double* rn = w.src + wrap_near(w.rw + i, w.n0) * w.n1;
+      const double* rf = w.src + wrap_near(w.rw + 63 - i, w.n0) * w.n1;
+      r.g[g][0] = d2u{rn[c0], rn[c1]};
+      r.g[g][1] = d2u{rn[c2], rn[c3]};
+      r.g[g][2] = d2u{rf[c0], rf[c1]};
+      r.g[g][3] = d2u{rf[c2], rf[c3]};
+    }
+  }
+}
+
+// Folded window: z[b][C] = rows near - far, z[2 + b][C] = near + far - 2c, differences taken in FP64.
+// Returns the DC offset c: the mean of 8 rows spread over the window (0, 8, 16, 24, 39, 47, 55, 63).  (A
+// constant left in the window is one term of a cyclic transform but a whole series of a negacyclic one,
+// each term of which rounds: with the centre sample, as in the 32-point kernels, the FP16 form's relative
+// error on Box2D25P 8192^2 x 32 was 3.7e-8 instead of 5.9e-9.)
+__device__ __forceinline__ double fold64(const Raw64& r, Tile16& z) {
+  const d2u s = (r.g[0][0] + r.g[0][1]) + (r.g[0][2] + r.g[0][3]);
+  const double c = wave_sum(s[0] + s[1]) * (1.0 / 512);
+#pragma unroll
+  for (int g = 0; g < 8; g++) {
+    const int b = g >> 2, v = g & 3;
+    const double n[4] = {r.g[g][0][0], r.g[g][0][1], r.g[g][1][1], r.g[g][1][0]};
+    const double f[4] = {r.g[g][2][0], r.g[g][2][1], r.g[g][3][1], r.g[g][3][0]};
+#pragma unroll
+    for (int C = 0; C < 4; C++) {
+      z[b][C][v] = (float)(n[C] - f[C]);
+      z[2 + b][C][v] = (float)((n[C] + f[C]) - (c + c));
+    }
+  }
+  return c;
+}
+
+// Valid outputs out[b0][b1]: rows 2 (4q + v) + b0, columns 2j + b1, two columns per store.
+__device__ __forceinline__ void store64(const TileArgs& a, const TilePos& p, int q, int j, const f4 (&out)[2][2],
+                                        double scale, double add) {
+  const int64_t r0 = p.t0 * a.V0, c0 = p.t1 * a.V1;
+  const int64_t rows = min((int64_t)a.V0, a.n0 - r0), cols = min((int64_t)a.V1, a.n1 - c0);
+#pragma unroll
+  for (int b0 = 0; b0 < 2; b0++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int wr = 2 * (4 * q + v) + b0;
+      const double x = __builtin_fma((double)out[b0][0][v], scale, add);
+      const double y = __builtin_fma((double)out[b0][1][v], scale, add);
+      double* at = a.dst + (r0 + wr) * a.n1 + c0 + 2 * j;
+      if (wr < rows) {
+        if (2 * j + 1 < cols)
+          __builtin_nontemporal_store(d2u{x, y}, reinterpret_cast<d2u*>(at));
+        else if (2 * j < cols)
+          put_out(at, x);
+      }
+    }
+}
+
+// One 64-point window.  H: filter entry ((2 b0 + b1) * 4 + v) * 64 + lane = (alpha, beta, gamma, delta) of
+// (k0 = 2 (4q + v) + b0, k1 = 2j + b1), in FP32.
+//
+// The next window's first kAhead row groups are requested before stage 3, whose output needs only half the
+// registers, and stay in flight through stages 3 and 4 (`next`: where it lies, if there is one).
+//
+// What bounds it (Box2D25P 8192^2, depth 8, one launch): gather and store alone take 264 us (1.07 GB, 200 us at
+// the copy rate), the stages and the store alone 226 us; without the requests ahead the two followed each
+// other (450 us at 2 waves per SIMD), with them the launch takes 337 us (FP16; BF16 451), against 684 (1000)
+// for the two 32-point blocks it replaces.  232 VGPRs, 2 waves per SIMD; at 3 the raw window spills (711 us).
+template <int PREC>
+__device__ __forceinline__ void tile64(const TileArgs& a, const TilePos& p, const u4* __restrict__ sW,
+                                       const f4* __restrict__ H, int lane, int q, int j, const Win64& cur, Raw64& raw,
+                                       bool more, const Win64& next) {
+  Tile16 z, y;
+  __builtin_amdgcn_s_setprio(1);
+  load64<kAhead, 8>(cur, q, j, raw);
+  const double c = fold64(raw, z);
+  int e = 0;
+  float sc = 1.0f;
+  if (PREC == PREC_F16) {
+    float m = 0.f;
+#pragma unroll
+    for (int R = 0; R < 4; R++)
+#pragma unroll
+      for (int C = 0; C < 4; C++)
+#pragma unroll
+        for (int v = 0; v < 4; v += 2) m = fmaxf(m, fmaxf(fabsf(z[R][C][v]), fabsf(z[R][C][v + 1])));
+    m = wave_max_nonneg(m);
+    int k;
+    (void)frexpf(m, &k);  // m < 2^k
+    e = __builtin_amdgcn_readfirstlane(min(max(a.scale_exp - k, -120), 120));
+    sc = ldexpf(1.0f, e);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  lds_fence();
+#pragma unroll
+  for (int C = 0; C < 4; C++) {  // stage 1: contract the rows of column block C
+    Split<PREC> A, B;
+    A.make_scaled(z[0][C], z[1][C], sc, a.unit);
+    B.make_scaled(z[2][C], z[3][C], sc, a.unit);
+    f4 oc[2], os[2];
+    contract<PREC>(A, B, sW, lane, oc, os);
+    y[C][0] = oc[0];
+    y[C][1] = oc[1];
+    y[C][2] = os[0];
+    y[C][3] = os[1];
+  }
+  lds_fence();
+#pragma unroll
+  for (int D = 0; D < 4; D++) {  // stage 2: fold and contract the window columns
+    Split<PREC> A, B;
+    A.make(y[0][D] - y[2][D], y[1][D] - y[3][D], a.unit);
+    B.make(y[0][D] + y[2][D], y[1][D] + y[3][D], a.unit);
+    f4 oc[2], os[2];
+    contract<PREC>(A, B, sW, lane, oc, os);
+    z[D][0] = oc[0];
+    z[D][1] = oc[1];
+    z[D][2] = os[0];
+    z[D][3] = os[1];
+  }
+  lds_fence();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int b0 = b >> 1, b1 = b & 1;
+      const f4 h = H[(b * 4 + v) * kLanes + lane];
+      float cc = z[b0][b1][v], cs = z[b0][2 + b1][v], sn = z[2 + b0][b1][v], ss = z[2 + b0][2 + b1][v];
+      filter4(cc, cs, sn, ss, h[0], h[1], h[2], h[3]);
+      z[b0][b1][v] = cc;
+      z[b0][2 + b1][v] = cs;
+      z[2 + b0][b1][v] = sn;
+      z[2 + b0][2 + b1][v] = ss;
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  if (more) load64<0, kAhead>(next, q, j, raw);
+  __builtin_amdgcn_sched_barrier(0);
+  lds_fence();
+#pragma unroll
+  for (int D = 0; D < 4; D++) {  // stage 3: contract the row frequencies, near rows only
+    Split<PREC> A, B;
+    A.make(z[0][D], z[1][D], a.unit);
+    B.make(z[2][D], z[3][D], a.unit);
+    f4 o[2];
+    contract_sum<PREC>(A, B, sW, lane, o);
+    y[D][0] = o[0];
+    y[D][1] = o[1];
+  }
+  lds_fence();
+  f4 out[2][2];
+#pragma unroll
+  for (int D = 0; D < 2; D++) {  // stage 4: contract the column frequencies, near columns only
+    Split<PREC> A, B;
+    A.make(y[0][D], y[1][D], a.unit);
+    B.make(y[2][D], y[3][D], a.unit);
+    contract_sum<PREC>(A, B, sW, lane, out[D]);
+  }
+  store64(a, p, q, j, out, ldexp(1.0, -e), c * a.dc_gain);
+}
+
+template <int PREC>
+__device__ __forceinline__ void stage_wide_ops(u4* sW, const uint32_t* __restrict__ opsm) {
+  constexpr int NT = Split<PREC>::NT;
+  for (int i = threadIdx.x; i < 4 * NT * kLanes; i += blockDim.x) sW[i] = reinterpret_cast<const u4*>(opsm)[i];
+}
+
+template <int PREC>
+__global__ __launch_bounds__(256, 2) void k_tile64(TileArgs a) {
+  __shared__ u4 sW[4 * Split<PREC>::NT * kLanes];  // operands, 8 KB (FP16) or 12 KB (BF16)
+  __shared__ f4 sH[16 * kLanes];                   // filter, 16 KB
+  stage_wide_ops<PREC>(sW, a.opsm);
+  for (int i = threadIdx.x; i < 16 * kLanes; i += blockDim.x) sH[i] = reinterpret_cast<const f4*>(a.Hf)[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int q = lane >> 4, j = lane & 15;
+  const int64_t W = (int64_t)gridDim.x * 4;
+  const int64_t gw = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  TilePos p = tile_pos(gw, a.tiles1);
+  const TilePos stride = tile_pos(W, a.tiles1);
+  Win64 cur = win64(a, p);
+  Raw64 raw;
+  if (gw < a.units) load64<0, kAhead>(cur, q, j, raw);
+  for (int64_t u = gw; u < a.units; u += W) {
+    TilePos pn = p;
+    tile_step(pn, stride, a.tiles1);
+    const Win64 next = win64(a, pn);
+    tile64<PREC>(a, p, sW, sH, lane, q, j, cur, raw, u + W < a.units, next);
+    p = pn;
+    cur = next;
+  }
+}
+
+// Multi-grid launch of the 64-point windows: the operands in LDS, each item's filter read per window from its
+// table (L2-resident).
+template <int PREC>
+__global__ __launch_bounds__(256, 2) void k_batch64(const TileArgs* __restrict__ items,
+                                                    const int64_t* __restrict__ prefix, int32_t n) {
+  __shared__ u4 sW[4 * Split<PREC>::NT * kLanes];
+  stage_wide_ops<PREC>(sW, items[0].opsm);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int q = lane >> 4, j = lane & 15;
+  const int64_t W = (int64_t)gridDim.x * 4;
+  const int64_t gw = block_order(items[0].linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t total = prefix[n];
+  int lo = -1;
+  int64_t next = 0;
+  Win64 cur{};
+  Raw64 raw;
+  TilePos p{};
+  if (gw < total) {
+    lo = batch_grid(prefix, n, gw, lo, next);
+    p = tile_pos(gw - prefix[lo], items[lo].tiles1);
+    cur = win64(items[lo], p);
+    load64<0, kAhead>(cur, q, j, raw);
+  }
+  for (int64_t idx = gw; idx < total; idx += W) {
+    const TileArgs a = items[lo];  // independent scalar loads, from the scalar cache while lo is unchanged
+    const bool more = idx + W < total;
+    TilePos pn = p;
+    Win64 nextw = cur;
+    if (more) {
+      lo = batch_grid(prefix, n, idx + W, lo, next);
+      pn = tile_pos(idx + W - prefix[lo], items[lo].tiles1);
+      nextw = win64(items[lo], pn);
+    }
+    tile64<PREC>(a, p, sW, reinterpret_cast<const f4*>(a.Hf), lane, q, j, cur, raw, more, nextw);
+    p = pn;
+    cur = nextw;
+  }
+}
+
+hipError_t launch_wide(const TileArgs& a, hipStream_t s, int num_cus) {
+  if (a.units <= 0) return hipSuccess;
+  const dim3 g((unsigned)std::min<int64_t>((a.units + 3) / 4, (int64_t)num_cus * 2)), b(256);
+  if (a.precision == PREC_F16)
+    hipLaunchKernelGGL(k_tile64<PREC_F16>, g, b, 0, s, a);
+  else if (a.precision == PREC_BF16)
+    hipLaunchKernelGGL(k_tile64<PREC_BF16>, g, b, 0, s, a);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_wide(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision,
+                             hipStream_t s, int num_cus) {
+  const dim3 g((unsigned)num_cus * 2), b(256);
+  if (precision == PREC_F16)
+    hipLaunchKernelGGL(k_batch64<PREC_F16>, g, b, 0, s, d_items, d_prefix, n);
+  else if (precision == PREC_BF16)
+    hipLaunchKernelGGL(k_batch64<PREC_BF16>, g, b, 0, s, d_items, d_prefix, n);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
 hipError_t launch_batch(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision, hipStream_t s,
                         int num_cus) {
   const dim3 g((unsigned)num_cus * (precision == 0 ? 4 : 3)), b(256);
@@ -2077,7 +2501,8 @@ __global__ void k_gen_operands_real(double* t) {
 //   cc' =  alpha cc + beta ss + gamma sc + delta cs,   ss' =  alpha ss + beta cc - delta sc - gamma cs,
 //   sc' =  alpha sc - beta cs - gamma cc + delta ss,   cs' =  alpha cs - beta sc + gamma ss - delta cc
 // (c and s: cosine and sine along axis 0, then axis 1).  The transforms' 4/P^2 is folded in.
-// The entry order is the family's: FP64 32-point, entry v * 64 + lane <-> (q + 4v, j).
+// Entry order: FP64 32-point (P = 32, doubles), entry v * 64 + lane <-> (q + 4v, j); 64-point (P = 64, floats),
+// entry ((2 b0 + b1) * 4 + v) * 64 + lane <-> (2 (4q + v) + b0, 2j + b1).
 __device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
   double pr = 1.0, pi = 0.0, br = kr, bi = ki;
   for (int64_t n = t; n > 0; n >>= 1) {
@@ -2093,12 +2518,13 @@ __device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
   kr = pr;
   ki = pi;
 }
-__global__ void k_gen_spectrum_real(double* H, int32_t P, const double* taps, int32_t K, int32_t convention,
+__global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int32_t K, int32_t convention,
                                     int64_t t) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= 4 * kLanes) return;
-  const int lane = e % kLanes, v = e / kLanes;
-  const int k0 = (lane >> 4) + 4 * v, k1 = lane & 15;
+  if (e >= P * P / 4) return;
+  const int lane = e % kLanes, v = (e / kLanes) % 4, b = e / (4 * kLanes);
+  const int k0 = P == 32 ? (lane >> 4) + 4 * v : 2 * (4 * (lane >> 4) + v) + (b >> 1);
+  const int k1 = P == 32 ? lane & 15 : 2 * (lane & 15) + (b & 1);
   double L1r = 0.0, L1i = 0.0, L2r = 0.0, L2i = 0.0;
   for (int a0 = 0; a0 < K; a0++)
     for (int a1 = 0; a1 < K; a1++) {
@@ -2119,10 +2545,45 @@ __global__ void k_gen_spectrum_real(double* H, int32_t P, const double* taps, in
   cpow_t(L1r, L1i, t);
   cpow_t(L2r, L2i, t);
   const double norm = 0.5 * 4.0 / ((double)P * (double)P);
-  H[4 * e + 0] = (L1r + L2r) * norm;
-  H[4 * e + 1] = (L2r - L1r) * norm;
-  H[4 * e + 2] = (L1i + L2i) * norm;
-  H[4 * e + 3] = (L1i - L2i) * norm;
+  const double h[4] = {(L1r + L2r) * norm, (L2r - L1r) * norm, (L1i + L2i) * norm, (L1i - L2i) * norm};
+  for (int i = 0; i < 4; i++) {
+    if (P == 32)
+      static_cast<double*>(H)[4 * e + i] = h[i];
+    else
+      static_cast<float*>(H)[4 * e + i] = (float)h[i];
+  }
+}
+
+// Operands of the 64-point windows: [cos, sin][block b][term][lane] of 4 words; element e of lane (j + 16q) is
+// entry (2 (4q + (e & 3)) + (e >> 2), 2j + b) of cos / sin (pi (2n + 1)(2k + 1)/128), split into 2 FP16 or 3
+// BF16 terms.
+__global__ void k_gen_operands_wide(uint32_t* t, int32_t f16) {
+  const int nt = f16 ? 2 : 3;
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= 4 * nt * kLanes) return;
+  const int lane = idx % kLanes, term = (idx / kLanes) % nt, b = (idx / (nt * kLanes)) % 2, sine = idx / (2 * nt * kLanes);
+  const int q = lane >> 4, j = lane & 15;
+  for (int w = 0; w < 4; w++) {
+    uint32_t word = 0;
+    for (int half = 0; half < 2; half++) {
+      const int e = 2 * w + half;
+      const int n = 2 * (4 * q + (e & 3)) + (e >> 2), k = 2 * j + b;
+      double s, c;
+      sincospi((double)(((2 * n + 1) * (2 * k + 1)) % 256) / 128.0, &s, &c);
+      const double x = sine ? s : c;
+      uint16_t bits;
+      if (f16) {
+        const _Float16 h = (_Float16)(float)x;
+        bits = __builtin_bit_cast(uint16_t, term == 0 ? h : (_Float16)(float)(x - (double)h));
+      } else {
+        __bf16 h, m, l;
+        split3_bf16(x, h, m, l);
+        bits = __builtin_bit_cast(uint16_t, term == 0 ? h : (term == 1 ? m : l));
+      }
+      word |= (uint32_t)bits << (16 * half);
+    }
+    t[idx * 4 + w] = word;
+  }
 }
 
 hipError_t gen_operands_real(double* ops, hipStream_t s) {
@@ -2130,9 +2591,15 @@ hipError_t gen_operands_real(double* ops, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t gen_spectrum_real(double* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
+hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s) {
+  const int n = 4 * (f16 ? 2 : 3) * kLanes;
+  hipLaunchKernelGGL(k_gen_operands_wide, dim3((unsigned)n / 256), dim3(256), 0, s, ops, (int32_t)f16);
+  return hipGetLastError();
+}
+
+hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
                              hipStream_t s) {
-  hipLaunchKernelGGL(k_gen_spectrum_real, dim3(4), dim3(64), 0, s, H, P, d_taps, K, convention, t);
+  hipLaunchKernelGGL(k_gen_spectrum_real, dim3((unsigned)(P * P / 4 / 64)), dim3(64), 0, s, H, P, d_taps, K, convention, t);
   return hipGetLastError();
 }
 

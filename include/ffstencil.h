@@ -132,7 +132,8 @@ typedef struct ffs_plan_info {
   int32_t fuse_tail;      /* T mod t (0 = no tail block) */
   int64_t blocks;         /* fused blocks per run, tail included */
   int64_t tiles;          /* tiles per block */
-  int64_t launches;       /* kernel launches per run */
+  int64_t launches;       /* kernel launches per run: `blocks`, or half of them (rounded up) where the mixed
+                             2D forms take two blocks per launch on 64-point windows (V <= 16, blocks >= 2) */
   double flops_per_block; /* flops one block executes: matrix-core flops (FFT; see the kernels' header
                              comment) or FP64 FMA flops including the halo recomputation (DIRECT) */
   double bytes_per_block; /* algorithmic HBM bytes of one block: 16 B per grid point */
@@ -174,6 +175,8 @@ ffs_status ffs_plan_get_info(const ffs_plan* plan, ffs_plan_info* info);
  *   OPS_MIXED:  split operands of the mixed forms (BF16/FP16 words, FP32 chunks)
  *   SPECTRUM:   [main | tail] x [re plane | im plane] of K^t / prod(P), in the tile family's order
  *   INVERSE16:  out16 inverse operands of the main and the tail depth
+ * The 32-point FP64 kernels run real half-sample transforms on tables of their own; for those plans the DFT
+ * tables above are generated at the call.
  * No reference counterpart (the reference's tables live in __constant__ memory, src/2D/create_fft_pfa_plan.cu:25-107). */
 typedef enum ffs_table {
   FFS_TABLE_OPS = 0,

@@ -255,3 +255,42 @@ def test_out16_bitwise_equals_full_stages(ffs, oracle, torch_cuda, form, convent
         outs.append(d)
     assert info["valid"][0] == 32 - 2 * radius * fuse
     assert torch.equal(outs[0], outs[1]), (form, convention, radius, fuse, float((outs[0] - outs[1]).abs().max()))
+
+
+@pytest.mark.parametrize("form", ["f16", "bf16"])
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,fuse,size,steps", [
+    (2, 4, (64, 64), 8), (2, 4, (65, 63), 9), (2, 4, (31, 200), 23), (1, 8, (33, 97), 17), (1, 15, (70, 45), 31),
+    (3, 3, (66, 130), 12), (8, 1, (50, 70), 2), (15, 1, (40, 41), 3), (2, 4, (1, 33), 16), (2, 4, (129, 1), 12)])
+def test_2d_mixed_two_blocks_per_launch(ffs, oracle, torch_cuda, form, convention, radius, fuse, size, steps):
+    # 32-point plans with V = 32 - 2 r t <= 16 run two blocks per launch on 64-point windows: grids one short
+    # of, equal to and one past a window or a tile of 2V, T below, at and past multiples of 2t, V from 2 to 16,
+    # the widest filter shift (radius 15), single rows and columns.
+    rng = np.random.default_rng(17 * radius + fuse)
+    w = rng.random((2 * radius + 1) ** 2)
+    w /= w.sum()
+    x = oracle.uniform(61 + radius, size)
+    got, info = _run(ffs, torch_cuda, x, radius, w, steps, precision=form, convention=convention, fuse=fuse)
+    assert info["valid"][0] <= 16 and info["launches"] == -(-steps // (2 * fuse)), info
+    ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
+    assert oracle.errors(got, ref)[1] <= TOL_MIXED, (form, convention, radius, fuse, info)
+
+
+@pytest.mark.parametrize("form", ["f16", "bf16"])
+@pytest.mark.parametrize("n1", [1 << 22, (1 << 22) + 96])
+def test_2d_mixed_two_blocks_long_rows(ffs, torch_cuda, form, n1):
+    # 64-point windows at the widest rows read through 32-bit buffer offsets and one past them (the general
+    # gather), against the FP64 form (itself held to the oracle on these rows)
+    torch = torch_cuda
+    _, r, w, _ = ffs.named_stencil("Heat-2D", seed=3)
+    d_in = torch.empty((66, n1), dtype=torch.float64, device="cuda")
+    ffs.fill_uniform_device(7, d_in)
+    outs = []
+    for precision in (form, "fp64"):
+        with ffs.Plan(2, (66, n1), w, r, 16, precision=precision, fuse=8, tile=32) as plan:
+            d = torch.empty_like(d_in)
+            plan.run(d_in, d)
+            torch.cuda.synchronize()
+            assert plan.info["launches"] == (2 if precision == "fp64" else 1)
+        outs.append(d)
+    assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) <= TOL_MIXED
