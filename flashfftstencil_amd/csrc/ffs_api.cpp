@@ -88,6 +88,12 @@ struct ffs_plan {
   int64_t t_wide_tail = 0;             // depth of the last launch when it is below 2t, else 0
   uint32_t* d_wide = nullptr;          // kOpsWide operand words, then kSpecWide floats for depth 2t and the tail
   double dc_wide = 1.0, dc_wide_tail = 1.0;
+  // 3D FP64 and BF16 plans: a run streams planes (ffsk::launch_stream3d), launches of depth stream_t, the last one
+  // of depth stream_tail; E taps along axis 0.  d_wide holds the operands, then the filters of both depths.
+  bool stream = false;
+  int32_t stream_E = 0, stream_V = 0, stream_nseg = 1;
+  int64_t stream_t = 0, stream_tail = 0, stream_seg = 0;
+  double stream_dc[2][7] = {};
   int32_t scale_wide = 0, scale_wide_tail = 0;
   double dc_main = 1.0, dc_tail = 1.0;  // K(0)^t and K(0)^t_tail
   int32_t scale_main = 0, scale_tail = 0;  // FP16 form: scale exponents of the main and tail depths
@@ -248,8 +254,56 @@ bool real_tiles(const ffs_plan* pl) {
   return pl->kind == ffsk::KIND_2D32 && pl->prob.precision == FFS_PREC_FP64;
 }
 
+// Streamed 3D runs: whether to stream, the depth per launch and the planes per segment, from modelled times of
+// the run (SIMD cycles at 2.4 GHz, fitted to MI355X timings of 16^3 .. 512^3).
+//   streamed: launch 8,000 + rounds of resident waves (FP64: one per SIMD; BF16: two), each walking its segment
+//     and the 2rt planes that fill its partial sums; per plane FP64 7,000 (E = 3) and 8,300 (E = 5), BF16 10,400
+//     (E = 5) and 12,400 (E = 7) with two waves on a SIMD, half of that with one.
+//   16^3 tiles: launch 8,000 + rounds of resident workgroups (FP64 2 per CU, BF16 3), 45,000 (FP64) and 36,000
+//     (BF16) each, 10,000 less while a CU holds one.
+// Below about 110^3 points the tiles win (Heat-3D 64^3 x 10: FP64 101 against 107 us, BF16 55 against 89; they go
+// deeper per launch there), above it the stream (201x187x230 x 20: FP64 1271 -> 642, BF16 799 -> 481 us).
+// A run that is one launch on tiles stays one.
+void choose_stream(ffs_plan* pl) {
+  const ffs_problem& p = pl->prob;
+  const int r = p.radius;
+  const bool fp64 = p.precision == FFS_PREC_FP64;
+  if (p.dims != 3 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
+  if (p.sizes[1] > ((int64_t)1 << 27) / p.sizes[2]) return;  // 32-bit byte offsets inside a plane
+  const int emax = fp64 ? 5 : 7;  // instantiated taps: the partial sums stay in registers
+  const double pairs = (double)pl->units;
+  double best = (double)pl->nblocks *
+                (8000.0 + std::ceil(pairs / (fp64 ? 512.0 : 768.0)) * (fp64 ? 45000.0 : 36000.0) - (pairs <= 256.0 ? 10000.0 : 0.0));
+  for (int64_t t = 1; 2 * r * t + 1 <= emax; t++) {
+    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
+    if (nl > 1 && pl->nblocks == 1) continue;
+    const int64_t V = 32 - 2 * r * te;
+    const int64_t tiles = ((p.sizes[1] + V - 1) / V) * ((p.sizes[2] + V - 1) / V);
+    const int E = (int)(2 * r * te + 1);
+    const double plane = fp64 ? 5050.0 + 650.0 * E : 5400.0 + 1000.0 * E;
+    for (int64_t nseg = 1; nseg <= std::min<int64_t>(p.sizes[0], 4096); nseg++) {
+      const int64_t seg = (p.sizes[0] + nseg - 1) / nseg;
+      if ((p.sizes[0] + seg - 1) / seg != nseg) continue;
+      const double units = (double)tiles * (double)nseg;
+      const double rounds = fp64 ? std::ceil(units / 1024.0) : units <= 1024.0 ? 0.5 : std::ceil(units / 2048.0);
+      const double cost = (double)nl * (8000.0 + rounds * (double)(seg + E - 1) * plane);
+      if (cost < best * (1 - 1e-9)) {
+        best = cost;
+        pl->stream = true;
+        pl->stream_t = te;
+        pl->stream_E = E;
+        pl->stream_V = (int32_t)V;
+        pl->stream_nseg = (int32_t)nseg;
+        pl->stream_seg = seg;
+      }
+    }
+  }
+  if (pl->stream) pl->stream_tail = p.steps % pl->stream_t;
+}
+
 // Launches of one run.
 int64_t run_launches(const ffs_plan* pl) {
+  if (pl->stream) return (pl->prob.steps + pl->stream_t - 1) / pl->stream_t;
   return pl->wide ? (pl->prob.steps + 2 * pl->t - 1) / (2 * pl->t) : pl->nblocks;
 }
 
@@ -388,6 +442,7 @@ ffs_status choose_config(ffs_plan* pl) {
   // two blocks to take: Box2D25P 8192^2, two t = 4 blocks 684 us, one 64-point launch 337 us (FP16; BF16 1000 and 445).
   pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2;
   if (pl->wide) pl->t_wide_tail = p.steps % (2 * pl->t);
+  choose_stream(pl);
   return FFS_OK;
 }
 
@@ -490,6 +545,36 @@ ffsk::TileArgs make_wide_args(const ffs_plan* pl, const double* src, double* dst
   return a;
 }
 
+size_t stream_ops_bytes(const ffs_plan* pl) {
+  return pl->prob.precision == FFS_PREC_FP64 ? sizeof(double) * ffsk::kOpsReal : sizeof(uint32_t) * ffsk::kOpsFold;
+}
+size_t stream_spec_bytes(const ffs_plan* pl) {
+  return (pl->prob.precision == FFS_PREC_FP64 ? sizeof(double) : sizeof(float)) * 4 * 256 * (size_t)pl->stream_E;
+}
+
+ffsk::Stream3Args make_stream_args(const ffs_plan* pl, const double* src, double* dst, bool tail) {
+  const ffs_problem& p = pl->prob;
+  ffsk::Stream3Args a{};
+  a.src = src;
+  a.dst = dst;
+  const char* base = reinterpret_cast<const char*>(pl->d_wide);
+  a.ops = base;
+  a.H = base + stream_ops_bytes(pl) + (tail ? stream_spec_bytes(pl) : 0);
+  a.n0 = p.sizes[0];
+  a.n1 = p.sizes[1];
+  a.n2 = p.sizes[2];
+  a.V = pl->stream_V;
+  a.tiles1 = (a.n1 + a.V - 1) / a.V;
+  a.tiles2 = (a.n2 + a.V - 1) / a.V;
+  a.seg = pl->stream_seg;
+  a.nseg = pl->stream_nseg;
+  const int hi = p.convention == FFS_CONV_REF ? 2 * p.radius : p.radius;
+  a.h0 = a.h = (int32_t)(hi * (tail ? pl->stream_tail : pl->stream_t));
+  a.linear_map = linear_map(pl) ? 1 : 0;
+  for (int e = 0; e < 7; e++) a.dc[e] = pl->stream_dc[tail ? 1 : 0][e];
+  return a;
+}
+
 // Direct path: launch geometry of one block of depth t (the window is fixed, the valid part shrinks
 // with t).  About two workgroups per CU along axis 0, each streaming a segment of rows (planes).
 ffsk::DirectArgs make_direct_args(const ffs_plan* pl, const double* src, double* dst, int64_t t) {
@@ -559,7 +644,9 @@ ffs_status enqueue_chain(ffs_plan* pl, const double* d_in, double* d_out, hipStr
   for (int64_t b = 0; b < nb; b++) {
     double* dst = ((nb - 1 - b) % 2 == 0) ? d_out : pl->d_scratch;
     const bool last = b == nb - 1;
-    hipError_t e = pl->wide ? ffsk::launch_wide(make_wide_args(pl, src, dst, last && pl->t_wide_tail > 0), s, pl->num_cus)
+    hipError_t e = pl->stream ? ffsk::launch_stream3d(make_stream_args(pl, src, dst, last && pl->stream_tail > 0),
+                                                      pl->prob.precision, pl->stream_E, s)
+                   : pl->wide ? ffsk::launch_wide(make_wide_args(pl, src, dst, last && pl->t_wide_tail > 0), s, pl->num_cus)
                             : launch_one_block(pl, src, dst, last && pl->t_tail > 0, s);
     if (e != hipSuccess) return fail(FFS_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     src = dst;
@@ -619,6 +706,24 @@ ffs_status plan_constants(ffs_plan* pl) {
     };
     pl->dc_main = ipow(sw, pl->t);
     pl->dc_tail = ipow(sw, pl->t_tail > 0 ? pl->t_tail : pl->t);
+    if (pl->stream) {  // gains of a constant plane per tap: the axis-0 marginal of the taps to the power t
+      const int K2 = K * K, hi = K - 1;
+      double m[7] = {};
+      for (int64_t i = 0; i < (int64_t)pl->weights.size(); i++) {
+        const int a0 = (int)(i / K2);
+        m[p.convention == FFS_CONV_REF ? hi - a0 : a0] += pl->weights[(size_t)i];
+      }
+      for (int d = 0; d < 2; d++) {
+        double g[7] = {1.0};
+        for (int64_t n = 0; n < (d ? pl->stream_tail : pl->stream_t); n++) {
+          double next[7] = {};
+          for (int i = 0; i < 7; i++)
+            for (int e = 0; e < K && i + e < 7; e++) next[i + e] += g[i] * m[e];
+          std::memcpy(g, next, sizeof g);
+        }
+        std::memcpy(pl->stream_dc[d], g, sizeof g);
+      }
+    }
     pl->dc_wide = ipow(sw, 2 * pl->t);
     pl->dc_wide_tail = ipow(sw, pl->t_wide_tail);
   }
@@ -688,6 +793,7 @@ TableSizes table_sizes(const ffs_plan* pl) {
     t.opsi = 0;
   }
   if (pl->wide) t.wide = sizeof(uint32_t) * ffsk::kOpsWide + sizeof(float) * 2 * ffsk::kSpecWide;
+  if (pl->stream) t.wide = stream_ops_bytes(pl) + 2 * stream_spec_bytes(pl);
   return t;
 }
 
@@ -702,6 +808,18 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s) {
     if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, s);
     if (e == hipSuccess && pl->t_wide_tail > 0)
       e = ffsk::gen_spectrum_real(H + ffsk::kSpecWide, 64, pl->d_taps, K, p.convention, pl->t_wide_tail, s);
+    if (e != hipSuccess) return e;
+  }
+  if (pl->stream) {
+    const bool mixed = p.precision != FFS_PREC_FP64;
+    char* base = reinterpret_cast<char*>(pl->d_wide);
+    char* H = base + stream_ops_bytes(pl);
+    hipError_t e = mixed ? ffsk::gen_operands_fold(pl->d_wide, s) : ffsk::gen_operands_real(reinterpret_cast<double*>(base), s);
+    if (e == hipSuccess)
+      e = ffsk::gen_stream3d(H, mixed, pl->stream_E, pl->d_taps, K, p.convention, (int32_t)pl->stream_t, s);
+    if (e == hipSuccess && pl->stream_tail > 0)
+      e = ffsk::gen_stream3d(H + stream_spec_bytes(pl), mixed, pl->stream_E, pl->d_taps, K, p.convention,
+                             (int32_t)pl->stream_tail, s);
     if (e != hipSuccess) return e;
   }
   if (!real_tiles(pl)) return dft_tables(pl, s);

@@ -136,6 +136,26 @@ hipError_t gen_spectrum(double* H, int kind, int layout, const int32_t* axis_len
 // Hf[2e], Hf[2e + 1] = (float)H[e], (float)H[len + e] for e < len: the FP32 copy of one depth's spectrum
 // that the mixed-form kernels read from global memory (the batch kernels and the 3D kernel).
 hipError_t spectrum_to_f32(const double* H, float* Hf, int64_t len, hipStream_t s);
+// One launch of the streamed 3D kernels (FP64, BF16): depth t, E = 2 r t + 1 rounded up to an instantiated tap count.
+struct Stream3Args {
+  const double* src;
+  double* dst;
+  const void* H;    // E x 256 filters of 4 values (FP64 or FP32)
+  const void* ops;  // kOpsReal doubles or kOpsFold words
+  int64_t n0, n1, n2;
+  int64_t tiles1, tiles2;
+  int64_t seg;          // output planes per work unit
+  int32_t nseg;
+  int32_t V;            // valid width in the plane, both axes
+  int32_t h0, h;        // window offset along the stream and in the plane
+  int32_t linear_map;   // as in TileArgs
+  double dc[7];         // mixed form: gain of a constant plane e planes ahead
+};
+constexpr int kOpsFold = 6 * kLanes * 4;
+hipError_t gen_stream3d(void* H, bool mixed, int32_t E, const double* d_taps, int32_t K, int32_t convention, int32_t t,
+                        hipStream_t s);
+hipError_t gen_operands_fold(uint32_t* ops, hipStream_t s);
+hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, hipStream_t s);
 // Two fused blocks of a 32-point mixed plan on 64-point windows (FP16, BF16), for one grid or a batch's items.
 hipError_t launch_wide(const TileArgs& a, hipStream_t s, int num_cus);
 hipError_t launch_batch_wide(const TileArgs* d_items, const int64_t* d_prefix, int32_t n, int32_t precision,

@@ -618,6 +618,7 @@ __global__ __launch_bounds__(256, 4) void k_batch32_f64(const TileArgs* __restri
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
 #define FFS_MFMA_BF16(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16((a), (b), (c), 0, 0, 0)
 #define FFS_MFMA_F32(a, b, c) __builtin_amdgcn_mfma_f32_16x16x4f32((a), (b), (c), 0, 0, 0)
@@ -2600,6 +2601,359 @@ hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s) {
 hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
                              hipStream_t s) {
   hipLaunchKernelGGL(k_gen_spectrum_real, dim3((unsigned)(P * P / 4 / 64)), dim3(64), 0, s, H, P, d_taps, K, convention, t);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------
+// 3D grids, streamed along axis 0: spectral in the planes, direct along the stream (FP64 and BF16 forms).
+//
+// The t-step operator is a polynomial in the axis-0 shift whose coefficients are 2D filters:
+//   S^t(x)[p] = sum_{e=0}^{2rt} G_e x[p + e],  G_e acting in the plane.
+// So only the planes are transformed (32-point real half-sample transforms, as in the 2D kernels), and the
+// 2rt + 1 filters of a plane's coefficients are added into the partial sums of the outputs it feeds.  One
+// wave owns a 32 x 32 window of axes 1 and 2 and walks a segment of planes: a plane is transformed once,
+// not once per overlapping window along axis 0, nothing passes through LDS and there are no barriers.  The
+// 16^3 complex tiles (k_tile3d) transform (16/12)^3 values per output in six stages through three LDS phases.
+//
+// Partial sums: acc[k] belongs to the output that still needs taps k + 1 more planes away; the arriving
+// plane finishes acc[0] with tap E - 1 and moves every other sum down by one as it adds to it, so the shift
+// costs nothing.  E (odd, 2rt + 1 rounded up; missing taps are zero) is a template parameter: the sums stay in
+// registers.
+//
+// Registers and occupancy: BF16 236 VGPRs at E = 7, 2 waves per SIMD; FP64 274 at E = 5, 1 wave (2 with spills
+// were 2% slower).  Bound by issue: BF16 E = 7 1068 VALU and 48 MFMAs per plane, 5,040 of the 6,300 cycles a
+// plane takes; FP64 E = 5 424 FP64 VALU and 64 FP64 MFMAs, 5,800 of 8,900.  Stores are ordinary ones: the rows
+// of 28 or 26 valid columns end inside cache lines, and as non-temporal stores they took 890 us per launch
+// instead of 626 (Box3D27P 512^3 BF16).  Box3D27P 512^3: BF16 262 -> 640, FP64 153 -> 355 GStencils/s.
+//
+// Mixed form: each plane's window is taken relative to its own mean c (FP64); the constant part of output
+// p is sum_e dc[e] c[p + e] with dc[e] the sum of the taps of G_e, added back in FP64 at the store.
+// ---------------------------------------------------------------------------------------------
+struct OpsFold {  // BF16 pairings (Fh|Fh), (Fm|Fm), (Fl|Fh) of the 16 x 16 cosine and sine matrices
+  bf8 c[3], s[3];
+};
+__device__ __forceinline__ void load_ops_fold(OpsFold& o, const u4* __restrict__ sW, int lane) {
+#pragma unroll
+  for (int g = 0; g < 3; g++) {
+    o.c[g] = as_bf8(sW[g * kLanes + lane]);
+    o.s[g] = as_bf8(sW[(3 + g) * kLanes + lane]);
+  }
+}
+
+template <int PREC>
+struct Plane3;
+template <>
+struct Plane3<0> {
+  typedef double V;
+  typedef d4 V4;
+  static constexpr int kOpsBytes = kOpsReal * 8;
+  static __device__ __forceinline__ int row(int q, int v) { return q + 4 * v; }
+  static __device__ __forceinline__ void fwd(const V4 (&z)[2][2], const void* sW, int lane, V4 (&y)[2][2]) {
+    OpsReal f;
+    load_ops_real(f, static_cast<const double*>(sW), lane);
+    fold_fwd(z, f, y);
+  }
+  static __device__ __forceinline__ void inv(const V4 (&x)[2][2], const void* sW, int lane, V4 (&y)[2][2]) {
+    OpsReal f;
+    load_ops_real(f, static_cast<const double*>(sW), lane);
+    fold_inv<2, 2>(x, f, y);
+  }
+};
+template <>
+struct Plane3<PREC_BF16> {
+  typedef float V;
+  typedef f4 V4;
+  static constexpr int kOpsBytes = 6 * kLanes * 16;
+  static __device__ __forceinline__ int row(int q, int v) { return 4 * q + v; }
+  // small split products first, the dominant pairing last (forward); summed on their own (inverse)
+  static __device__ __forceinline__ void fwd(const V4 (&z)[2][2], const void* sW, int lane, V4 (&y)[2][2]) {
+    OpsFold f;
+    load_ops_fold(f, static_cast<const u4*>(sW), lane);
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int C = 0; C < 2; C++) {
+      bf8 A[3], B[3];
+      split_a<3>(z[0][C] - z[1][C], A);
+      split_a<3>(z[0][C] + z[1][C], B);
+      f4 oc = FFS_MFMA_BF16(A[2], f.c[2], zero), os = FFS_MFMA_BF16(B[2], f.s[2], zero);
+      oc = FFS_MFMA_BF16(A[1], f.c[1], oc);
+      os = FFS_MFMA_BF16(B[1], f.s[1], os);
+      y[C][0] = FFS_MFMA_BF16(A[0], f.c[0], oc);
+      y[C][1] = FFS_MFMA_BF16(B[0], f.s[0], os);
+    }
+  }
+  static __device__ __forceinline__ void inv(const V4 (&x)[2][2], const void* sW, int lane, V4 (&y)[2][2]) {
+    OpsFold f;
+    load_ops_fold(f, static_cast<const u4*>(sW), lane);
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int C = 0; C < 2; C++) {
+      bf8 A[3], B[3];
+      split_a<3>(x[0][C], A);
+      split_a<3>(x[1][C], B);
+      f4 ec = FFS_MFMA_BF16(A[2], f.c[2], zero), es = FFS_MFMA_BF16(B[2], f.s[2], zero);
+      ec = FFS_MFMA_BF16(A[1], f.c[1], ec);
+      es = FFS_MFMA_BF16(B[1], f.s[1], es);
+      const f4 oc = FFS_MFMA_BF16(A[0], f.c[0], zero) + ec, os = FFS_MFMA_BF16(B[0], f.s[0], zero) + es;
+      y[C][0] = os + oc;
+      y[C][1] = os - oc;
+    }
+  }
+};
+
+// a += filter (h) x on one (k1, k2): the rows of filter4, each started from the partial sum.
+template <typename T, typename H4>
+__device__ __forceinline__ void filter4_add(T (&o)[4], T cc, T cs, T sc, T ss, const H4& h) {
+  o[0] = fma_t(h[0], cc, fma_t(h[1], ss, fma_t(h[2], sc, fma_t(h[3], cs, o[0]))));
+  o[1] = fma_t(h[0], cs, fma_t(h[2], ss, fma_t(-h[1], sc, fma_t(-h[3], cc, o[1]))));
+  o[2] = fma_t(h[0], sc, fma_t(h[3], ss, fma_t(-h[1], cs, fma_t(-h[2], cc, o[2]))));
+  o[3] = fma_t(h[0], ss, fma_t(h[1], cc, fma_t(-h[3], sc, fma_t(-h[2], cs, o[3]))));
+}
+
+template <int PREC, int E>
+__global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args a) {
+  typedef Plane3<PREC> P;
+  typedef typename P::V V;
+  typedef typename P::V4 V4;
+  constexpr bool MIXED = PREC != 0;
+  __shared__ V4 sH[E * 4 * kLanes];  // filters, entry (e * 4 + v) * 64 + lane
+  __shared__ u4 sW[P::kOpsBytes / 16];
+  for (int i = threadIdx.x; i < E * 4 * kLanes; i += blockDim.x) sH[i] = static_cast<const V4*>(a.H)[i];
+  for (int i = threadIdx.x; i < P::kOpsBytes / 16; i += blockDim.x) sW[i] = static_cast<const u4*>(a.ops)[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int q = lane >> 4, j = lane & 15;
+  const int64_t u = block_order(a.linear_map, blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t per = a.tiles1 * a.tiles2;
+  if (u >= per * a.nseg) return;  // whole waves; no barrier below
+  const int64_t sg = u / per, rem = u - sg * per;
+  const int64_t t1 = rem / a.tiles2, t2 = rem - t1 * a.tiles2;
+  const int64_t p0 = sg * a.seg, len = min(a.seg, a.n0 - p0);
+  // Byte offsets in a plane (below 2^31): loads per row (near, far) and column, stores likewise with
+  // out-of-range rows and columns sent past the plane's end, where the buffer store drops them.
+  const int64_t rw = t1 * a.V - a.h, cw = t2 * a.V - a.h;
+  const int64_t r0 = t1 * a.V, c0 = t2 * a.V;
+  const uint32_t kDrop = 0x80000000u;
+  uint32_t lrow[2][4], srow[2][4], lcol[2], scol[2];
+#pragma unroll
+  for (int R = 0; R < 2; R++) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int i = R ? 31 - P::row(q, v) : P::row(q, v);
+      lrow[R][v] = (uint32_t)(wrap_near(rw + i, a.n1) * a.n2 * 8);
+      srow[R][v] = i < a.V && r0 + i < a.n1 ? (uint32_t)((r0 + i) * a.n2 * 8) : kDrop;
+    }
+    const int i = R ? 31 - j : j;
+    lcol[R] = (uint32_t)(wrap_near(cw + i, a.n2) * 8);
+    scol[R] = i < a.V && c0 + i < a.n2 ? (uint32_t)((c0 + i) * 8) : kDrop;
+  }
+  const int64_t plane = a.n1 * a.n2;
+  auto rsrc = [&](const double* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base), 0, (int)(plane * 8), 0x00020000);
+  };
+  d4 raw[2][2];
+  auto load = [&](int64_t pl) {
+    const __amdgpu_buffer_rsrc_t rs = rsrc(a.src + pl * plane);
+#pragma unroll
+    for (int R = 0; R < 2; R++)
+#pragma unroll
+      for (int C = 0; C < 2; C++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) raw[R][C][v] = window_load(rs, lrow[R][v] + lcol[C], 0);
+  };
+  V4 acc[E - 1][2][2];
+#pragma unroll
+  for (int k = 0; k < E - 1; k++)
+#pragma unroll
+    for (int b = 0; b < 4; b++) acc[k][b >> 1][b & 1] = V4{0, 0, 0, 0};
+  double dacc[MIXED ? E - 1 : 1] = {};
+  int64_t pl = wrap_near(p0 - a.h0, a.n0);
+  load(pl);
+  // One plane: transform it, add its filters to the partial sums, leave the finished coefficients in z.
+  auto take = [&](V4 (&z)[2][2], double& dout) {
+    V4 y[2][2];
+    dout = 0.0;
+    if constexpr (MIXED) {
+      // plane mean over rows 0, 4, 8, 12, 19, 23, 27, 31
+      const double c =
+          wave_sum((raw[0][0][0] + raw[0][1][0]) + (raw[1][0][0] + raw[1][1][0])) * (1.0 / 256);
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) z[b >> 1][b & 1][v] = (V)(raw[b >> 1][b & 1][v] - c);
+      dout = __builtin_fma(a.dc[E - 1], c, dacc[0]);
+#pragma unroll
+      for (int k = 1; k < E; k++) dacc[k - 1] = k < E - 1 ? __builtin_fma(a.dc[E - 1 - k], c, dacc[k < E - 1 ? k : 0]) : a.dc[0] * c;
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) z[b >> 1][b & 1][v] = raw[b >> 1][b & 1][v];
+    }
+    lds_fence();
+    pl = pl + 1 == a.n0 ? 0 : pl + 1;
+    __builtin_amdgcn_sched_barrier(0);
+    load(pl);  // the next plane's window, in flight through this plane's work
+    __builtin_amdgcn_sched_barrier(0);
+    P::fwd(z, sW, lane, y);
+    __builtin_amdgcn_sched_barrier(0);
+    P::fwd(y, sW, lane, z);
+    lds_fence();
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const V cc = z[0][0][v], cs = z[0][1][v], sc = z[1][0][v], ss = z[1][1][v];
+      __builtin_amdgcn_sched_barrier(0);  // one row's filters at a time: hoisted together they spill
+#pragma unroll
+      for (int k = 0; k < E; k++) {
+        const V4 h = sH[((E - 1 - k) * 4 + v) * kLanes + lane];
+        V o[4] = {0, 0, 0, 0};
+        if (k < E - 1) {
+#pragma unroll
+          for (int b = 0; b < 4; b++) o[b] = acc[k < E - 1 ? k : 0][b >> 1][b & 1][v];
+        }
+        filter4_add(o, cc, cs, sc, ss, h);
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+          if (k == 0)
+            z[b >> 1][b & 1][v] = o[b];
+          else
+            acc[k > 0 ? k - 1 : 0][b >> 1][b & 1][v] = o[b];
+        }
+      }
+    }
+  };
+  V4 z[2][2], y[2][2];
+  double dout;
+  // The first E - 1 planes finish no output.  A loop of their own: with a branch around the stores instead,
+  // the wait for the next window's loads would have to cover the stores issued after them.
+  for (int m = 0; m < E - 1; m++) take(z, dout);
+  for (int64_t m = 0; m < len; m++) {
+    take(z, dout);
+    lds_fence();
+    __builtin_amdgcn_sched_barrier(0);
+    P::inv(z, sW, lane, y);
+    __builtin_amdgcn_sched_barrier(0);
+    P::inv(y, sW, lane, z);
+    __builtin_amdgcn_sched_barrier(0);
+    const __amdgpu_buffer_rsrc_t ro = rsrc(a.dst + (p0 + m) * plane);
+#pragma unroll
+    for (int R = 0; R < 2; R++)
+#pragma unroll
+      for (int C = 0; C < 2; C++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const uint32_t off = (srow[R][v] | scol[C]) & kDrop ? kDrop : srow[R][v] + scol[C];
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, (double)z[R][C][v] + dout), ro, (int)off, 0, 0);
+        }
+  }
+}
+
+// Filters of the streamed kernel: entry (e * 4 + v) * 64 + lane of (row frequency k1, column frequency k2) and
+// axis-0 tap e <= 2 r t (zero above), as k_gen_spectrum_real forms them from the coefficients of z^e of
+// (sum_e0 z^e0 sum g[e0][e1][e2] exp(i (w1 e1 + w2 e2)))^t and its mirror (w2 -> -w2).  FP64 order (row q + 4v) or
+// FP32 order (row 4q + v).  Then the operands: 16 x 16 cosine and sine matrices, FP64 chunks or BF16 pairings.
+constexpr int kStreamMaxE = 7;
+__global__ void k_gen_stream3d(void* H, int32_t mixed, int32_t E, const double* taps, int32_t K, int32_t convention,
+                               int32_t t) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= 4 * kLanes) return;
+  const int lane = x % kLanes, v = x / kLanes;
+  const int k1 = mixed ? 4 * (lane >> 4) + v : (lane >> 4) + 4 * v, k2 = lane & 15;
+  double L[2][2][kStreamMaxE];  // [w2, -w2][re, im][tap]
+  for (int sgn = 0; sgn < 2; sgn++) {
+    double one[2][kStreamMaxE] = {}, pw[2][kStreamMaxE] = {};
+    for (int a0 = 0; a0 < K; a0++)
+      for (int a1 = 0; a1 < K; a1++)
+        for (int a2 = 0; a2 < K; a2++) {
+          const double w = taps[(a0 * K + a1) * K + a2];
+          if (w == 0.0) continue;
+          const int e0 = convention == 0 ? K - 1 - a0 : a0, e1 = convention == 0 ? K - 1 - a1 : a1;
+          const int e2 = convention == 0 ? K - 1 - a2 : a2;
+          int m = (2 * k1 + 1) * e1 + (sgn ? -1 : 1) * (2 * k2 + 1) * e2;
+          m = ((m % 64) + 64) % 64;
+          double s, c;
+          sincospi((double)m / 32.0, &s, &c);
+          one[0][e0] += w * c;
+          one[1][e0] += w * s;
+        }
+    pw[0][0] = 1.0;
+    for (int n = 0; n < t; n++) {  // pw *= one (degree n (K - 1) before)
+      double nr[kStreamMaxE] = {}, ni[kStreamMaxE] = {};
+      for (int i = 0; i <= n * (K - 1); i++)
+        for (int e = 0; e < K && i + e < kStreamMaxE; e++) {
+          nr[i + e] += pw[0][i] * one[0][e] - pw[1][i] * one[1][e];
+          ni[i + e] += pw[0][i] * one[1][e] + pw[1][i] * one[0][e];
+        }
+      for (int i = 0; i < kStreamMaxE; i++) {
+        pw[0][i] = nr[i];
+        pw[1][i] = ni[i];
+      }
+    }
+    for (int i = 0; i < kStreamMaxE; i++) {
+      L[sgn][0][i] = pw[0][i];
+      L[sgn][1][i] = pw[1][i];
+    }
+  }
+  const double norm = 0.5 / 256.0;
+  for (int e = 0; e < E; e++) {
+    const double h[4] = {(L[0][0][e] + L[1][0][e]) * norm, (L[1][0][e] - L[0][0][e]) * norm,
+                         (L[0][1][e] + L[1][1][e]) * norm, (L[0][1][e] - L[1][1][e]) * norm};
+    for (int i = 0; i < 4; i++) {
+      if (mixed)
+        static_cast<float*>(H)[(e * 4 * kLanes + x) * 4 + i] = (float)h[i];
+      else
+        static_cast<double*>(H)[(e * 4 * kLanes + x) * 4 + i] = h[i];
+    }
+  }
+}
+
+// BF16 pairings of the 16 x 16 cosine and sine matrices: [cos, sin][(h|h), (m|m), (l|h)][lane] of 4 words, element
+// e of lane (j + 16q): row 4q + (e & 3), column j, term (e < 4 ? first : second).
+__global__ void k_gen_operands_fold(uint32_t* t) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= 6 * kLanes) return;
+  const int lane = idx % kLanes, g = (idx / kLanes) % 3, sine = idx / (3 * kLanes);
+  for (int w = 0; w < 4; w++) {
+    uint32_t word = 0;
+    for (int half = 0; half < 2; half++) {
+      const int e = 2 * w + half;
+      const int row = 4 * (lane >> 4) + (e & 3), col = lane & 15;
+      double s, c;
+      sincospi((double)(((2 * row + 1) * (2 * col + 1)) % 128) / 64.0, &s, &c);
+      __bf16 h, m, l;
+      split3_bf16(sine ? s : c, h, m, l);
+      const __bf16 first[3] = {h, m, l}, second[3] = {h, m, h};
+      word |= (uint32_t)__builtin_bit_cast(uint16_t, e < 4 ? first[g] : second[g]) << (16 * half);
+    }
+    t[idx * 4 + w] = word;
+  }
+}
+
+hipError_t gen_stream3d(void* H, bool mixed, int32_t E, const double* d_taps, int32_t K, int32_t convention, int32_t t,
+                        hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_stream3d, dim3(4), dim3(64), 0, s, H, (int32_t)mixed, E, d_taps, K, convention, t);
+  return hipGetLastError();
+}
+hipError_t gen_operands_fold(uint32_t* ops, hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_operands_fold, dim3(6), dim3(64), 0, s, ops);
+  return hipGetLastError();
+}
+
+hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, hipStream_t s) {
+  const int64_t units = a.tiles1 * a.tiles2 * a.nseg;
+  const dim3 g((unsigned)((units + 3) / 4)), b(256);
+  if (precision == 0 && E == 3)
+    hipLaunchKernelGGL((k_stream3d<0, 3>), g, b, 0, s, a);
+  else if (precision == 0 && E == 5)
+    hipLaunchKernelGGL((k_stream3d<0, 5>), g, b, 0, s, a);
+  else if (precision == PREC_BF16 && E == 3)
+    hipLaunchKernelGGL((k_stream3d<PREC_BF16, 3>), g, b, 0, s, a);
+  else if (precision == PREC_BF16 && E == 5)
+    hipLaunchKernelGGL((k_stream3d<PREC_BF16, 5>), g, b, 0, s, a);
+  else if (precision == PREC_BF16 && E == 7)
+    hipLaunchKernelGGL((k_stream3d<PREC_BF16, 7>), g, b, 0, s, a);
+  else
+    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

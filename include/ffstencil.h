@@ -132,8 +132,10 @@ typedef struct ffs_plan_info {
   int32_t fuse_tail;      /* T mod t (0 = no tail block) */
   int64_t blocks;         /* fused blocks per run, tail included */
   int64_t tiles;          /* tiles per block */
-  int64_t launches;       /* kernel launches per run: `blocks`, or half of them (rounded up) where the mixed
-                             2D forms take two blocks per launch on 64-point windows (V <= 16, blocks >= 2) */
+  int64_t launches;       /* kernel launches per run: `blocks`; half of them (rounded up) where the mixed 2D
+                             forms take two blocks per launch on 64-point windows (V <= 16, blocks >= 2); in 3D
+                             (FP64, BF16) those of the streamed kernel, whose depth is its own, on grids where
+                             it is the faster one.  ffs_run_block always runs one block of depth `fuse`. */
   double flops_per_block; /* flops one block executes: matrix-core flops (FFT; see the kernels' header
                              comment) or FP64 FMA flops including the halo recomputation (DIRECT) */
   double bytes_per_block; /* algorithmic HBM bytes of one block: 16 B per grid point */

@@ -334,3 +334,29 @@ def test_3d_mappings_bitwise_equal(ffs, oracle, torch_cuda, precision):
             assert info["mapping"] == (2 if precision == "fp64" else 1), info
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
     assert oracle.errors(outs[0], oracle.sweep(x, r, w, 5))[1] <= (1e-12 if precision == "fp64" else 1e-6)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("bf16", 1e-6)])
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,sizes,steps", [(1, (150, 131, 139), 7), (1, (127, 130, 141), 12), (1, (3, 400, 380), 5),
+                                                (1, (260, 78, 84), 2), (2, (121, 113, 140), 3), (3, (90, 131, 157), 2),
+                                                (1, (129, 257, 65), 1)])
+def test_3d_streamed(ffs, oracle, torch_cuda, precision, tol, convention, radius, sizes, steps):
+    """3D grids large enough for the streamed kernel: every tap count (3, 5, 7), main and tail depths, planes one
+    past and one short of a multiple of the valid width, segments of unequal length, fewer planes than
+    the stencil reaches (3), signed taps."""
+    torch = torch_cuda
+    rng = np.random.default_rng(40 * radius + steps)
+    w = rng.standard_normal((2 * radius + 1) ** 3)
+    w += 2.0 * np.abs(w).sum() / w.size
+    w /= w.sum()
+    x = oracle.uniform(300 + steps, sizes)
+    d_in = torch.from_numpy(x).cuda()
+    d_out = torch.empty_like(d_in)
+    with ffs.Plan(3, sizes, w, radius, steps, precision=precision, convention=convention) as plan:
+        plan.run(d_in, d_out)
+        torch.cuda.synchronize()
+        info = plan.info
+    ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
+    rel = oracle.errors(d_out.cpu().numpy(), ref)[1]
+    assert rel <= tol, (precision, convention, radius, sizes, steps, info, rel)
