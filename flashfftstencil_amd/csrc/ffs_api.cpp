@@ -77,6 +77,7 @@ struct ffs_plan {
   int64_t tiles[3] = {1, 1, 1};
   int64_t units = 0;  // work units of one block: tiles (32-point FP64 family) or tile pairs
   int32_t h_main[3] = {0, 0, 0}, h_tail[3] = {0, 0, 0};
+  char* d_tables = nullptr;  // one allocation, which holds every table below (null where a table is not used)
   void* d_opsi = nullptr;  // 32-point family with V <= 16: inverse operands of the main and tail depths
   double* d_ops = nullptr;
   uint32_t* d_opsm = nullptr;  // mixed-form operand table
@@ -456,13 +457,7 @@ void release(ffs_plan* pl) {
   if (!pl) return;
   for (ffs_plan::GraphSlot& g : pl->graphs) drop_graph(g);
   if (pl->cap_stream) (void)hipStreamDestroy(pl->cap_stream);
-  if (pl->d_ops) (void)hipFree(pl->d_ops);
-  if (pl->d_opsm) (void)hipFree(pl->d_opsm);
-  if (pl->d_opsi) (void)hipFree(pl->d_opsi);
-  if (pl->d_H) (void)hipFree(pl->d_H);
-  if (pl->d_Hf) (void)hipFree(pl->d_Hf);
-  if (pl->d_wide) (void)hipFree(pl->d_wide);
-  if (pl->d_taps) (void)hipFree(pl->d_taps);
+  if (pl->d_tables) (void)hipFree(pl->d_tables);
   if (pl->d_scratch) (void)hipFree(pl->d_scratch);
   delete pl;
 }
@@ -671,21 +666,39 @@ ffs_status plan_host(const ffs_problem* p, ffs_plan* pl) {
   return choose_config(pl);
 }
 
+// CU count of a device that is a gfx950, else 0 with the reason in `arch`.  Asked once per device (a query
+// takes longer than a small run's launches).
+struct DeviceFacts {
+  std::once_flag once;
+  hipError_t err = hipSuccess;
+  int num_cus = 0;
+  char arch[32] = {};
+};
+constexpr int kMaxDevices = 256;
+DeviceFacts g_devices[kMaxDevices];
+
 // The plan's device exists and is a gfx950; makes it current and records its CU count (no allocation).
 ffs_status plan_device(ffs_plan* pl) {
   int ndev = 0;
   const hipError_t ce = hipGetDeviceCount(&ndev);
   if (ce != hipSuccess || ndev <= 0)
     return fail(FFS_ERR_NO_DEVICE, "no HIP device visible (%s, count %d)", hipGetErrorString(ce), ndev);
-  if (pl->prob.device < 0 || pl->prob.device >= ndev)
+  if (pl->prob.device < 0 || pl->prob.device >= ndev || pl->prob.device >= kMaxDevices)
     return fail(FFS_ERR_INVALID_ARG, "device %d out of range (%d devices)", pl->prob.device, ndev);
   pl->dev = pl->prob.device;
-  hipDeviceProp_t prop;
-  if (hipSetDevice(pl->dev) != hipSuccess || hipGetDeviceProperties(&prop, pl->dev) != hipSuccess)
-    return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
-  if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
-    return fail(FFS_ERR_NO_DEVICE, "device %d is %s; this library is built for gfx950 only", pl->dev, prop.gcnArchName);
-  pl->num_cus = prop.multiProcessorCount;
+  if (hipSetDevice(pl->dev) != hipSuccess) return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
+  DeviceFacts& f = g_devices[pl->dev];
+  std::call_once(f.once, [&] {
+    hipDeviceProp_t prop;
+    f.err = hipGetDeviceProperties(&prop, pl->dev);
+    if (f.err != hipSuccess) return;
+    std::snprintf(f.arch, sizeof f.arch, "%.*s", 31, prop.gcnArchName);
+    f.num_cus = prop.multiProcessorCount;
+  });
+  if (f.err != hipSuccess) return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
+  if (std::strncmp(f.arch, "gfx950", 6) != 0)
+    return fail(FFS_ERR_NO_DEVICE, "device %d is %s; this library is built for gfx950 only", pl->dev, f.arch);
+  pl->num_cus = f.num_cus;
   return FFS_OK;
 }
 
@@ -728,21 +741,37 @@ ffs_status plan_constants(ffs_plan* pl) {
     pl->dc_wide_tail = ipow(sw, pl->t_wide_tail);
   }
   if (p.precision == FFS_PREC_MIXED_F16) {
-    // largest |K(k)| over the 32 x 32 frequencies (direct DFT of the taps; |K| does not depend on the
-    // convention), then scale_exp = floor(10 - log2 max(1, |K|^t)) for each depth
+    // largest |K(k)| over the 32 x 32 frequencies (|K| does not depend on the convention), axis by axis from
+    // the 32 distinct angles, then scale_exp = floor(10 - log2 max(1, |K|^t)) for each depth
     double kmax = 0.0;
     const int P = 32;
-    for (int k0 = 0; k0 < P; k0++)
-      for (int k1 = 0; k1 < P; k1++) {
+    double co[P], si[P];
+    for (int m = 0; m < P; m++) {
+      co[m] = std::cos(-2.0 * M_PI * (double)m / P);
+      si[m] = std::sin(-2.0 * M_PI * (double)m / P);
+    }
+    std::vector<double> gr((size_t)K), gi((size_t)K);
+    for (int k1 = 0; k1 < P; k1++) {
+      for (int a0 = 0; a0 < K; a0++) {
         double re = 0.0, im = 0.0;
-        for (int a0 = 0; a0 < K; a0++)
-          for (int a1 = 0; a1 < K; a1++) {
-            const double ang = -2.0 * M_PI * (double)((a0 * k0 + a1 * k1) % P) / P;
-            re += pl->weights[a0 * K + a1] * std::cos(ang);
-            im += pl->weights[a0 * K + a1] * std::sin(ang);
-          }
+        for (int a1 = 0; a1 < K; a1++) {
+          const double w = pl->weights[(size_t)(a0 * K + a1)];
+          re += w * co[(a1 * k1) % P];
+          im += w * si[(a1 * k1) % P];
+        }
+        gr[(size_t)a0] = re;
+        gi[(size_t)a0] = im;
+      }
+      for (int k0 = 0; k0 < P; k0++) {
+        double re = 0.0, im = 0.0;
+        for (int a0 = 0; a0 < K; a0++) {
+          const int m = (a0 * k0) % P;
+          re += gr[(size_t)a0] * co[m] - gi[(size_t)a0] * si[m];
+          im += gr[(size_t)a0] * si[m] + gi[(size_t)a0] * co[m];
+        }
         kmax = std::max(kmax, std::sqrt(re * re + im * im));
       }
+    }
     auto expo = [&](int64_t t) {
       const double lg = kmax > 1.0 ? (double)t * std::log2(kmax) : 0.0;
       return std::floor(10.0 - lg);
@@ -797,9 +826,29 @@ TableSizes table_sizes(const ffs_plan* pl) {
   return t;
 }
 
+// Points the plan's tables into one allocation at `base` (256-byte steps); returns the bytes they take.
+size_t place_tables(ffs_plan* pl, const TableSizes& t, char* base) {
+  size_t off = 0;
+  auto at = [&](size_t n) -> char* {
+    if (!n) return nullptr;
+    char* p = base ? base + off : nullptr;  // no base yet: only the size is asked for
+    off += (n + 255) & ~size_t(255);
+    return p;
+  };
+  pl->d_ops = reinterpret_cast<double*>(at(t.ops));
+  pl->d_opsm = reinterpret_cast<uint32_t*>(at(t.opsm));
+  pl->d_H = reinterpret_cast<double*>(at(t.H));
+  pl->d_Hf = reinterpret_cast<float*>(at(t.Hf));
+  pl->d_opsi = at(t.opsi);
+  pl->d_taps = reinterpret_cast<double*>(at(t.taps));
+  pl->d_wide = reinterpret_cast<uint32_t*>(at(t.wide));
+  return off;
+}
+
 // Operands and spectra into the plan's device tables, on stream s (the taps are already in d_taps).
+// run_only: those that ffs_run reads, without the ones only ffs_run_block needs.
 hipError_t dft_tables(const ffs_plan* pl, hipStream_t s);
-hipError_t plan_tables(const ffs_plan* pl, hipStream_t s) {
+hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
   const ffs_problem& p = pl->prob;
   const int K = 2 * p.radius + 1;
   if (pl->wide) {
@@ -822,6 +871,7 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s) {
                              (int32_t)pl->stream_tail, s);
     if (e != hipSuccess) return e;
   }
+  if (run_only && (pl->wide || pl->stream)) return hipSuccess;
   if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
   if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);
@@ -1007,13 +1057,8 @@ ffs_status ffs_plan_create(const ffs_problem* p, ffs_plan** out) {
   };
   const TableSizes ts = table_sizes(pl);
   if (!pl->direct) {
-    chk(hipMalloc(&pl->d_ops, ts.ops));
-    if (ts.opsm) chk(hipMalloc(&pl->d_opsm, ts.opsm));
-    chk(hipMalloc(&pl->d_H, ts.H));
-    if (ts.Hf) chk(hipMalloc(&pl->d_Hf, ts.Hf));
-    if (ts.opsi) chk(hipMalloc(&pl->d_opsi, ts.opsi));
-    if (ts.wide) chk(hipMalloc(&pl->d_wide, ts.wide));
-    chk(hipMalloc(&pl->d_taps, ts.taps));
+    chk(hipMalloc(&pl->d_tables, place_tables(pl, ts, nullptr)));
+    if (e == hipSuccess) place_tables(pl, ts, pl->d_tables);
   }
   if (run_launches(pl) >= 2) chk(hipMalloc(&pl->d_scratch, sizeof(double) * pl->npoints));
   if (e != hipSuccess) {
@@ -1023,7 +1068,7 @@ ffs_status ffs_plan_create(const ffs_problem* p, ffs_plan** out) {
   }
   if (!pl->direct) {
     chk(hipMemcpy(pl->d_taps, pl->weights.data(), ts.taps, hipMemcpyHostToDevice));
-    chk(plan_tables(pl, nullptr));
+    chk(plan_tables(pl, nullptr, false));
     chk(hipDeviceSynchronize());
   }
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&pl->cap_stream, hipStreamNonBlocking);
@@ -1254,14 +1299,7 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
   if (st == FFS_OK) st = plan_constants(&pl);
   if (st != FFS_OK) return st;
   const TableSizes ts = table_sizes(&pl);
-  size_t off = 0;
-  auto carve = [&](size_t n) {
-    const size_t at = off;
-    off += (n + 255) & ~size_t(255);
-    return at;
-  };
-  const size_t o_ops = carve(ts.ops), o_opsm = carve(ts.opsm), o_H = carve(ts.H), o_Hf = carve(ts.Hf),
-               o_opsi = carve(ts.opsi), o_taps = carve(ts.taps), o_wide = carve(ts.wide);
+  const size_t off = pl.direct ? 0 : place_tables(&pl, ts, nullptr);
   if (off > FFS_STATIC_TABLE_BYTES)
     return fail(FFS_ERR_INTERNAL, "plan tables need %zu bytes of the %llu reserved", off, FFS_STATIC_TABLE_BYTES);
   const size_t grid_bytes = pl.nblocks >= 2 ? sizeof(double) * (size_t)pl.npoints : 0;
@@ -1275,20 +1313,12 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
   st = static_scratch(pl.dev, &base);
   if (st != FFS_OK) return st;
   char* b = static_cast<char*>(base);
-  if (!pl.direct) {
-    pl.d_ops = reinterpret_cast<double*>(b + o_ops);
-    pl.d_opsm = ts.opsm ? reinterpret_cast<uint32_t*>(b + o_opsm) : nullptr;
-    pl.d_H = reinterpret_cast<double*>(b + o_H);
-    pl.d_Hf = ts.Hf ? reinterpret_cast<float*>(b + o_Hf) : nullptr;
-    pl.d_opsi = ts.opsi ? static_cast<void*>(b + o_opsi) : nullptr;
-    pl.d_taps = reinterpret_cast<double*>(b + o_taps);
-    pl.d_wide = ts.wide ? reinterpret_cast<uint32_t*>(b + o_wide) : nullptr;
-  }
+  if (!pl.direct) place_tables(&pl, ts, b);
   pl.d_scratch = grid_bytes ? reinterpret_cast<double*>(b + FFS_STATIC_TABLE_BYTES) : nullptr;
   hipStream_t s = (hipStream_t)stream;
   if (!pl.direct) {
     hipError_t e = ffsk::put_taps(pl.d_taps, pl.weights.data(), (int64_t)pl.weights.size(), s);
-    if (e == hipSuccess) e = plan_tables(&pl, s);
+    if (e == hipSuccess) e = plan_tables(&pl, s, true);
     if (e != hipSuccess) return fail(FFS_ERR_HIP, "table generation failed: %s", hipGetErrorString(e));
   }
   if (pl.nblocks == 0) {

@@ -2521,6 +2521,13 @@ __device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
 }
 __global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int32_t K, int32_t convention,
                                     int64_t t) {
+  __shared__ double2 root[128];  // exp(i pi m / P), m < 2P <= 128
+  for (int m = threadIdx.x; m < 2 * P; m += blockDim.x) {
+    double s, c;
+    sincospi((double)m / (double)P, &s, &c);
+    root[m] = make_double2(c, s);
+  }
+  __syncthreads();
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= P * P / 4) return;
   const int lane = e % kLanes, v = (e / kLanes) % 4, b = e / (4 * kLanes);
@@ -2532,16 +2539,12 @@ __global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int3
       const double w = taps[a0 * K + a1];
       if (w == 0.0) continue;
       const int e0 = convention == 0 ? K - 1 - a0 : a0, e1 = convention == 0 ? K - 1 - a1 : a1;
-      const int64_t x0 = (int64_t)(2 * k0 + 1) * e0, x1 = (int64_t)(2 * k1 + 1) * e1;
-      const int64_t m1 = (x0 + x1) % (2 * P);
-      const int64_t m2 = (((x0 - x1) % (2 * P)) + 2 * P) % (2 * P);
-      double s, c;
-      sincospi((double)m1 / (double)P, &s, &c);
-      L1r += w * c;
-      L1i += w * s;
-      sincospi((double)m2 / (double)P, &s, &c);
-      L2r += w * c;
-      L2i += w * s;
+      const int x0 = (2 * k0 + 1) * e0, x1 = (2 * k1 + 1) * e1;
+      const double2 u1 = root[(x0 + x1) & (2 * P - 1)], u2 = root[(x0 - x1) & (2 * P - 1)];
+      L1r += w * u1.x;
+      L1i += w * u1.y;
+      L2r += w * u2.x;
+      L2i += w * u2.y;
     }
   cpow_t(L1r, L1i, t);
   cpow_t(L2r, L2i, t);
