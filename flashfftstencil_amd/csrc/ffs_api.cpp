@@ -95,6 +95,11 @@ struct ffs_plan {
   int32_t stream_E = 0, stream_V = 0, stream_nseg = 1;
   int64_t stream_t = 0, stream_tail = 0, stream_seg = 0;
   double stream_dc[2][7] = {};
+  // 1D FP64 and BF16 plans: launches of depth line_t as one banded product (ffsk::launch_line), the last one of
+  // depth line_tail; line_nb contraction blocks.  d_wide holds both depths' taps, then (BF16) their operands.
+  bool line = false;
+  int32_t line_nb = 0;
+  int64_t line_t = 0, line_tail = 0;
   int32_t scale_wide = 0, scale_wide_tail = 0;
   double dc_main = 1.0, dc_tail = 1.0;  // K(0)^t and K(0)^t_tail
   int32_t scale_main = 0, scale_tail = 0;  // FP16 form: scale exponents of the main and tail depths
@@ -302,8 +307,37 @@ void choose_stream(ffs_plan* pl) {
   if (pl->stream) pl->stream_tail = p.steps % pl->stream_t;
 }
 
+// 1D runs by banded products: depth per launch, from the modelled time of the run (SIMD cycles): per launch 8,000,
+// plus 6,000 for a wave's chain of load, product and store, plus the larger of the memory time (16 B per point at
+// 5.3 TB/s) and the products (FP64: 256 cycles per block of 16 and tile; BF16: 120 per block of 32 and tile, LDS reads
+// included, and 250 for the tile's split).
+void choose_line(ffs_plan* pl) {
+  const ffs_problem& p = pl->prob;
+  const int64_t r = p.radius;
+  const bool fp64 = p.precision == FFS_PREC_FP64;
+  if (p.dims != 1 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
+  const int64_t block = fp64 ? 16 : 32, nbmax = fp64 ? ffsk::kLineMaxNb64 : ffsk::kLineMaxNbBF;
+  const int64_t most = std::min<int64_t>(ffsk::kLineMaxTaps, block * nbmax - 15);
+  double best = 1e300;
+  for (int64_t t = 1; 2 * r * t + 1 <= most && t <= p.steps; t++) {
+    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
+    const int64_t nb = (2 * r * te + 16 + block - 1) / block;
+    const double n = (double)p.sizes[0];
+    const double work = std::ceil(n / 256.0 / 1024.0) * (fp64 ? (double)nb * 256.0 : (double)nb * 120.0 + 250.0);
+    const double cost = (double)nl * (14000.0 + std::max(work, 16.0 * n / 5.3e12 * 2.4e9));
+    if (cost < best * (1 - 1e-9) && nl <= pl->nblocks) {
+      best = cost;
+      pl->line = true;
+      pl->line_t = te;
+      pl->line_nb = (int32_t)nb;
+    }
+  }
+  if (pl->line) pl->line_tail = p.steps % pl->line_t;
+}
+
 // Launches of one run.
 int64_t run_launches(const ffs_plan* pl) {
+  if (pl->line) return (pl->prob.steps + pl->line_t - 1) / pl->line_t;
   if (pl->stream) return (pl->prob.steps + pl->stream_t - 1) / pl->stream_t;
   return pl->wide ? (pl->prob.steps + 2 * pl->t - 1) / (2 * pl->t) : pl->nblocks;
 }
@@ -444,6 +478,7 @@ ffs_status choose_config(ffs_plan* pl) {
   pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2;
   if (pl->wide) pl->t_wide_tail = p.steps % (2 * pl->t);
   choose_stream(pl);
+  choose_line(pl);
   return FFS_OK;
 }
 
@@ -536,6 +571,26 @@ ffsk::TileArgs make_wide_args(const ffs_plan* pl, const double* src, double* dst
   a.opsm = pl->d_wide;
   a.Hf = reinterpret_cast<const float*>(pl->d_wide + ffsk::kOpsWide) + (tail ? ffsk::kSpecWide : 0);
   a.scale_exp = tail ? pl->scale_wide_tail : pl->scale_wide;
+  a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
+  return a;
+}
+
+size_t line_ops_bytes(const ffs_plan* pl) {
+  return pl->prob.precision == FFS_PREC_FP64 ? 0 : (size_t)pl->line_nb * 3 * ffsk::kLanes * 16;
+}
+
+ffsk::LineArgs make_line_args(const ffs_plan* pl, const double* src, double* dst, bool tail) {
+  const ffs_problem& p = pl->prob;
+  const int64_t t = tail ? pl->line_tail : pl->line_t;
+  ffsk::LineArgs a{};
+  a.src = src;
+  a.dst = dst;
+  a.taps = reinterpret_cast<const double*>(pl->d_wide) + (tail ? ffsk::kLineMaxTaps : 0);
+  a.ops = reinterpret_cast<const char*>(pl->d_wide) + 2 * sizeof(double) * ffsk::kLineMaxTaps + (tail ? line_ops_bytes(pl) : 0);
+  a.n = p.sizes[0];
+  a.h = (p.convention == FFS_CONV_REF ? 2 * p.radius : p.radius) * t;
+  a.taps_n = (int32_t)(2 * p.radius * t + 1);
+  a.nb = pl->line_nb;
   a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
   return a;
 }
@@ -639,7 +694,9 @@ ffs_status enqueue_chain(ffs_plan* pl, const double* d_in, double* d_out, hipStr
   for (int64_t b = 0; b < nb; b++) {
     double* dst = ((nb - 1 - b) % 2 == 0) ? d_out : pl->d_scratch;
     const bool last = b == nb - 1;
-    hipError_t e = pl->stream ? ffsk::launch_stream3d(make_stream_args(pl, src, dst, last && pl->stream_tail > 0),
+    hipError_t e = pl->line ? ffsk::launch_line(make_line_args(pl, src, dst, last && pl->line_tail > 0),
+                                                pl->prob.precision, s, pl->num_cus)
+                   : pl->stream ? ffsk::launch_stream3d(make_stream_args(pl, src, dst, last && pl->stream_tail > 0),
                                                       pl->prob.precision, pl->stream_E, s)
                    : pl->wide ? ffsk::launch_wide(make_wide_args(pl, src, dst, last && pl->t_wide_tail > 0), s, pl->num_cus)
                             : launch_one_block(pl, src, dst, last && pl->t_tail > 0, s);
@@ -737,8 +794,8 @@ ffs_status plan_constants(ffs_plan* pl) {
         std::memcpy(pl->stream_dc[d], g, sizeof g);
       }
     }
-    pl->dc_wide = ipow(sw, 2 * pl->t);
-    pl->dc_wide_tail = ipow(sw, pl->t_wide_tail);
+    pl->dc_wide = ipow(sw, pl->line ? pl->line_t : 2 * pl->t);
+    pl->dc_wide_tail = ipow(sw, pl->line ? pl->line_tail : pl->t_wide_tail);
   }
   if (p.precision == FFS_PREC_MIXED_F16) {
     // largest |K(k)| over the 32 x 32 frequencies (|K| does not depend on the convention), axis by axis from
@@ -822,6 +879,7 @@ TableSizes table_sizes(const ffs_plan* pl) {
     t.opsi = 0;
   }
   if (pl->wide) t.wide = sizeof(uint32_t) * ffsk::kOpsWide + sizeof(float) * 2 * ffsk::kSpecWide;
+  if (pl->line) t.wide = 2 * (sizeof(double) * ffsk::kLineMaxTaps + line_ops_bytes(pl));
   if (pl->stream) t.wide = stream_ops_bytes(pl) + 2 * stream_spec_bytes(pl);
   return t;
 }
@@ -871,7 +929,18 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
                              (int32_t)pl->stream_tail, s);
     if (e != hipSuccess) return e;
   }
-  if (run_only && (pl->wide || pl->stream)) return hipSuccess;
+  if (pl->line) {
+    double* g = reinterpret_cast<double*>(pl->d_wide);
+    char* ops = reinterpret_cast<char*>(pl->d_wide) + 2 * sizeof(double) * ffsk::kLineMaxTaps;
+    const size_t n = line_ops_bytes(pl);
+    hipError_t e = ffsk::gen_line(g, n ? reinterpret_cast<uint32_t*>(ops) : nullptr, pl->d_taps, K, p.convention,
+                                  (int32_t)pl->line_t, pl->line_nb, s);
+    if (e == hipSuccess && pl->line_tail > 0)
+      e = ffsk::gen_line(g + ffsk::kLineMaxTaps, n ? reinterpret_cast<uint32_t*>(ops + n) : nullptr, pl->d_taps, K,
+                         p.convention, (int32_t)pl->line_tail, pl->line_nb, s);
+    if (e != hipSuccess) return e;
+  }
+  if (run_only && (pl->wide || pl->stream || pl->line)) return hipSuccess;
   if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
   if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);

@@ -136,6 +136,22 @@ hipError_t gen_spectrum(double* H, int kind, int layout, const int32_t* axis_len
 // Hf[2e], Hf[2e + 1] = (float)H[e], (float)H[len + e] for e < len: the FP32 copy of one depth's spectrum
 // that the mixed-form kernels read from global memory (the batch kernels and the 3D kernel).
 hipError_t spectrum_to_f32(const double* H, float* Hf, int64_t len, hipStream_t s);
+// One launch of the 1D kernels (FP64, BF16): depth t as one banded Toeplitz product.
+constexpr int kLineMaxTaps = 512;  // taps of the t-fold stencil
+constexpr int kLineMaxNb64 = 32;   // contraction blocks of 16 (FP64) and 32 (BF16): nb blocks hold 16 (32) nb - 15 taps
+constexpr int kLineMaxNbBF = 10;
+struct LineArgs {
+  const double* src;
+  double* dst;
+  const double* taps;  // kLineMaxTaps doubles, zero beyond taps_n
+  const void* ops;     // BF16: operand table
+  int64_t n, h;        // grid length, window offset
+  int32_t taps_n, nb;
+  double dc_gain;      // BF16: sum of the taps
+};
+hipError_t gen_line(double* g, uint32_t* ops, const double* d_taps, int32_t K, int32_t convention, int32_t t, int32_t nb,
+                    hipStream_t s);
+hipError_t launch_line(const LineArgs& a, int32_t precision, hipStream_t s, int num_cus);
 // One launch of the streamed 3D kernels (FP64, BF16): depth t, E = 2 r t + 1 rounded up to an instantiated tap count.
 struct Stream3Args {
   const double* src;

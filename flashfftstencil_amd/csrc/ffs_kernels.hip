@@ -2960,6 +2960,214 @@ hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, h
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------------------------
+// 1D grids: one banded Toeplitz product per launch (FP64 and BF16 forms).
+//
+// t steps are one correlation with the E = 2rt + 1 taps g of the t-fold stencil.  With 16 consecutive outputs as
+// the rows of a matrix and 16 such groups as its columns, a tile of 256 outputs is Y = T X, T[i][k] = g[k - i]
+// (16 x (E + 15), banded) and X[k][j] = x[16 j + k]: a single contraction, E + 15 multiply-adds per output.  The
+// 240-point DFT windows take 4 stages in sequence and 219 FP64 multiply-adds per output at depth 64 (V = 112)
+// against 144 here, and, in the mixed form, split every value four times instead of once.
+//
+// A wave owns one tile (mixed form: M) and stages its window in its own LDS region (mixed form: split into BF16
+// terms, relative to the window's mean c; the store adds c times the sum of g back in FP64).  Rows of T are
+// ordered so that a lane ends with 4 consecutive outputs.
+//
+// FP64 is bound by the matrix pipe (64 cycles per chunk; two tiles per wave, which halve the LDS reads, were 2%
+// slower), BF16 by HBM at the depths it takes (2rt up to 304) with LDS reads close behind.  Heat-1D 2^20 x 64
+// FP64 14.7 -> 10 us, 2^24 x 256 787 -> 320; 1D7P 2^24 x 100 FP64 954 -> 369, BF16 770 -> 184 us.
+// ---------------------------------------------------------------------------------------------
+// FP64: taps in LDS (zero-padded on both sides), operands of both sides read per K = 4 chunk; the window with one
+// pad per 16 values (the column stride).
+__global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
+  extern __shared__ double lds[];
+  const int kk = 16 * a.nb;                    // contraction length
+  double* sT = lds;                            // g[-15 .. kk - 1], zeros outside the taps
+  const int win = 240 + kk;                    // window of a tile
+  const int wstride = win + (win >> 4) + 1;
+  for (int i = threadIdx.x; i < kk + 15; i += blockDim.x) sT[i] = i >= 15 && i - 15 < a.taps_n ? a.taps[i - 15] : 0.0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane >> 4, j = lane & 15;
+  double* sX = lds + kk + 16 + (int64_t)w * wstride;
+  const int row = 4 * (j & 3) + (j >> 2);      // output offset of A row i = j
+  const int64_t units = (a.n + 255) / 256;
+  for (int64_t u = (int64_t)blockIdx.x * 4 + w; u < units; u += (int64_t)gridDim.x * 4) {
+    const int64_t p0 = u * 256, base = p0 - a.h;
+    if (base >= 0 && base + win <= a.n) {
+      for (int i = lane; i < win; i += 64) sX[i + (i >> 4)] = a.src[base + i];
+    } else {
+      for (int i = lane; i < win; i += 64) sX[i + (i >> 4)] = a.src[wrap_near(base + i, a.n)];
+    }
+    d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+    for (int b = 0; b < a.nb; b++) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int k = 16 * b + 4 * c + q;      // this lane's contraction index, in both operands
+        acc[c & 1] = FFS_MFMA64(sT[k - row + 15], sX[17 * (j + b) + 4 * c + q], acc[c & 1]);
+      }
+    }
+    const int64_t p = p0 + 16 * j + 4 * q;
+    const d4 y = acc[0] + acc[1];
+    if (p + 3 < a.n) {
+      *reinterpret_cast<d2u*>(a.dst + p) = d2u{y[0], y[1]};
+      *reinterpret_cast<d2u*>(a.dst + p + 2) = d2u{y[2], y[3]};
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (p + v < a.n) a.dst[p + v] = y[v];
+    }
+  }
+}
+
+// BF16: three-term split of the window (once, into LDS) and of T (operand table, [K = 32 block][term][lane]); the six
+// products of order <= 2^-16, the five small ones summed apart from the dominant one.
+template <int M>
+__global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
+  extern __shared__ double lds[];
+  const int kk = 32 * a.nb;
+  const int win = 256 * M + kk - 16;           // multiple of 16
+  u4* sT = reinterpret_cast<u4*>(lds);
+  for (int i = threadIdx.x; i < a.nb * 3 * kLanes; i += blockDim.x) sT[i] = reinterpret_cast<const u4*>(a.ops)[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane >> 4, j = lane & 15;
+  uint32_t* sX = reinterpret_cast<uint32_t*>(sT + a.nb * 3 * kLanes) + (int64_t)w * 3 * (win / 2);
+  const int64_t units = (a.n + 256 * M - 1) / (256 * M);
+  for (int64_t u = (int64_t)blockIdx.x * 4 + w; u < units; u += (int64_t)gridDim.x * 4) {
+    const int64_t p0 = u * (256 * M), base = p0 - a.h;
+    const bool interior = base >= 0 && base + win <= a.n;
+    // c: mean of 128 values spread over the window
+    const int s0 = (int)((int64_t)lane * (win - 2) / 63);
+    const double c = wave_sum(a.src[interior ? base + s0 : wrap_near(base + s0, a.n)] +
+                              a.src[interior ? base + s0 + 1 : wrap_near(base + s0 + 1, a.n)]) * (1.0 / 128);
+    for (int i = 2 * lane; i < win; i += 128) {
+      double x0, x1;
+      if (interior) {
+        const d2u x = *reinterpret_cast<const d2u*>(a.src + base + i);
+        x0 = x[0];
+        x1 = x[1];
+      } else {
+        x0 = a.src[wrap_near(base + i, a.n)];
+        x1 = a.src[wrap_near(base + i + 1, a.n)];
+      }
+      const float y0 = (float)(x0 - c), y1 = (float)(x1 - c);
+      const uint32_t h = pk_bf16(y0, y1);
+      const float r0 = y0 - bf_lo(h), r1 = y1 - bf_hi(h);
+      const uint32_t m = pk_bf16(r0, r1);
+      sX[i / 2] = h;
+      sX[win / 2 + i / 2] = m;
+      sX[win + i / 2] = pk_bf16(r0 - bf_lo(m), r1 - bf_hi(m));
+    }
+    lds_fence();
+    f4 big[M], small[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) big[m] = small[m] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < a.nb; b++) {
+      bf8 T[3];
+#pragma unroll
+      for (int t = 0; t < 3; t++) T[t] = as_bf8(sT[(b * 3 + t) * kLanes + lane]);
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        // contraction index 8q + e of block b <-> window position 16 (16 m + j) + 32 b + 8q + e
+        const u4* x = reinterpret_cast<const u4*>(sX + (16 * (16 * m + j) + 32 * b + 8 * q) / 2);
+        const bf8 xh = as_bf8(x[0]), xm = as_bf8(x[win / 8]), xl = as_bf8(x[win / 4]);
+        small[m] = FFS_MFMA_BF16(T[2], xh, small[m]);
+        small[m] = FFS_MFMA_BF16(T[1], xm, small[m]);
+        small[m] = FFS_MFMA_BF16(T[0], xl, small[m]);
+        small[m] = FFS_MFMA_BF16(T[1], xh, small[m]);
+        small[m] = FFS_MFMA_BF16(T[0], xm, small[m]);
+        big[m] = FFS_MFMA_BF16(T[0], xh, big[m]);
+      }
+    }
+    const double add = c * a.dc_gain;
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      const int64_t p = p0 + 256 * m + 16 * j + 4 * q;
+      const f4 y = big[m] + small[m];
+      if (p + 3 < a.n) {
+        *reinterpret_cast<d2u*>(a.dst + p) = d2u{(double)y[0] + add, (double)y[1] + add};
+        *reinterpret_cast<d2u*>(a.dst + p + 2) = d2u{(double)y[2] + add, (double)y[3] + add};
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          if (p + v < a.n) a.dst[p + v] = (double)y[v] + add;
+      }
+    }
+  }
+}
+
+// Taps of the t-fold 1D stencil in correlation order (ref: e = 2r - a; centred: e = a), by t - 1 convolutions in
+// FP64; one workgroup.
+__global__ void k_gen_line_taps(double* out, const double* taps, int32_t K, int32_t convention, int32_t t) {
+  __shared__ double buf[2][kLineMaxTaps];
+  const int n = (K - 1) * t + 1;
+  for (int i = threadIdx.x; i < kLineMaxTaps; i += blockDim.x) buf[0][i] = i < K ? taps[convention == 0 ? K - 1 - i : i] : 0.0;
+  __syncthreads();
+  int cur = 0;
+  for (int s = 1; s < t; s++) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+      double sum = 0.0;
+      for (int e = 0; e < K && e <= i; e++) sum = __builtin_fma(taps[convention == 0 ? K - 1 - e : e], buf[cur][i - e], sum);
+      buf[cur ^ 1][i] = sum;
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+  for (int i = threadIdx.x; i < kLineMaxTaps; i += blockDim.x) out[i] = i < n ? buf[cur][i] : 0.0;
+}
+
+// Operands of k_line_bf16: [block b][term][lane] of 4 words; element e of lane (i + 16q) is T[i][32 b + 8q + e] =
+// g[32 b + 8q + e - i].
+__global__ void k_gen_line_ops(uint32_t* t, const double* g, int32_t n, int32_t nb) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= nb * 3 * kLanes) return;
+  const int lane = idx % kLanes, term = (idx / kLanes) % 3, b = idx / (3 * kLanes);
+  for (int w = 0; w < 4; w++) {
+    uint32_t word = 0;
+    for (int half = 0; half < 2; half++) {
+      const int k = 32 * b + 8 * (lane >> 4) + 2 * w + half - (lane & 15);
+      __bf16 h, m, l;
+      split3_bf16(k >= 0 && k < n ? g[k] : 0.0, h, m, l);
+      word |= (uint32_t)__builtin_bit_cast(uint16_t, term == 0 ? h : (term == 1 ? m : l)) << (16 * half);
+    }
+    t[idx * 4 + w] = word;
+  }
+}
+
+hipError_t gen_line(double* g, uint32_t* ops, const double* d_taps, int32_t K, int32_t convention, int32_t t, int32_t nb,
+                    hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_line_taps, dim3(1), dim3(512), 0, s, g, d_taps, K, convention, t);
+  if (ops)
+    hipLaunchKernelGGL(k_gen_line_ops, dim3((unsigned)nb), dim3(3 * kLanes), 0, s, ops, g, (K - 1) * t + 1, nb);
+  return hipGetLastError();
+}
+
+template <int M>
+void launch_line_bf16(const LineArgs& a, hipStream_t s, int num_cus) {
+  const size_t win = 256 * M + 32 * (size_t)a.nb - 16;
+  const size_t lds = (size_t)a.nb * 3 * kLanes * 16 + 4 * 3 * (win / 2) * 4;
+  const int64_t per = 4 * 256 * M, resident = std::max<int64_t>(1, std::min<int64_t>(4, (int64_t)(160 * 1024 / lds)));
+  const dim3 g((unsigned)std::min<int64_t>((a.n + per - 1) / per, (int64_t)num_cus * resident)), b(256);
+  hipLaunchKernelGGL(k_line_bf16<M>, g, b, lds, s, a);
+}
+
+hipError_t launch_line(const LineArgs& a, int32_t precision, hipStream_t s, int num_cus) {
+  if (precision == 0) {
+    const size_t kk = 16 * (size_t)a.nb, win = 240 + kk, lds = 8 * (kk + 16 + 4 * (win + (win >> 4) + 1));
+    const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)(160 * 1024 / lds)));
+    const dim3 g((unsigned)std::min<int64_t>((a.n + 1023) / 1024, (int64_t)num_cus * resident)), b(256);
+    hipLaunchKernelGGL(k_line_f64, g, b, lds, s, a);
+  } else if (a.n > 4096 * (int64_t)num_cus * 4) {
+    // Two tiles per wave share the operand reads (1D7P 2^24 x 100: 184 us, one tile 207, four 209) once every SIMD
+    // has eight such waves; below that one tile per wave keeps its chain short (2,000,000 x 64: 39.8 against 40.6).
+    launch_line_bf16<2>(a, s, num_cus);
+  } else {
+    launch_line_bf16<1>(a, s, num_cus);
+  }
+  return hipGetLastError();
+}
+
 struct TapChunk {
   double w[kTapsPerLaunch];
   int32_t n;

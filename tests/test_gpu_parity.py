@@ -360,3 +360,44 @@ def test_3d_streamed(ffs, oracle, torch_cuda, precision, tol, convention, radius
     ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
     rel = oracle.errors(d_out.cpu().numpy(), ref)[1]
     assert rel <= tol, (precision, convention, radius, sizes, steps, info, rel)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("bf16", 1e-6)])
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,n,steps", [(1, 256, 7), (1, 257, 8), (1, 255, 9), (1, 1023, 64), (3, 10, 50), (1, 1, 3),
+                                            (2, 4099, 130), (1, 5000, 248), (12, 1500, 30), (40, 700, 2), (60, 2000, 9)])
+def test_1d_banded_product(ffs, oracle, torch_cuda, precision, tol, convention, radius, n, steps):
+    """1D runs as banded products: grids around a tile of 256 outputs, smaller than the stencil's reach, numbers of
+    taps around a multiple of the contraction block (2rt + 16 = 16 b, 32 b and one past), up to the deepest launch and past it
+    (a tail of another depth), wide stencils, signed taps."""
+    torch = torch_cuda
+    rng = np.random.default_rng(radius + steps)
+    w = rng.standard_normal(2 * radius + 1)
+    w += 2.0 * np.abs(w).sum() / w.size
+    w /= w.sum()
+    x = oracle.uniform(70 + n, (n,))
+    d_in = torch.from_numpy(x).cuda()
+    d_out = torch.empty_like(d_in)
+    with ffs.Plan(1, (n,), w, radius, steps, precision=precision, convention=convention) as plan:
+        plan.run(d_in, d_out)
+        torch.cuda.synchronize()
+        info = plan.info
+    ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
+    rel = oracle.errors(d_out.cpu().numpy(), ref)[1]
+    assert rel <= tol, (precision, convention, radius, n, steps, info, rel)
+
+
+def test_1d_banded_product_large(ffs, torch_cuda):
+    """The two-tile variant of the mixed kernel (above 4 Mi points) against the FP64 form, a ragged length."""
+    torch = torch_cuda
+    _, r, w, _ = ffs.named_stencil("1D7P", seed=2)
+    d_in = torch.empty((1 << 22) + 8191, dtype=torch.float64, device="cuda")
+    ffs.fill_uniform_device(3, d_in)
+    outs = []
+    for precision in ("bf16", "fp64"):
+        with ffs.Plan(1, tuple(d_in.shape), w, r, 71, precision=precision) as plan:
+            d = torch.empty_like(d_in)
+            plan.run(d_in, d)
+            torch.cuda.synchronize()
+        outs.append(d)
+    assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) <= 1e-6
