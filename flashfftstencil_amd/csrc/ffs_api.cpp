@@ -211,6 +211,61 @@ bool star_support(const ffs_plan* pl) {
   return true;
 }
 
+// 1D runs by banded products: depth per launch, from the modelled time of the run (SIMD cycles): per launch 8,000,
+// plus 6,000 for a wave's chain of load, product and store, plus the larger of the memory time (16 B per point at
+// 5.3 TB/s) and the products (FP64: 256 cycles per block of 16 and tile; BF16: 120 per block of 32 and tile, LDS reads
+// included, and 250 for the tile's split).
+void choose_line(ffs_plan* pl) {
+  const ffs_problem& p = pl->prob;
+  const int64_t r = p.radius;
+  const bool fp64 = p.precision == FFS_PREC_FP64;
+  if (p.dims != 1 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
+  const int64_t block = fp64 ? 16 : 32, nbmax = fp64 ? ffsk::kLineMaxNb64 : ffsk::kLineMaxNbBF;
+  const int64_t most = std::min<int64_t>(ffsk::kLineMaxTaps, block * nbmax - 15);
+  double best = 1e300;
+  for (int64_t t = 1; 2 * r * t + 1 <= most && t <= p.steps; t++) {
+    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
+    const int64_t nb = (2 * r * te + 16 + block - 1) / block;
+    const double n = (double)p.sizes[0];
+    const double work = std::ceil(n / 256.0 / 1024.0) * (fp64 ? (double)nb * 256.0 : (double)nb * 120.0 + 250.0);
+    const double cost = (double)nl * (14000.0 + std::max(work, 16.0 * n / 5.3e12 * 2.4e9));
+    if (cost < best * (1 - 1e-9) && nl <= pl->nblocks) {
+      best = cost;
+      pl->line = true;
+      pl->line_t = te;
+      pl->line_nb = (int32_t)nb;
+    }
+  }
+  if (pl->line) pl->line_tail = p.steps % pl->line_t;
+}
+
+// Direct path, 2D and 3D: workgroups along axis 0.  Each streams a segment of rows (planes) and the 2rt + t - 1 that
+// fill its pipeline; the launch lasts as many rounds of resident workgroups (2 per CU in 2D, 1 in 3D: 512 threads of
+// up to 211 VGPRs) as the strips times the segments need.  Returns the segment with the shortest launch.  One workgroup
+// past a full round costs a whole one: 2999x4111 at t = 4 has 9 strips, and 57 segments of 53 rows made 513 workgroups
+// for 512 places (900 us for 37 steps; 56 segments 776).  In 2D a CU with one workgroup walks a row in about 0.68 of
+// the time it takes with two.  Segments are 16 rows or longer (shorter ones are mostly fill: Box2D25P 1024^2, 13 rows
+// 2.5% slower than 16) unless those leave half of the CUs without a workgroup (Heat-2D 128^2 x 64 211 -> 148 us).
+int64_t direct_segments(const ffs_problem& p, int num_cus, int64_t t, int64_t strips) {
+  const int64_t n0 = p.sizes[0], fill = 2 * (int64_t)p.radius * t + t - 1;
+  const int64_t resident = (int64_t)num_cus * (p.dims == 2 ? 2 : 1);
+  double best = 1e300;
+  int64_t best_seg = n0;
+  int64_t most = std::min<int64_t>(n0, std::max<int64_t>(1, 8 * resident / strips + 1));
+  const int64_t of16 = (n0 + 15) / 16;
+  if (strips * of16 >= num_cus / 2) most = std::min(most, of16);
+  for (int64_t nseg = 1; nseg <= most; nseg++) {
+    const int64_t seg = (n0 + nseg - 1) / nseg, units = strips * ((n0 + seg - 1) / seg);
+    const double rounds = p.dims == 2 && units <= num_cus ? 0.68 : (double)((units + resident - 1) / resident);
+    const double cost = rounds * (double)(seg + fill);
+    if (cost < best * (1 - 1e-9)) {
+      best = cost;
+      best_seg = seg;
+    }
+  }
+  return best_seg;
+}
+
 // Direct path: fused depth per launch.  Per point-step cost max(compute, memory): FMAs x window/valid area
 // x pipeline fill along axis 0 at ~24e12 FP64 FMA/s, against 16 B x window/valid area / t at an effective
 // 2.5e12 B/s (fitted to MI355X timings of t = 1..6: the row stream is latency- rather than
@@ -251,6 +306,7 @@ ffs_status choose_config_direct(ffs_plan* pl) {
     }
   }
   set_blocks(pl, tbest, p.fuse > 0);
+  choose_line(pl);  // 1D: banded products, the direct sum of t steps at once
   return FFS_OK;
 }
 
@@ -305,34 +361,6 @@ void choose_stream(ffs_plan* pl) {
     }
   }
   if (pl->stream) pl->stream_tail = p.steps % pl->stream_t;
-}
-
-// 1D runs by banded products: depth per launch, from the modelled time of the run (SIMD cycles): per launch 8,000,
-// plus 6,000 for a wave's chain of load, product and store, plus the larger of the memory time (16 B per point at
-// 5.3 TB/s) and the products (FP64: 256 cycles per block of 16 and tile; BF16: 120 per block of 32 and tile, LDS reads
-// included, and 250 for the tile's split).
-void choose_line(ffs_plan* pl) {
-  const ffs_problem& p = pl->prob;
-  const int64_t r = p.radius;
-  const bool fp64 = p.precision == FFS_PREC_FP64;
-  if (p.dims != 1 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
-  const int64_t block = fp64 ? 16 : 32, nbmax = fp64 ? ffsk::kLineMaxNb64 : ffsk::kLineMaxNbBF;
-  const int64_t most = std::min<int64_t>(ffsk::kLineMaxTaps, block * nbmax - 15);
-  double best = 1e300;
-  for (int64_t t = 1; 2 * r * t + 1 <= most && t <= p.steps; t++) {
-    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
-    const int64_t nb = (2 * r * te + 16 + block - 1) / block;
-    const double n = (double)p.sizes[0];
-    const double work = std::ceil(n / 256.0 / 1024.0) * (fp64 ? (double)nb * 256.0 : (double)nb * 120.0 + 250.0);
-    const double cost = (double)nl * (14000.0 + std::max(work, 16.0 * n / 5.3e12 * 2.4e9));
-    if (cost < best * (1 - 1e-9) && nl <= pl->nblocks) {
-      best = cost;
-      pl->line = true;
-      pl->line_t = te;
-      pl->line_nb = (int32_t)nb;
-    }
-  }
-  if (pl->line) pl->line_tail = p.steps % pl->line_t;
 }
 
 // Launches of one run.
@@ -626,7 +654,7 @@ ffsk::Stream3Args make_stream_args(const ffs_plan* pl, const double* src, double
 }
 
 // Direct path: launch geometry of one block of depth t (the window is fixed, the valid part shrinks
-// with t).  About two workgroups per CU along axis 0, each streaming a segment of rows (planes).
+// with t).
 ffsk::DirectArgs make_direct_args(const ffs_plan* pl, const double* src, double* dst, int64_t t) {
   const ffs_problem& p = pl->prob;
   const int r = p.radius, K = 2 * r + 1;
@@ -671,9 +699,7 @@ ffsk::DirectArgs make_direct_args(const ffs_plan* pl, const double* src, double*
     a.strips2 = (int32_t)cdiv(a.n2, a.valid2);
     strips = (int64_t)a.strips1 * a.strips2;
   }
-  int64_t nseg = std::max<int64_t>(1, (2 * (int64_t)pl->num_cus + strips / 2) / strips);
-  nseg = std::min<int64_t>(nseg, cdiv(a.n0, 16));
-  a.seg = cdiv(a.n0, nseg);
+  a.seg = direct_segments(p, pl->num_cus, t, strips);
   a.nseg = (int32_t)cdiv(a.n0, a.seg);
   return a;
 }
@@ -873,6 +899,7 @@ TableSizes dft_table_sizes(const ffs_plan* pl) {
 // The tables the plan's kernels read.
 TableSizes table_sizes(const ffs_plan* pl) {
   TableSizes t = dft_table_sizes(pl);
+  if (pl->line) t.taps = sizeof(double) * pl->weights.size();
   if (!pl->direct && real_tiles(pl)) {
     t.ops = sizeof(double) * ffsk::kOpsReal;
     t.H = sizeof(double) * 2 * ffsk::kSpecReal;
@@ -940,7 +967,7 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
                          p.convention, (int32_t)pl->line_tail, pl->line_nb, s);
     if (e != hipSuccess) return e;
   }
-  if (run_only && (pl->wide || pl->stream || pl->line)) return hipSuccess;
+  if (pl->direct || (run_only && (pl->wide || pl->stream || pl->line))) return hipSuccess;
   if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
   if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);
@@ -1125,7 +1152,8 @@ ffs_status ffs_plan_create(const ffs_problem* p, ffs_plan** out) {
     if (x != hipSuccess && e == hipSuccess) e = x;
   };
   const TableSizes ts = table_sizes(pl);
-  if (!pl->direct) {
+  const bool tables = !pl->direct || pl->line;
+  if (tables) {
     chk(hipMalloc(&pl->d_tables, place_tables(pl, ts, nullptr)));
     if (e == hipSuccess) place_tables(pl, ts, pl->d_tables);
   }
@@ -1135,7 +1163,7 @@ ffs_status ffs_plan_create(const ffs_problem* p, ffs_plan** out) {
     return fail(e == hipErrorOutOfMemory ? FFS_ERR_OUT_OF_MEMORY : FFS_ERR_HIP, "device allocation failed: %s",
                 hipGetErrorString(e));
   }
-  if (!pl->direct) {
+  if (tables) {
     chk(hipMemcpy(pl->d_taps, pl->weights.data(), ts.taps, hipMemcpyHostToDevice));
     chk(plan_tables(pl, nullptr, false));
     chk(hipDeviceSynchronize());
@@ -1194,7 +1222,8 @@ ffs_status ffs_plan_get_info(const ffs_plan* pl, ffs_plan_info* info) {
     }
     info->fuse = (int32_t)pl->t;
     info->fuse_tail = (int32_t)pl->t_tail;
-    info->blocks = info->launches = pl->nblocks;
+    info->blocks = pl->nblocks;
+    info->launches = run_launches(pl);
     info->flops_per_block = 2.0 * taps * computed;
     info->bytes_per_block = 16.0 * (double)pl->npoints;
     return FFS_OK;
@@ -1368,7 +1397,8 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
   if (st == FFS_OK) st = plan_constants(&pl);
   if (st != FFS_OK) return st;
   const TableSizes ts = table_sizes(&pl);
-  const size_t off = pl.direct ? 0 : place_tables(&pl, ts, nullptr);
+  const bool tables = !pl.direct || pl.line;
+  const size_t off = tables ? place_tables(&pl, ts, nullptr) : 0;
   if (off > FFS_STATIC_TABLE_BYTES)
     return fail(FFS_ERR_INTERNAL, "plan tables need %zu bytes of the %llu reserved", off, FFS_STATIC_TABLE_BYTES);
   const size_t grid_bytes = pl.nblocks >= 2 ? sizeof(double) * (size_t)pl.npoints : 0;
@@ -1382,10 +1412,10 @@ ffs_status ffs_run_static(const ffs_problem* p, const double* d_in, double* d_ou
   st = static_scratch(pl.dev, &base);
   if (st != FFS_OK) return st;
   char* b = static_cast<char*>(base);
-  if (!pl.direct) place_tables(&pl, ts, b);
+  if (tables) place_tables(&pl, ts, b);
   pl.d_scratch = grid_bytes ? reinterpret_cast<double*>(b + FFS_STATIC_TABLE_BYTES) : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  if (!pl.direct) {
+  if (tables) {
     hipError_t e = ffsk::put_taps(pl.d_taps, pl.weights.data(), (int64_t)pl.weights.size(), s);
     if (e == hipSuccess) e = plan_tables(&pl, s, true);
     if (e != hipSuccess) return fail(FFS_ERR_HIP, "table generation failed: %s", hipGetErrorString(e));
