@@ -3097,24 +3097,29 @@ __global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
   }
 }
 
-// Taps of the t-fold 1D stencil in correlation order (ref: e = 2r - a; centred: e = a), by t - 1 convolutions in
-// FP64; one workgroup.
-__global__ void k_gen_line_taps(double* out, const double* taps, int32_t K, int32_t convention, int32_t t) {
-  __shared__ double buf[2][kLineMaxTaps];
-  const int n = (K - 1) * t + 1;
-  for (int i = threadIdx.x; i < kLineMaxTaps; i += blockDim.x) buf[0][i] = i < K ? taps[convention == 0 ? K - 1 - i : i] : 0.0;
+// Taps of the t-fold 1D stencil in correlation order (ref: e = 2r - a; centred: e = a), by repeated squaring of the
+// tap polynomial in FP64; one workgroup of kLineMaxTaps threads, thread i forms coefficient i.
+__global__ __launch_bounds__(kLineMaxTaps) void k_gen_line_taps(double* out, const double* taps, int32_t K,
+                                                                int32_t convention, int32_t t) {
+  __shared__ double one[kLineMaxTaps], cur[kLineMaxTaps];
+  const int i = threadIdx.x;
+  one[i] = i < K ? taps[convention == 0 ? K - 1 - i : i] : 0.0;
+  cur[i] = one[i];
   __syncthreads();
-  int cur = 0;
-  for (int s = 1; s < t; s++) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      double sum = 0.0;
-      for (int e = 0; e < K && e <= i; e++) sum = __builtin_fma(taps[convention == 0 ? K - 1 - e : e], buf[cur][i - e], sum);
-      buf[cur ^ 1][i] = sum;
-    }
+  int n = K;  // coefficients of cur
+  auto times = [&](const double* f, int m) {  // cur *= f (m coefficients)
+    double sum = 0.0;
+    for (int e = max(0, i - n + 1); e < m && e <= i; e++) sum = __builtin_fma(f[e], cur[i - e], sum);
     __syncthreads();
-    cur ^= 1;
+    cur[i] = sum;
+    n += m - 1;
+    __syncthreads();
+  };
+  for (int bit = 30 - __builtin_clz(t); bit >= 0; bit--) {
+    times(cur, n);
+    if ((t >> bit) & 1) times(one, K);
   }
-  for (int i = threadIdx.x; i < kLineMaxTaps; i += blockDim.x) out[i] = i < n ? buf[cur][i] : 0.0;
+  out[i] = i < n ? cur[i] : 0.0;
 }
 
 // Operands of k_line_bf16: [block b][term][lane] of 4 words; element e of lane (i + 16q) is T[i][32 b + 8q + e] =
@@ -3137,7 +3142,7 @@ __global__ void k_gen_line_ops(uint32_t* t, const double* g, int32_t n, int32_t 
 
 hipError_t gen_line(double* g, uint32_t* ops, const double* d_taps, int32_t K, int32_t convention, int32_t t, int32_t nb,
                     hipStream_t s) {
-  hipLaunchKernelGGL(k_gen_line_taps, dim3(1), dim3(512), 0, s, g, d_taps, K, convention, t);
+  hipLaunchKernelGGL(k_gen_line_taps, dim3(1), dim3(kLineMaxTaps), 0, s, g, d_taps, K, convention, t);
   if (ops)
     hipLaunchKernelGGL(k_gen_line_ops, dim3((unsigned)nb), dim3(3 * kLanes), 0, s, ops, g, (K - 1) * t + 1, nb);
   return hipGetLastError();
