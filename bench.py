@@ -18,16 +18,18 @@ Workloads (seed 0x5EED0000 + index, SplitMix64; weights uniform[0,1) normalised 
 form (full T) and against the FP64 direct sweep (the oracle, on a bounded sample), and the oracle's CPU
 time on the host's cores.
 
-Roofline of the dominant kernel (one fused block = one launch), algorithmic counts only:
-  flops  = the real GEMMs the kernel's formulation needs, each counted once (the Gauss 3-GEMM complex
-           product, the inverse stages cut to the kept output block, never the split products of the
-           mixed forms: executed MFMA flops / products per real GEMM, 1 FP64/FP32 (2 for the
-           compensated FP32 form in 3D), 3 FP16, 6 BF16),
+Roofline of one fused block (ffs_run_block: one launch of the plan's block kernel), algorithmic counts only:
+  flops  = the real GEMMs the kernel's formulation needs, each counted once (FP64 2D: the folded real
+           transforms; elsewhere the complex products, Gauss form in FP64; the inverse stages cut to the kept
+           output block; never the split products of the mixed forms: executed MFMA flops / products
+           per real GEMM, 1 FP64/FP32 (2 for the compensated FP32 form in 3D), 3 FP16, 6 BF16),
            against the matrix peak of the form's arithmetic (FP64 78.6 TF, FP32 157.3 TF, FP16/BF16
            2.5 PF); direct kernel: 2 |S| t per point against the FP64 vector peak;
   bytes  = 16 x points (FP64 state read once and written once per block) against 8 TB/s;
   frac   = the larger of the two fractions, `bound` names which.
-Beside it: `matrix_frac_dense`, the dense count tiles x 8 d P^(d+1) per real tile (per-axis complex DFT
+`run` beside it: what a whole run launches (the mixed 2D forms two blocks at once, 3D and 1D kernels of
+their own): launches, ms per launch, and the same 16 x points per launch against 8 TB/s.
+Also: `matrix_frac_dense`, the dense count tiles x 8 d P^(d+1) per real tile (per-axis complex DFT
 GEMMs with real-pair packing; 1D prime-factor window 240 = 15 x 16: 8 x 240 x (15 + 16)), and
 `executed_mfma_tflops` (split products included).
 
@@ -290,8 +292,8 @@ def bench_grid(name, args, torch, ffs, forms=None):
         t0 = time.perf_counter()
         ms, reps = timed(torch, lambda: plan.run(d_in, d_out), args.warmup, args.steps, stream)
         wall = time.perf_counter() - t0
-        # dominant kernel alone: one fused block per launch on the launch stream, ping-ponging between two
-        # grids as inside a run (each launch reads the previous block's output)
+        # the block kernel alone: one fused block per launch on the launch stream, ping-ponging between two
+        # grids (each launch reads the previous block's output)
         d_a, d_b = d_in.clone(), torch.empty_like(d_in)
         flip = [0]
 
@@ -306,6 +308,9 @@ def bench_grid(name, args, torch, ffs, forms=None):
         rl["traffic"] = traffic(name, form)
         if rl["traffic"] is not None:
             rl["traffic_from"] = "profiles/traffic.json (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, copy-calibrated)"
+        launch_ms = ms / max(info["launches"], 1)
+        rl["run"] = {"launches": info["launches"], "launch_ms": launch_ms,
+                     "hbm_frac": 16.0 * npts / (launch_ms * 1e-3) / HBM_PEAK}
         gst = npts * T / (ms * 1e-3) / 1e9
         res[form] = dict(value=gst, ms_per_step=ms, timed_runs=reps, wall_s=wall, roofline=rl,
                          plan={k: info[k] for k in ("tile", "valid", "fuse", "fuse_tail", "blocks", "algorithm",
@@ -313,7 +318,8 @@ def bench_grid(name, args, torch, ffs, forms=None):
         outputs[form] = d_out
         log(f"{name} {form}: {gst:.1f} GStencil/s, {ms:.3f} ms/run, block {kms:.3f} ms, roofline {rl['bound']} "
             f"{rl['frac']:.1%} (matrix {rl['matrix_frac']:.1%}, hbm {rl['hbm_frac']:.1%}), P={info['tile']} "
-            f"t={info['fuse']} V={info['valid']} blocks={info['blocks']}")
+            f"t={info['fuse']} V={info['valid']} blocks={info['blocks']}; run: {info['launches']} launches of "
+            f"{launch_ms:.3f} ms, hbm {rl['run']['hbm_frac']:.1%}")
         plan.close()
     if "fp64" in outputs:
         ref64 = outputs["fp64"]
@@ -419,12 +425,12 @@ def bench_batch(args, torch, ffs, forms=None):
         rounds = 0
         for i in range(len(specs)):
             inf = batch.info(i)
-            rounds = max(rounds, inf["blocks"])
+            rounds = max(rounds, inf["launches"])
             flops += inf["flops_per_block"] / products(form, inf) * inf["blocks"]
-            bytes_alg += 16.0 * inf["sizes"][0] * inf["sizes"][1] * inf["blocks"]
+            bytes_alg += 16.0 * inf["sizes"][0] * inf["sizes"][1] * inf["launches"]
         s = ms * 1e-3
         f_frac, b_frac = flops / s / MATRIX_PEAK[form], bytes_alg / s / HBM_PEAK
-        rl = {"scope": f"whole run ({rounds} launches, one per round)", "flops_per_run": flops,
+        rl = {"scope": f"whole run ({rounds} rounds); flops as of the blocks it stands for", "flops_per_run": flops,
               "bytes_per_run": bytes_alg, "matrix_frac": f_frac, "hbm_frac": b_frac, "traffic": None}
         if b_frac >= f_frac:
             rl.update(bound="hbm", achieved=bytes_alg / s / 1e9, peak=HBM_PEAK / 1e9, unit="GB/s", frac=b_frac)

@@ -10,7 +10,7 @@ enum TileKind : int32_t {
   KIND_2D16 = 0,   // 2D, 16x16 window
   KIND_1DPFA = 1,  // 1D, 240-sample window as a 15x16 prime-factor (Good-Thomas) matrix
   KIND_3D16 = 2,   // 3D, 16x16x16 window (one workgroup of 4 waves per tile pair)
-  KIND_2D32 = 3,   // 2D, 32x32 window (mixed forms: the contraction fills K = 32 of the MFMA; FP64: 8 chunks)
+  KIND_2D32 = 3,   // 2D, 32x32 window (mixed forms: the contraction fills K = 32 of the MFMA; FP64: real transforms)
 };
 
 // Operand-table layout in doubles (one table per plan, generated on the GPU in FP64):
@@ -44,7 +44,7 @@ inline int64_t spectrum_len(int kind) {  // complex values per spectrum (one dep
 // element e of lane (j + 16q) is row 16 (e >> 2) + 4q + (e & 3), column 16 Kb + j of that term.
 constexpr int kOps32Words = 3 * 2 * 3 * 4 * kLanes;  // 4608
 
-// 32-point FP64 B operands (KIND_2D32, FP64 form): [R][chunk v][column block Kb][arr: R, S, D][lane], lane
+// 32-point FP64 DFT operands (read back by ffs_plan_read_table; the kernels run real transforms): [R][chunk v][column block Kb][arr: R, S, D][lane], lane
 // (n + 16k) holding entry (row 16 R + 4 v + k, column 16 Kb + n) of Fr, -(Fr + Fi) or Fi - Fr (the sum is
 // stored negated so that both output accumulators chain from the shared Gauss product).
 constexpr int kOps32F64 = 2 * 4 * 2 * 3 * kLanes;  // 3072 doubles
@@ -53,8 +53,10 @@ struct TileArgs {
   const double* src;
   double* dst;
   const double* ops;  // DFT operands (doubles)
-  const double* H;    // spectrum^t / (P0 P1 [P2]) for this block, family layout, [re plane | im plane]
-  const float* Hf;    // mixed forms: the same spectrum rounded to FP32, (re, im) pairs (one 8-byte load each)
+  const double* H;    // spectrum^t / (P0 P1 [P2]) for this block, family layout, [re plane | im plane]; 32-point
+                      // FP64: 4 filter values per (k0, k1) (gen_spectrum_real)
+  const float* Hf;    // mixed forms: the same spectrum rounded to FP32, (re, im) pairs (one 8-byte load each);
+                      // 64-point launches: 4 FP32 filter values per (k0, k1)
   const uint32_t* opsm;  // mixed-form operand table (kOpsMixedLen words)
   int64_t n0, n1, n2;       // grid sides (unused axes = 1); 1D uses n1
   int64_t tiles0, tiles1, tiles2;
@@ -66,12 +68,13 @@ struct TileArgs {
   double dc_gain;  // K(0)^t: gain of the constant mode (mixed forms add mean * gain back in FP64)
   int32_t linear_map;  // 1: workgroups take tiles in hardware order; 0: XCD-contiguous bands
   // 32-point family: 1 when the valid region fits one 16 x 16 block (V0, V1 <= 16).  The two inverse
-  // stages then compute only output block 0 (2 and 1 of 4 output blocks) with the inverse operands of
-  // window columns h .. h + 15 (`opsi`), so output index m is window position h + m: every value kept is
-  // the one the full stages would produce at that position, from the same operands (the batch kernels
-  // read those columns from the forward operands they hold in LDS instead of `opsi`).
+  // stages then compute only output block 0.  Mixed forms (2 and 1 of 4 output blocks): with the inverse
+  // operands of window columns h .. h + 15 (`opsi`), so output index m is window position h + m: every value
+  // kept is the one the full stages would produce at that position, from the same operands (the batch
+  // kernels read those columns from the forward operands they hold in LDS instead of `opsi`).  FP64: the
+  // valid region starts at window position 0, in the near half that the real inverse computes anyway.
   int32_t out16;
-  const void* opsi;  // out16: inverse operands (kInv32Words words or kInv32F64 doubles, see below)
+  const void* opsi;  // out16, mixed forms: inverse operands (kInv32Words words, see below)
   float unit;  // 1.0f: a multiplier the kernels must not see as a constant (the FP16 split's residual FMA)
 };
 

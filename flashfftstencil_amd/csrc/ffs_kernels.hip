@@ -16,6 +16,9 @@
 // (fwd axis0, fwd axis1, inv axis0, inv axis1) chain in registers with no data exchange.  This
 // replaces the reference's permuted-row DFT copy for accumulator reuse (src/2D/create_fft_pfa_plan.cu:27-37).
 //
+// The 32-point FP64 tiles, the 64-point mixed windows and the streamed 3D planes run real half-sample transforms
+// with the same chaining and no pairing of tiles; whole 1D runs are banded products (see those sections).
+//
 // Complex GEMMs use the 3-multiplication (Gauss/Karatsuba) form, as the reference's 1D kernel does
 // (src/1D/rfftstencil_pfa/rfft_8_pfa_fastcomplex.cu:84-101):
 //   k1 = (Ar+Ai)Br, k2 = Ar(Bi-Br), k3 = Ai(Br+Bi);  Re = k1-k3, Im = k1+k2.
