@@ -211,6 +211,15 @@ bool star_support(const ffs_plan* pl) {
   return true;
 }
 
+// The run kernels go deeper per launch than the blocks, so a strongly growing or damping stencil leaves the range of
+// their tables earlier: FP32 (mixed forms) must hold |K|^t within 2^+-40 or so beside the field's own range, FP64 has
+// 2^+-1022.  sum |w| bounds |K| (and is within sqrt(taps) of its maximum).  Out of range: the plan's own blocks.
+bool depth_in_range(const ffs_plan* pl, int64_t depth) {
+  double s1 = 0.0;
+  for (double w : pl->weights) s1 += std::fabs(w);
+  return (double)depth * std::fabs(std::log2(s1)) <= (pl->prob.precision == FFS_PREC_FP64 ? 800.0 : 40.0);
+}
+
 // 1D runs by banded products: depth per launch, from the modelled time of the run (SIMD cycles): per launch 8,000,
 // plus 6,000 for a wave's chain of load, product and store, plus the larger of the memory time (16 B per point at
 // 5.3 TB/s) and the products (FP64: 256 cycles per block of 16 and tile; BF16: 120 per block of 32 and tile, LDS reads
@@ -229,7 +238,7 @@ void choose_line(ffs_plan* pl) {
     const double n = (double)p.sizes[0];
     const double work = std::ceil(n / 256.0 / 1024.0) * (fp64 ? (double)nb * 256.0 : (double)nb * 120.0 + 250.0);
     const double cost = (double)nl * (14000.0 + std::max(work, 16.0 * n / 5.3e12 * 2.4e9));
-    if (cost < best * (1 - 1e-9) && nl <= pl->nblocks) {
+    if (cost < best * (1 - 1e-9) && nl <= pl->nblocks && depth_in_range(pl, te)) {
       best = cost;
       pl->line = true;
       pl->line_t = te;
@@ -338,7 +347,7 @@ void choose_stream(ffs_plan* pl) {
                 (8000.0 + std::ceil(pairs / (fp64 ? 512.0 : 768.0)) * (fp64 ? 45000.0 : 36000.0) - (pairs <= 256.0 ? 10000.0 : 0.0));
   for (int64_t t = 1; 2 * r * t + 1 <= emax; t++) {
     const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
-    if (nl > 1 && pl->nblocks == 1) continue;
+    if ((nl > 1 && pl->nblocks == 1) || !depth_in_range(pl, te)) continue;
     const int64_t V = 32 - 2 * r * te;
     const int64_t tiles = ((p.sizes[1] + V - 1) / V) * ((p.sizes[2] + V - 1) / V);
     const int E = (int)(2 * r * te + 1);
@@ -503,7 +512,8 @@ ffs_status choose_config(ffs_plan* pl) {
   // Two blocks per launch on 64-point windows wherever the valid region of the doubled tile still fits the
   // near half of the window (2V <= 32; beyond it the inverse stages would need both halves) and there are
   // two blocks to take: Box2D25P 8192^2, two t = 4 blocks 684 us, one 64-point launch 337 us (FP16; BF16 1000 and 445).
-  pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2;
+  pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2 &&
+             depth_in_range(pl, 2 * pl->t);
   if (pl->wide) pl->t_wide_tail = p.steps % (2 * pl->t);
   choose_stream(pl);
   choose_line(pl);

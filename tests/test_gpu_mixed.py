@@ -294,3 +294,18 @@ def test_2d_mixed_two_blocks_long_rows(ffs, torch_cuda, form, n1):
             assert plan.info["launches"] == (2 if precision == "fp64" else 1)
         outs.append(d)
     assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) <= TOL_MIXED
+
+
+@pytest.mark.parametrize("form,tol", [("bf16", TOL_MIXED), ("fp64", 1e-12)])
+@pytest.mark.parametrize("decades", [-40, 40])
+@pytest.mark.parametrize("size,radius,fuse,steps", [((200, 180), 2, 4, 8), ((130, 140, 131), 1, 2, 6), ((3000,), 1, 4, 16)])
+def test_strong_growth_and_damping(ffs, oracle, torch_cuda, form, tol, decades, size, radius, fuse, steps):
+    # The taps sum to 10^(decades / steps) and the field runs from 10^-(decades / 2) to 10^(decades / 2): every block of
+    # t steps fits FP32 (|K|^t <= 10^20), the whole run in one launch would not (10^+-40), so the plan goes less deep.
+    rng = np.random.default_rng(steps)
+    w = rng.random((2 * radius + 1) ** len(size))
+    w *= 10.0 ** (decades / steps) / w.sum()
+    x = oracle.uniform(5, size) * 10.0 ** (-decades / 2)
+    got, info = _run(ffs, torch_cuda, x, radius, w, steps, precision=form, fuse=fuse)
+    ref = oracle.sweep(x, radius, w, steps)
+    assert np.isfinite(got).all() and oracle.errors(got, ref)[1] <= tol, (form, decades, size, info)
