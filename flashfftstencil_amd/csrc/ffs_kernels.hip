@@ -3024,7 +3024,9 @@ __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
 }
 
 // BF16: three-term split of the window (once, into LDS) and of T (operand table, [K = 32 block][term][lane]); the six
-// products of order <= 2^-16, the five small ones summed apart from the dominant one.
+// products of order <= 2^-16, the five small ones summed apart from the dominant one.  c is the mean of the window.  Bound by
+// HBM; the next window is requested before the products of this one, 3 waves/SIMD alone did not cover the loads (1D7P
+// 2^24 x 100, two launches: 173 us without, 153 with, 3.5 TB/s; 33,000,001 points in one launch 134 and 119, 4.4 TB/s).
 template <int M>
 __global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
   extern __shared__ double lds[];
@@ -3037,31 +3039,46 @@ __global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
   const int q = lane >> 4, j = lane & 15;
   uint32_t* sX = reinterpret_cast<uint32_t*>(sT + a.nb * 3 * kLanes) + (int64_t)w * 3 * (win / 2);
   const int64_t units = (a.n + 256 * M - 1) / (256 * M);
-  for (int64_t u = (int64_t)blockIdx.x * 4 + w; u < units; u += (int64_t)gridDim.x * 4) {
-    const int64_t p0 = u * (256 * M), base = p0 - a.h;
-    const bool interior = base >= 0 && base + win <= a.n;
-    // c: mean of 128 values spread over the window
-    const int s0 = (int)((int64_t)lane * (win - 2) / 63);
-    const double c = wave_sum(a.src[interior ? base + s0 : wrap_near(base + s0, a.n)] +
-                              a.src[interior ? base + s0 + 1 : wrap_near(base + s0 + 1, a.n)]) * (1.0 / 128);
-    for (int i = 2 * lane; i < win; i += 128) {
-      double x0, x1;
-      if (interior) {
-        const d2u x = *reinterpret_cast<const d2u*>(a.src + base + i);
-        x0 = x[0];
-        x1 = x[1];
-      } else {
-        x0 = a.src[wrap_near(base + i, a.n)];
-        x1 = a.src[wrap_near(base + i + 1, a.n)];
+  constexpr int kLoads = (256 * M + 32 * kLineMaxNbBF - 16 + 127) / 128;  // pairs of window values per lane
+  d2u x[kLoads];
+  auto request = [&](int64_t u) {
+    const int64_t base = u * (256 * M) - a.h;
+    if (base >= 0 && base + win <= a.n) {
+#pragma unroll
+      for (int c = 0; c < kLoads; c++)
+        if (128 * c + 2 * lane < win) x[c] = *reinterpret_cast<const d2u*>(a.src + base + 128 * c + 2 * lane);
+    } else {
+#pragma unroll
+      for (int c = 0; c < kLoads; c++) {
+        const int64_t i = base + 128 * c + 2 * lane;
+        if (128 * c + 2 * lane < win) x[c] = d2u{a.src[wrap_near(i, a.n)], a.src[wrap_near(i + 1, a.n)]};
       }
-      const float y0 = (float)(x0 - c), y1 = (float)(x1 - c);
-      const uint32_t h = pk_bf16(y0, y1);
-      const float r0 = y0 - bf_lo(h), r1 = y1 - bf_hi(h);
-      const uint32_t m = pk_bf16(r0, r1);
-      sX[i / 2] = h;
-      sX[win / 2 + i / 2] = m;
-      sX[win + i / 2] = pk_bf16(r0 - bf_lo(m), r1 - bf_hi(m));
     }
+  };
+  const int64_t stride = (int64_t)gridDim.x * 4;
+  int64_t u = (int64_t)blockIdx.x * 4 + w;
+  if (u < units) request(u);
+  for (; u < units; u += stride) {
+    const int64_t p0 = u * (256 * M);
+    double c = 0.0;
+#pragma unroll
+    for (int k = 0; k < kLoads; k++)
+      if (128 * k + 2 * lane < win) c += x[k][0] + x[k][1];
+    c = wave_sum(c) / (double)win;
+#pragma unroll
+    for (int k = 0; k < kLoads; k++) {
+      const int i = 128 * k + 2 * lane;
+      if (i < win) {
+        const float y0 = (float)(x[k][0] - c), y1 = (float)(x[k][1] - c);
+        const uint32_t h = pk_bf16(y0, y1);
+        const float r0 = y0 - bf_lo(h), r1 = y1 - bf_hi(h);
+        const uint32_t m = pk_bf16(r0, r1);
+        sX[i / 2] = h;
+        sX[win / 2 + i / 2] = m;
+        sX[win + i / 2] = pk_bf16(r0 - bf_lo(m), r1 - bf_hi(m));
+      }
+    }
+    if (u + stride < units) request(u + stride);
     lds_fence();
     f4 big[M], small[M];
 #pragma unroll
@@ -3167,7 +3184,7 @@ hipError_t launch_line(const LineArgs& a, int32_t precision, hipStream_t s, int 
     const dim3 g((unsigned)std::min<int64_t>((a.n + 1023) / 1024, (int64_t)num_cus * resident)), b(256);
     hipLaunchKernelGGL(k_line_f64, g, b, lds, s, a);
   } else if (a.n > 4096 * (int64_t)num_cus * 4) {
-    // Two tiles per wave share the operand reads (1D7P 2^24 x 100: 184 us, one tile 207, four 209) once every SIMD
+    // Two tiles per wave share the operand reads (1D7P 2^24 x 100, before the requests ahead: 184 us, one tile 207, four 209) once every SIMD
     // has eight such waves; below that one tile per wave keeps its chain short (2,000,000 x 64: 39.8 against 40.6).
     launch_line_bf16<2>(a, s, num_cus);
   } else {

@@ -387,11 +387,13 @@ def test_1d_banded_product(ffs, oracle, torch_cuda, precision, tol, convention, 
     assert rel <= tol, (precision, convention, radius, n, steps, info, rel)
 
 
-def test_1d_banded_product_large(ffs, torch_cuda):
-    """The two-tile variant of the mixed kernel (above 4 Mi points) against the FP64 form, a ragged length."""
+@pytest.mark.parametrize("n", [(1 << 22) + 8191, (1 << 21) + 13])
+def test_1d_banded_product_large(ffs, torch_cuda, n):
+    """Several windows per wave, the next one requested ahead: the two-tile variant of the mixed kernel (above 4 Mi points)
+    and the one-tile variant, against the FP64 form, ragged lengths."""
     torch = torch_cuda
     _, r, w, _ = ffs.named_stencil("1D7P", seed=2)
-    d_in = torch.empty((1 << 22) + 8191, dtype=torch.float64, device="cuda")
+    d_in = torch.empty(n, dtype=torch.float64, device="cuda")
     ffs.fill_uniform_device(3, d_in)
     outs = []
     for precision in ("bf16", "fp64"):
