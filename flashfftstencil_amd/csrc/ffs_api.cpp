@@ -100,7 +100,7 @@ struct ffs_plan {
   bool line = false;
   int32_t line_nb = 0;
   int64_t line_t = 0, line_tail = 0;
-  int32_t scale_wide = 0, scale_wide_tail = 0;
+  int32_t norm_wide = 0, norm_wide_tail = 0;  // FP16 64-point launches: exponents the filters are normalised by
   double dc_main = 1.0, dc_tail = 1.0;  // K(0)^t and K(0)^t_tail
   int32_t scale_main = 0, scale_tail = 0;  // FP16 form: scale exponents of the main and tail depths
   double* d_taps = nullptr;
@@ -608,7 +608,8 @@ ffsk::TileArgs make_wide_args(const ffs_plan* pl, const double* src, double* dst
   a.units = a.tiles0 * a.tiles1;
   a.opsm = pl->d_wide;
   a.Hf = reinterpret_cast<const float*>(pl->d_wide + ffsk::kOpsWide) + (tail ? ffsk::kSpecWide : 0);
-  a.scale_exp = tail ? pl->scale_wide_tail : pl->scale_wide;
+  a.scale_exp = ffsk::kWideScaleExp;
+  a.filter_exp = tail ? pl->norm_wide_tail : pl->norm_wide;
   a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
   return a;
 }
@@ -795,6 +796,43 @@ ffs_status plan_device(ffs_plan* pl) {
   return FFS_OK;
 }
 
+// Largest |K| at the frequencies of a 64-point window, pi (2k + 1)/64 per axis.  Taps of one sign: the sum of |w|, which
+// bounds it and is within a few percent of it at the lowest frequency; else the maximum over the window's frequencies.
+double wide_gain(const std::vector<double>& w, int K) {
+  double sum = 0.0, abs = 0.0;
+  for (double x : w) {
+    sum += x;
+    abs += std::fabs(x);
+  }
+  if (std::fabs(sum) >= abs * (1 - 1e-12)) return abs;
+  static const std::vector<double> cosine = [] {  // cos(pi m / 64)
+    std::vector<double> c(128);
+    for (int m = 0; m < 128; m++) c[(size_t)m] = std::cos(M_PI * m / 64.0);
+    return c;
+  }();
+  auto co = [&](int m) { return cosine[(size_t)(m & 127)]; };
+  auto si = [&](int m) { return cosine[(size_t)((m - 32) & 127)]; };
+  double most = 0.0;
+  for (int k1 = -32; k1 < 32; k1++) {  // axis 0 from 0: K(-w) is the conjugate of K(w)
+    double re[32] = {}, im[32] = {};
+    for (int a0 = 0; a0 < K; a0++) {
+      double gr = 0.0, gi = 0.0;
+      for (int a1 = 0; a1 < K; a1++) {
+        const double x = w[(size_t)(a0 * K + a1)];
+        gr += x * co(a1 * (2 * k1 + 1));
+        gi += x * si(a1 * (2 * k1 + 1));
+      }
+      for (int k0 = 0; k0 < 32; k0++) {
+        const double c = co(a0 * (2 * k0 + 1)), s = si(a0 * (2 * k0 + 1));
+        re[k0] += gr * c - gi * s;
+        im[k0] += gr * s + gi * c;
+      }
+    }
+    for (int k0 = 0; k0 < 32; k0++) most = std::max(most, re[k0] * re[k0] + im[k0] * im[k0]);
+  }
+  return std::sqrt(most);
+}
+
 // Host constants: the constant-mode gains K(0)^t and, for the FP16 form, the tile scale exponents.
 ffs_status plan_constants(ffs_plan* pl) {
   if (pl->direct) return FFS_OK;
@@ -876,15 +914,11 @@ ffs_status plan_constants(ffs_plan* pl) {
     pl->scale_main = (int32_t)em;
     pl->scale_tail = (int32_t)et;
     if (pl->wide) {
-      // 64-point windows scale their folded inputs below 2^9 (one bit for the fold of stage 2).  A doubled
-      // depth beyond the FP16 range keeps the plan's single blocks.
-      const double ew = expo(2 * pl->t) - 1.0, ewt = expo(pl->t_wide_tail) - 1.0;
-      if (ew < -100.0 || ewt < -100.0) {
-        pl->wide = false;
-      } else {
-        pl->scale_wide = (int32_t)ew;
-        pl->scale_wide_tail = (int32_t)ewt;
-      }
+      const double lg = std::log2(wide_gain(pl->weights, K));
+      // 1e-9: taps that sum to 1 with a rounding error are not taken for growth
+      auto norm = [&](int64_t t) { return std::isfinite(lg) ? -(int32_t)std::ceil((double)t * lg - 1e-9) : 0; };
+      pl->norm_wide = norm(2 * pl->t);
+      pl->norm_wide_tail = norm(pl->t_wide_tail);
     }
   }
   return FFS_OK;
@@ -949,9 +983,10 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
   if (pl->wide) {
     float* H = reinterpret_cast<float*>(pl->d_wide + ffsk::kOpsWide);
     hipError_t e = ffsk::gen_operands_wide(pl->d_wide, p.precision == FFS_PREC_MIXED_F16, s);
-    if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, s);
+    if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, pl->norm_wide, s);
     if (e == hipSuccess && pl->t_wide_tail > 0)
-      e = ffsk::gen_spectrum_real(H + ffsk::kSpecWide, 64, pl->d_taps, K, p.convention, pl->t_wide_tail, s);
+      e = ffsk::gen_spectrum_real(H + ffsk::kSpecWide, 64, pl->d_taps, K, p.convention, pl->t_wide_tail,
+                                  pl->norm_wide_tail, s);
     if (e != hipSuccess) return e;
   }
   if (pl->stream) {
@@ -980,9 +1015,9 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
   if (pl->direct || (run_only && (pl->wide || pl->stream || pl->line))) return hipSuccess;
   if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
-  if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, s);
+  if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, 0, s);
   if (e == hipSuccess && pl->t_tail > 0)
-    e = ffsk::gen_spectrum_real(pl->d_H + ffsk::kSpecReal, 32, pl->d_taps, K, p.convention, pl->t_tail, s);
+    e = ffsk::gen_spectrum_real(pl->d_H + ffsk::kSpecReal, 32, pl->d_taps, K, p.convention, pl->t_tail, 0, s);
   return e;
 }
 // The DFT tables of the plan's family (complex operands, spectrum of the cyclic DFT, inverse operands).

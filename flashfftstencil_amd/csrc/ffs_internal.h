@@ -65,6 +65,7 @@ struct TileArgs {
   int32_t h0, h1, h2;       // window start offset (valid region starts at h in the window)
   int32_t precision;
   int32_t scale_exp;  // FP16 form: the tile pair is scaled so that its largest fluctuation is below 2^scale_exp
+  int32_t filter_exp;  // FP16 64-point launches: the filter table holds 2^filter_exp times the filter
   double dc_gain;  // K(0)^t: gain of the constant mode (mixed forms add mean * gain back in FP64)
   int32_t linear_map;  // 1: workgroups take tiles in hardware order; 0: XCD-contiguous bands
   // 32-point family: 1 when the valid region fits one 16 x 16 block (V0, V1 <= 16).  The two inverse
@@ -110,15 +111,16 @@ hipError_t gen_operands32(uint32_t* ops32, bool f16, hipStream_t s);
 hipError_t gen_operands32_f64(double* ops, hipStream_t s);
 // Tables of the real half-sample transforms.  32-point FP64 kernels: kOpsReal operand doubles, and the filter
 // of one depth, 4 doubles per (k0, k1) in kernel order.  64-point mixed kernels: kOpsWide operand words (the
-// BF16 form's size; FP16 uses two thirds), and kSpecWide floats per depth.
+// BF16 form's size; FP16 uses two thirds), and kSpecWide floats per depth, times 2^filter_exp.
 constexpr int kOpsReal = 2 * 4 * kLanes;
 constexpr int kSpecReal = 4 * 16 * 16;
 constexpr int kOpsWide = 4 * 3 * 4 * kLanes;
 constexpr int kSpecWide = 4 * 32 * 32;
+constexpr int kWideScaleExp = 9;  // FP16 64-point windows: folded fluctuations are scaled below 2^9
 hipError_t gen_operands_real(double* ops, hipStream_t s);
 hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s);
 hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
-                             hipStream_t s);
+                             int32_t filter_exp, hipStream_t s);
 // Inverse operands of an out16 block, output column j <- window column (j + shift) mod 32:
 //   mixed forms: u4 per lane, [arr: R, I, NI][term 0..2][lane] (the kOps32Words entries of block Kb = 0);
 //   FP64: [R][chunk v][arr: Fr, -(Fr + Fi), Fi - Fr][lane] doubles (the kOps32F64 entries of block Kb = 0).

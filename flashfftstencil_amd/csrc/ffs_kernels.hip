@@ -1514,10 +1514,15 @@ __global__ __launch_bounds__(256, 3) void k_batch32_f16(const TileArgs* __restri
 //   stage 3 u[type1 block][near row block]; stage 4 out[near row block][near col block]
 // The near halves alone hold the valid region (positions 0 .. 2V - 1 < 32).
 //
-// FP16 range: the folded inputs are scaled below 2^s, s <= 9.  The absolute row sums of both matrices are
-// 1/(2 sin(pi/128)) = 20.4, so stage 1 stays below 20.4 * 2^9, its folds below 41 * 2^9 = 20,900; stage 2 is not
-// split before the filter, which carries the transforms' 1/1024; the stage 3 outputs are 1/32 of the column
-// transforms of the filtered window, below 1.3 max |out|.
+// FP16 range: the folded inputs are scaled below 2^9, and the filter is normalised by a power of two so that |K|^depth
+// is at most 1 and above 1/2 at its largest over the window's frequencies (TileArgs::filter_exp; the store undoes
+// both).  The absolute row sums of both matrices are 1/(2 sin(pi/128)) = 20.4, so stage 1 stays below 20.4 * 2^9, its
+// folds below 41 * 2^9 = 20,900.  Stage 2 (below 20.4 * 20,900) is not split before the filter, which turns the four
+// coefficients of a frequency pair as a vector of at most the same length, twice the largest, times the transforms'
+// 1/1024: below 835 into stage 3, and stage 3's outputs, two such contractions, below 2 * 20.4 * 835 = 34,000 into
+// stage 4.  All under FP16's 65,504 for every radius and depth.  Downwards, the low terms reach 2^-25 absolute beside
+// a scaled window of 2^8 or more: without the normalisation a damping stencil's filtered coefficients went subnormal
+// (Heat-2D 200x180, depth 16, taps summing to 0.25: error 0.18 of max |out|, with it 4.9e-8; to 0.5: 1.3e-4 and 4.9e-8).
 // ---------------------------------------------------------------------------------------------
 typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
@@ -1819,7 +1824,7 @@ __device__ __forceinline__ void tile64(const TileArgs& a, const TilePos& p, cons
     B.make(y[2][D], y[3][D], a.unit);
     contract_sum<PREC>(A, B, sW, lane, out[D]);
   }
-  store64(a, p, q, j, out, ldexp(1.0, -e), c * a.dc_gain);
+  store64(a, p, q, j, out, ldexp(1.0, -e - a.filter_exp), c * a.dc_gain);
 }
 
 template <int PREC>
@@ -2504,7 +2509,8 @@ __global__ void k_gen_operands_real(double* t) {
 // delta = Im(L1 - L2)/2 give
 //   cc' =  alpha cc + beta ss + gamma sc + delta cs,   ss' =  alpha ss + beta cc - delta sc - gamma cs,
 //   sc' =  alpha sc - beta cs - gamma cc + delta ss,   cs' =  alpha cs - beta sc + gamma ss - delta cc
-// (c and s: cosine and sine along axis 0, then axis 1).  The transforms' 4/P^2 is folded in.
+// (c and s: cosine and sine along axis 0, then axis 1).  The transforms' 4/P^2 and the
+// factor 2^filter_exp are folded in.
 // Entry order: FP64 32-point (P = 32, doubles), entry v * 64 + lane <-> (q + 4v, j); 64-point (P = 64, floats),
 // entry ((2 b0 + b1) * 4 + v) * 64 + lane <-> (2 (4q + v) + b0, 2j + b1).
 __device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
@@ -2523,7 +2529,7 @@ __device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
   ki = pi;
 }
 __global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int32_t K, int32_t convention,
-                                    int64_t t) {
+                                    int64_t t, int32_t filter_exp) {
   __shared__ double2 root[128];  // exp(i pi m / P), m < 2P <= 128
   for (int m = threadIdx.x; m < 2 * P; m += blockDim.x) {
     double s, c;
@@ -2551,7 +2557,7 @@ __global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int3
     }
   cpow_t(L1r, L1i, t);
   cpow_t(L2r, L2i, t);
-  const double norm = 0.5 * 4.0 / ((double)P * (double)P);
+  const double norm = ldexp(0.5 * 4.0 / ((double)P * (double)P), filter_exp);
   const double h[4] = {(L1r + L2r) * norm, (L2r - L1r) * norm, (L1i + L2i) * norm, (L1i - L2i) * norm};
   for (int i = 0; i < 4; i++) {
     if (P == 32)
@@ -2605,8 +2611,9 @@ hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s) {
 }
 
 hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
-                             hipStream_t s) {
-  hipLaunchKernelGGL(k_gen_spectrum_real, dim3((unsigned)(P * P / 4 / 64)), dim3(64), 0, s, H, P, d_taps, K, convention, t);
+                             int32_t filter_exp, hipStream_t s) {
+  hipLaunchKernelGGL(k_gen_spectrum_real, dim3((unsigned)(P * P / 4 / 64)), dim3(64), 0, s, H, P, d_taps, K, convention, t,
+                     filter_exp);
   return hipGetLastError();
 }
 

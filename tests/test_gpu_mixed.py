@@ -309,3 +309,34 @@ def test_strong_growth_and_damping(ffs, oracle, torch_cuda, form, tol, decades, 
     got, info = _run(ffs, torch_cuda, x, radius, w, steps, precision=form, fuse=fuse)
     ref = oracle.sweep(x, radius, w, steps)
     assert np.isfinite(got).all() and oracle.errors(got, ref)[1] <= tol, (form, decades, size, info)
+
+
+@pytest.mark.parametrize("radius,fuse", [(1, 8), (2, 4), (8, 1), (15, 1)])
+@pytest.mark.parametrize("gain", [0.25, 0.5, 0.75, 1.5, 2.0])
+@pytest.mark.parametrize("signed", [False, True])
+def test_2d_f16_gain_per_step(ffs, oracle, torch_cuda, radius, fuse, gain, signed):
+    # Two FP16 blocks per launch under damping and growth: the filter of one launch is |K|^(2t) (down to 2^-32 here), and
+    # its products are split into FP16 terms again, so it has to be normalised.  Single plans and a batch (the
+    # filters and exponents of its items differ); signed taps, whose |K| is largest away from the lowest frequency.
+    torch = torch_cuda
+    rng = np.random.default_rng(3 * radius + fuse)
+    K = 2 * radius + 1
+    w = rng.standard_normal((K, K)) if signed else rng.random((K, K))
+    w *= gain / (np.abs(np.fft.fft2(w, (64, 64))).max())
+    w = w.ravel()
+    x = oracle.uniform(17 + radius, (75, 90))
+    steps = 4 * fuse + (3 if fuse > 1 else 1)
+    got, info = _run(ffs, torch_cuda, x, radius, w, steps, precision="f16", fuse=fuse)
+    assert info["launches"] == 3, info
+    ref = oracle.sweep(x, radius, w, steps)
+    assert oracle.errors(got, ref)[1] <= TOL_MIXED, (radius, fuse, gain, signed, oracle.errors(got, ref))
+    specs = [dict(sizes=(75, 90), weights=w * s, radius=radius, steps=steps, fuse=fuse) for s in (1.0, 1.0 / gain)]
+    d_in = [torch.from_numpy(x).cuda() for _ in specs]
+    d_out = [torch.empty_like(d) for d in d_in]
+    batch = ffs.Batch(specs, precision="f16")
+    batch.run(d_in, d_out)
+    torch.cuda.synchronize()
+    batch.close()
+    assert np.array_equal(d_out[0].cpu().numpy(), got)
+    ref = oracle.sweep(x, radius, w / gain, steps)
+    assert oracle.errors(d_out[1].cpu().numpy(), ref)[1] <= TOL_MIXED, (radius, fuse, gain, signed)
