@@ -631,6 +631,12 @@ ffsk::LineArgs make_line_args(const ffs_plan* pl, const double* src, double* dst
   a.taps_n = (int32_t)(2 * p.radius * t + 1);
   a.nb = pl->line_nb;
   a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
+  if (pl->direct) {
+    a.steps = (int32_t)t;
+    a.step_taps = 2 * p.radius + 1;
+    for (int e = 0; e < a.step_taps; e++)
+      a.step[e] = pl->weights[(size_t)(p.convention == FFS_CONV_REF ? a.step_taps - 1 - e : e)];
+  }
   return a;
 }
 

@@ -153,6 +153,9 @@ struct LineArgs {
   int64_t n, h;        // grid length, window offset
   int32_t taps_n, nb;
   double dc_gain;      // BF16: sum of the taps
+  int32_t steps;       // direct algorithm: depth of the launch (0 otherwise), and the stencil's own taps in correlation
+  int32_t step_taps;   // order, for windows that hold an infinity or NaN
+  double step[7];
 };
 hipError_t gen_line(double* g, uint32_t* ops, const double* d_taps, int32_t K, int32_t convention, int32_t t, int32_t nb,
                     hipStream_t s);

@@ -2989,6 +2989,11 @@ hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, h
 // ---------------------------------------------------------------------------------------------
 // FP64: taps in LDS (zero-padded on both sides), operands of both sides read per K = 4 chunk; the window with one
 // pad per 16 values (the column stride).
+// STEPS, the direct algorithm: its sums hold no values from beyond the stencil's reach, but the zeros around the band
+// turn an infinity or NaN anywhere in a group's window into NaN for the whole group.  A wave that has such a result takes
+// the launch's steps one by one in its LDS window, as k_direct1d does.  The test and the
+// path cost 1-4% of a launch (1D7P 2^24 x 100 351 -> 355 us, 5000 x 200 23.4 -> 24.5).
+template <bool STEPS>
 __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
   extern __shared__ double lds[];
   const int kk = 16 * a.nb;                    // contraction length
@@ -3017,8 +3022,26 @@ __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
         acc[c & 1] = FFS_MFMA64(sT[k - row + 15], sX[17 * (j + b) + 4 * c + q], acc[c & 1]);
       }
     }
+    d4 y = acc[0] + acc[1];
+    if (STEPS) {
+      const bool finite = __builtin_isfinite(y[0]) & __builtin_isfinite(y[1]) & __builtin_isfinite(y[2]) & __builtin_isfinite(y[3]);
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0)) {
+        int len = 255 + a.taps_n;              // window values that the outputs depend on
+        for (int s = 0; s < a.steps; s++) {
+          len -= a.step_taps - 1;
+          for (int i = lane; i < len; i += 64) {  // ascending, in place: a group of 64 reads ahead of what it writes
+            double sum = 0.0;
+            for (int e = 0; e < a.step_taps; e++) sum = __builtin_fma(a.step[e], sX[i + e + ((i + e) >> 4)], sum);
+            lds_fence();
+            sX[i + (i >> 4)] = sum;
+            lds_fence();
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) y[v] = sX[17 * j + 4 * q + v];
+      }
+    }
     const int64_t p = p0 + 16 * j + 4 * q;
-    const d4 y = acc[0] + acc[1];
     if (p + 3 < a.n) {
       *reinterpret_cast<d2u*>(a.dst + p) = d2u{y[0], y[1]};
       *reinterpret_cast<d2u*>(a.dst + p + 2) = d2u{y[2], y[3]};
@@ -3189,7 +3212,10 @@ hipError_t launch_line(const LineArgs& a, int32_t precision, hipStream_t s, int 
     const size_t kk = 16 * (size_t)a.nb, win = 240 + kk, lds = 8 * (kk + 16 + 4 * (win + (win >> 4) + 1));
     const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)(160 * 1024 / lds)));
     const dim3 g((unsigned)std::min<int64_t>((a.n + 1023) / 1024, (int64_t)num_cus * resident)), b(256);
-    hipLaunchKernelGGL(k_line_f64, g, b, lds, s, a);
+    if (a.steps > 0)
+      hipLaunchKernelGGL(k_line_f64<true>, g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL(k_line_f64<false>, g, b, lds, s, a);
   } else if (a.n > 4096 * (int64_t)num_cus * 4) {
     // Two tiles per wave share the operand reads (1D7P 2^24 x 100, before the requests ahead: 184 us, one tile 207, four 209) once every SIMD
     // has eight such waves; below that one tile per wave keeps its chain short (2,000,000 x 64: 39.8 against 40.6).

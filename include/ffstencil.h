@@ -77,7 +77,8 @@ typedef enum ffs_convention { FFS_CONV_REF = 0, FFS_CONV_CENTRED = 1 } ffs_conve
  *           blocking); precision must be FFS_PREC_FP64.  No kernel counterpart in the reference (its
  *           CPU check, src/2D/check_correct.hpp:64-100, is the semantics): a fallback and a baseline.
  *           Radius <= 3 in 1D and 2D, <= 1 in 3D.  1D runs take the t steps of a launch as one banded FP64
- *           matrix product with the taps of the t-fold stencil (ffs_run_block steps one by one).
+ *           matrix product with the taps of the t-fold stencil (ffs_run_block steps one by one).  Infinities and NaN
+ *           reach exactly the outputs whose sums, taken step by step, hold them.
  *   AUTO:   DIRECT where it is offered, else FFT.  On MI355X the FP64 vector and FP64 matrix peaks are
  *           equal, so the direct sum, with several times fewer FP64 operations per point-step than the
  *           transform path at these radii, is the faster one (ffs_autotune with AUTO measures both).

@@ -166,3 +166,43 @@ def test_direct_run_block_is_one_depth(ffs, oracle, torch_cuda):
     torch.cuda.synchronize()
     assert oracle.errors(d_out.cpu().numpy(), oracle.sweep(x, r, w, 2))[1] <= TOL
     plan.close()
+
+
+@pytest.mark.parametrize("algorithm", ["direct", "auto"])
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,n,steps", [(1, 256, 1), (1, 255, 7), (2, 1000, 31), (3, 700, 82), (3, 3, 4), (1, 5000, 300),
+                                            (2, 300000, 40)])
+def test_direct_1d_infinities_and_nan(ffs, torch_cuda, algorithm, convention, radius, n, steps):
+    # An infinity or NaN reaches exactly the outputs whose stencil sums hold it, in the direct sum of every step (a zero
+    # tap times an infinity included, opposite infinities meeting); every other output is finite and as exact as without
+    # it.  Windows that wrap, a grid smaller than the reach, one and several launches.
+    torch = torch_cuda
+    rng = np.random.default_rng(radius + steps)
+    K = 2 * radius + 1
+    for taps in ("positive", "signed", "gap"):
+        w = rng.random(K) + 0.1
+        if taps == "signed":
+            w[0] = -w[0]
+        if taps == "gap" and radius > 1:
+            w[1] = 0.0
+        w /= np.abs(w).sum()
+        x = rng.random(n)
+        where = [n // 3] + ([n - 1] if n > 1000 else []) + ([n // 2, n // 2 + 1] if n > 4 * radius * steps else [])
+        for k, i in enumerate(where):
+            x[i] = (np.inf, np.nan, -np.inf, np.inf)[k]
+        ref = x
+        with np.errstate(invalid="ignore"):
+            for _ in range(steps):
+                shift = range(K) if convention == "ref" else range(radius, radius - K, -1)
+                ref = sum(w[e] * np.roll(ref, s) for e, s in enumerate(shift))
+        d_in = torch.from_numpy(x).cuda()
+        d_out = torch.empty_like(d_in)
+        with ffs.Plan(1, (n,), w, radius, steps, algorithm=algorithm, convention=convention) as plan:
+            plan.run(d_in, d_out)
+            torch.cuda.synchronize()
+        got = d_out.cpu().numpy()
+        ok = np.isfinite(ref)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), (taps, np.flatnonzero(np.isnan(got) != np.isnan(ref))[:8])
+        assert np.array_equal(got[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)]), taps
+        # |out| <= max |in| < 1 in every step, each rounding K + 1 times
+        assert np.abs(got[ok] - ref[ok]).max(initial=0.0) <= 2 ** -53 * (K + 1) * steps, taps
