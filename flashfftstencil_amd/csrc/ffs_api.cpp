@@ -89,6 +89,7 @@ struct ffs_plan {
   int64_t t_wide_tail = 0;             // depth of the last launch when it is below 2t, else 0
   uint32_t* d_wide = nullptr;          // kOpsWide operand words, then kSpecWide floats for depth 2t and the tail
   double dc_wide = 1.0, dc_wide_tail = 1.0;
+  double lin_wide[2][2] = {};          // [main, tail][axis]: first moments of the t-fold taps
   // 3D FP64 and BF16 plans: a run streams planes (ffsk::launch_stream3d), launches of depth stream_t, the last one
   // of depth stream_tail; E taps along axis 0.  d_wide holds the operands, then the filters of both depths.
   bool stream = false;
@@ -611,6 +612,8 @@ ffsk::TileArgs make_wide_args(const ffs_plan* pl, const double* src, double* dst
   a.scale_exp = ffsk::kWideScaleExp;
   a.filter_exp = tail ? pl->norm_wide_tail : pl->norm_wide;
   a.dc_gain = tail ? pl->dc_wide_tail : pl->dc_wide;
+  a.lin0 = pl->lin_wide[tail][0];
+  a.lin1 = pl->lin_wide[tail][1];
   return a;
 }
 
@@ -876,6 +879,18 @@ ffs_status plan_constants(ffs_plan* pl) {
     }
     pl->dc_wide = ipow(sw, pl->line ? pl->line_t : 2 * pl->t);
     pl->dc_wide_tail = ipow(sw, pl->line ? pl->line_tail : pl->t_wide_tail);
+    if (pl->wide) {  // correlation taps at offsets 0 .. 2r per step: moments of the t-fold taps, t (sum w)^(t - 1) m
+      double m[2] = {};
+      for (int64_t i = 0; i < (int64_t)pl->weights.size(); i++) {
+        const int a[2] = {(int)(i / K), (int)(i % K)};
+        for (int d = 0; d < 2; d++)
+          m[d] += pl->weights[(size_t)i] * (p.convention == FFS_CONV_REF ? K - 1 - a[d] : a[d]);
+      }
+      const int64_t depth[2] = {2 * pl->t, pl->t_wide_tail};
+      for (int k = 0; k < 2; k++)
+        for (int d = 0; d < 2; d++)
+          pl->lin_wide[k][d] = depth[k] > 0 ? (double)depth[k] * ipow(sw, depth[k] - 1) * m[d] : 0.0;
+    }
   }
   if (p.precision == FFS_PREC_MIXED_F16) {
     // largest |K(k)| over the 32 x 32 frequencies (|K| does not depend on the convention), axis by axis from

@@ -67,6 +67,8 @@ struct TileArgs {
   int32_t scale_exp;  // FP16 form: the tile pair is scaled so that its largest fluctuation is below 2^scale_exp
   int32_t filter_exp;  // FP16 64-point launches: the filter table holds 2^filter_exp times the filter
   double dc_gain;  // K(0)^t: gain of the constant mode (mixed forms add mean * gain back in FP64)
+  double lin0, lin1;  // 64-point launches: first moments of the t-fold taps, sum of e0 g_t[e] and of e1 g_t[e] (a slope
+                      // s of the window moves the constant by s times this)
   int32_t linear_map;  // 1: workgroups take tiles in hardware order; 0: XCD-contiguous bands
   // 32-point family: 1 when the valid region fits one 16 x 16 block (V0, V1 <= 16).  The two inverse
   // stages then compute only output block 0.  Mixed forms (2 and 1 of 4 output blocks): with the inverse
