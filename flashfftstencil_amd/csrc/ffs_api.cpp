@@ -95,7 +95,7 @@ struct ffs_plan {
   bool stream = false;
   int32_t stream_E = 0, stream_V = 0, stream_nseg = 1;
   int64_t stream_t = 0, stream_tail = 0, stream_seg = 0;
-  double stream_dc[2][7] = {};
+  double stream_dc[2][3][7] = {};  // per depth: gain of every axis-0 tap, first moments of its filter along axes 1 and 2
   // 1D FP64 and BF16 plans: launches of depth line_t as one banded product (ffsk::launch_line), the last one of
   // depth line_tail; line_nb contraction blocks.  d_wide holds both depths' taps, then (BF16) their operands.
   bool line = false;
@@ -669,7 +669,11 @@ ffsk::Stream3Args make_stream_args(const ffs_plan* pl, const double* src, double
   const int hi = p.convention == FFS_CONV_REF ? 2 * p.radius : p.radius;
   a.h0 = a.h = (int32_t)(hi * (tail ? pl->stream_tail : pl->stream_t));
   a.linear_map = linear_map(pl) ? 1 : 0;
-  for (int e = 0; e < 7; e++) a.dc[e] = pl->stream_dc[tail ? 1 : 0][e];
+  for (int e = 0; e < 7; e++) {
+    a.dc[e] = pl->stream_dc[tail][0][e];
+    a.m1[e] = pl->stream_dc[tail][1][e];
+    a.m2[e] = pl->stream_dc[tail][2][e];
+  }
   return a;
 }
 
@@ -859,19 +863,28 @@ ffs_status plan_constants(ffs_plan* pl) {
     };
     pl->dc_main = ipow(sw, pl->t);
     pl->dc_tail = ipow(sw, pl->t_tail > 0 ? pl->t_tail : pl->t);
-    if (pl->stream) {  // gains of a constant plane per tap: the axis-0 marginal of the taps to the power t
-      const int K2 = K * K, hi = K - 1;
-      double m[7] = {};
+    if (pl->stream) {  // gain and first moments per axis-0 tap of the t-fold taps: products of polynomials in the axis-0
+                       // shift whose coefficients are (gain, moment 1, moment 2) of a filter in the plane
+      const int hi = K - 1;
+      double m[3][7] = {};
       for (int64_t i = 0; i < (int64_t)pl->weights.size(); i++) {
-        const int a0 = (int)(i / K2);
-        m[p.convention == FFS_CONV_REF ? hi - a0 : a0] += pl->weights[(size_t)i];
+        int e[3] = {(int)(i / (K * K)), (int)(i / K % K), (int)(i % K)};
+        if (p.convention == FFS_CONV_REF)
+          for (int& x : e) x = hi - x;
+        const double w = pl->weights[(size_t)i];
+        m[0][e[0]] += w;
+        m[1][e[0]] += w * e[1];
+        m[2][e[0]] += w * e[2];
       }
       for (int d = 0; d < 2; d++) {
-        double g[7] = {1.0};
+        double g[3][7] = {{1.0}};
         for (int64_t n = 0; n < (d ? pl->stream_tail : pl->stream_t); n++) {
-          double next[7] = {};
+          double next[3][7] = {};
           for (int i = 0; i < 7; i++)
-            for (int e = 0; e < K && i + e < 7; e++) next[i + e] += g[i] * m[e];
+            for (int e = 0; e < K && i + e < 7; e++) {
+              next[0][i + e] += g[0][i] * m[0][e];
+              for (int k = 1; k < 3; k++) next[k][i + e] += g[0][i] * m[k][e] + g[k][i] * m[0][e];
+            }
           std::memcpy(g, next, sizeof g);
         }
         std::memcpy(pl->stream_dc[d], g, sizeof g);

@@ -175,7 +175,8 @@ struct Stream3Args {
   int32_t V;            // valid width in the plane, both axes
   int32_t h0, h;        // window offset along the stream and in the plane
   int32_t linear_map;   // as in TileArgs
-  double dc[7];         // mixed form: gain of a constant plane e planes ahead
+  double dc[7];         // mixed form: gain of a constant plane e planes ahead, and the first moments of that tap's
+  double m1[7], m2[7];  // filter along both axes of the plane (a slope s moves the constant by s times this)
 };
 constexpr int kOpsFold = 6 * kLanes * 4;
 hipError_t gen_stream3d(void* H, bool mixed, int32_t E, const double* d_taps, int32_t K, int32_t convention, int32_t t,

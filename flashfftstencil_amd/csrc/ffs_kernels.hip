@@ -1634,6 +1634,14 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
 }
 
+// Lane k of a row takes lane k + 1's value, the row's last lane zero (row_shl:1).
+__device__ __forceinline__ double dpp_shl1(double x) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, x);
+  const uint32_t a = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x101, 0xF, 0xF, true);
+  const uint32_t b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(w >> 32), 0x101, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (uint64_t)a | ((uint64_t)b << 32));
+}
+
 // kx, ky, kz times the sums of x, y and z over the wave, as wave-uniform values (scalar registers).  The three share the lanes from the first exchange on (lane 4k carries
 // x, 4k + 1 y, 4k + 2 z), so they cost five exchanges inside the rows and two across them instead of three times four
 // and three times three row sums.
@@ -2688,14 +2696,18 @@ hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K
 // costs nothing.  E (odd, 2rt + 1 rounded up; missing taps are zero) is a template parameter: the sums stay in
 // registers.
 //
-// Registers and occupancy: BF16 236 VGPRs at E = 7, 2 waves per SIMD; FP64 274 at E = 5, 1 wave (2 with spills
+// Registers and occupancy: BF16 250 VGPRs at E = 7, 2 waves per SIMD; FP64 274 at E = 5, 1 wave (2 with spills
 // were 2% slower).  Bound by issue: BF16 E = 7 1068 VALU and 48 MFMAs per plane, 5,040 of the 6,300 cycles a
 // plane takes; FP64 E = 5 424 FP64 VALU and 64 FP64 MFMAs, 5,800 of 8,900.  Stores are ordinary ones: the rows
 // of 28 or 26 valid columns end inside cache lines, and as non-temporal stores they took 890 us per launch
 // instead of 626 (Box3D27P 512^3 BF16).  Box3D27P 512^3: BF16 262 -> 640, FP64 153 -> 355 GStencils/s.
 //
-// Mixed form: each plane's window is taken relative to its own mean c (FP64); the constant part of output
-// p is sum_e dc[e] c[p + e] with dc[e] the sum of the taps of G_e, added back in FP64 at the store.
+// Mixed form: each plane's window is taken relative to a fitted plane c + s1 (row - 15.5) + s2 (column - 15.5) (FP64,
+// read off 8 of its rows like the 64-point windows'); its image in output p, sum_e dc[e] (c, s1, s2)[p + e] with dc[e] the
+// sum of the taps of G_e and their first moments for the constant, is added back in FP64 at the store.  The pending
+// sums of the three live one per lane (lane k: the output k planes away), moved down by one lane per plane.  With the
+// mean alone the l2 error on waves of 60 to 130 points was 1.14 to 1.33 times that of the 16^3 tiles, with the plane 0.54
+// to 0.81 times (geometric means of 24 random cases; Box3D27P 512^3 x 32 6.90 -> 6.95 ms).
 // ---------------------------------------------------------------------------------------------
 struct OpsFold {  // BF16 pairings (Fh|Fh), (Fm|Fm), (Fl|Fh) of the 16 x 16 cosine and sine matrices
   bf8 c[3], s[3];
@@ -2735,14 +2747,19 @@ struct Plane3<PREC_BF16> {
   static __device__ __forceinline__ int row(int q, int v) { return 4 * q + v; }
   // small split products first, the dominant pairing last (forward); summed on their own (inverse)
   static __device__ __forceinline__ void fwd(const V4 (&z)[2][2], const void* sW, int lane, V4 (&y)[2][2]) {
+    const V4 d[2] = {z[0][0] - z[1][0], z[0][1] - z[1][1]}, m[2] = {z[0][0] + z[1][0], z[0][1] + z[1][1]};
+    fwd_folded(d, m, sW, lane, y);
+  }
+  // d, m: near - far and near + far rows of the column blocks
+  static __device__ __forceinline__ void fwd_folded(const V4 (&d)[2], const V4 (&m)[2], const void* sW, int lane, V4 (&y)[2][2]) {
     OpsFold f;
     load_ops_fold(f, static_cast<const u4*>(sW), lane);
     const f4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int C = 0; C < 2; C++) {
       bf8 A[3], B[3];
-      split_a<3>(z[0][C] - z[1][C], A);
-      split_a<3>(z[0][C] + z[1][C], B);
+      split_a<3>(d[C], A);
+      split_a<3>(m[C], B);
       f4 oc = FFS_MFMA_BF16(A[2], f.c[2], zero), os = FFS_MFMA_BF16(B[2], f.s[2], zero);
       oc = FFS_MFMA_BF16(A[1], f.c[1], oc);
       os = FFS_MFMA_BF16(B[1], f.s[1], os);
@@ -2834,24 +2851,44 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
   for (int k = 0; k < E - 1; k++)
 #pragma unroll
     for (int b = 0; b < 4; b++) acc[k][b >> 1][b & 1] = V4{0, 0, 0, 0};
-  double dacc[MIXED ? E - 1 : 1] = {};
+  // mixed form: this lane's gains and moments (lane k: tap E - 1 - k), and the pending images of the fitted planes
+  double gain = 0.0, mom1 = 0.0, mom2 = 0.0, pend = 0.0, pend1 = 0.0, pend2 = 0.0;
+  if constexpr (MIXED) {
+#pragma unroll
+    for (int k = 0; k < E; k++) {
+      gain = lane == k ? a.dc[E - 1 - k] : gain;
+      mom1 = lane == k ? a.m1[E - 1 - k] : mom1;
+      mom2 = lane == k ? a.m2[E - 1 - k] : mom2;
+    }
+  }
+  const double mid = (double)(4 * q) - 15.5, col = (double)j - 15.5;
   int64_t pl = wrap_near(p0 - a.h0, a.n0);
   load(pl);
   // One plane: transform it, add its filters to the partial sums, leave the finished coefficients in z.
-  auto take = [&](V4 (&z)[2][2], double& dout) {
-    V4 y[2][2];
-    dout = 0.0;
+  auto take = [&](V4 (&z)[2][2]) {
+    V4 y[2][2], d[2], m[2];
     if constexpr (MIXED) {
-      // plane mean over rows 0, 4, 8, 12, 19, 23, 27, 31
-      const double c =
-          wave_sum((raw[0][0][0] + raw[0][1][0]) + (raw[1][0][0] + raw[1][1][0])) * (1.0 / 256);
+      // rows 0, 4, 8, 12, 19, 23, 27, 31; the halves' means are 19 rows and 16 columns apart
+      const double nn = raw[0][0][0], nf = raw[0][1][0], fn = raw[1][0][0], ff = raw[1][1][0];
+      const double near = nn + nf, far = fn + ff;
+      double c = near + far, s1 = far - near, s2 = (nf + ff) - (nn + fn);
+      wave_sum3(c, s1, s2, 1.0 / 256, 1.0 / (128 * 19), 1.0 / (128 * 16), lane);
+      const double two = c + c, e = (s2 + s2) * col, sum[2] = {two + e, two - e};
 #pragma unroll
-      for (int b = 0; b < 4; b++)
+      for (int v = 0; v < 4; v++) {
+        const double diff = (s1 + s1) * (mid + v);
 #pragma unroll
-        for (int v = 0; v < 4; v++) z[b >> 1][b & 1][v] = (V)(raw[b >> 1][b & 1][v] - c);
-      dout = __builtin_fma(a.dc[E - 1], c, dacc[0]);
-#pragma unroll
-      for (int k = 1; k < E; k++) dacc[k - 1] = k < E - 1 ? __builtin_fma(a.dc[E - 1 - k], c, dacc[k < E - 1 ? k : 0]) : a.dc[0] * c;
+        for (int C = 0; C < 2; C++) {
+          d[C][v] = (V)((raw[0][C][v] - raw[1][C][v]) - diff);
+          m[C][v] = (V)((raw[0][C][v] + raw[1][C][v]) - sum[C]);
+        }
+      }
+      // Lanes from E on stay zero also when c, s1 or s2 is not finite, so that it leaves with the plane's last output.
+      const double p0 = __builtin_fma(gain, c, __builtin_fma(mom1, s1, __builtin_fma(mom2, s2, dpp_shl1(pend))));
+      const double p1 = __builtin_fma(gain, s1, dpp_shl1(pend1)), p2 = __builtin_fma(gain, s2, dpp_shl1(pend2));
+      pend = lane < E ? p0 : 0.0;
+      pend1 = lane < E ? p1 : 0.0;
+      pend2 = lane < E ? p2 : 0.0;
     } else {
 #pragma unroll
       for (int b = 0; b < 4; b++)
@@ -2863,7 +2900,10 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
     __builtin_amdgcn_sched_barrier(0);
     load(pl);  // the next plane's window, in flight through this plane's work
     __builtin_amdgcn_sched_barrier(0);
-    P::fwd(z, sW, lane, y);
+    if constexpr (MIXED)
+      P::fwd_folded(d, m, sW, lane, y);
+    else
+      P::fwd(z, sW, lane, y);
     __builtin_amdgcn_sched_barrier(0);
     P::fwd(y, sW, lane, z);
     lds_fence();
@@ -2891,12 +2931,11 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
     }
   };
   V4 z[2][2], y[2][2];
-  double dout;
   // The first E - 1 planes finish no output.  A loop of their own: with a branch around the stores instead,
   // the wait for the next window's loads would have to cover the stores issued after them.
-  for (int m = 0; m < E - 1; m++) take(z, dout);
+  for (int m = 0; m < E - 1; m++) take(z);
   for (int64_t m = 0; m < len; m++) {
-    take(z, dout);
+    take(z);
     lds_fence();
     __builtin_amdgcn_sched_barrier(0);
     P::inv(z, sW, lane, y);
@@ -2904,6 +2943,13 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
     P::inv(y, sW, lane, z);
     __builtin_amdgcn_sched_barrier(0);
     const __amdgpu_buffer_rsrc_t ro = rsrc(a.dst + (p0 + m) * plane);
+    double at[2] = {0.0, 0.0}, g1 = 0.0;  // the fitted planes' image at this lane's columns, and its slope along the rows
+    if constexpr (MIXED) {
+      const double c = lane_value(pend, 0), g2 = lane_value(pend2, 0) * col;
+      g1 = lane_value(pend1, 0);
+      at[0] = c + g2;
+      at[1] = c - g2;
+    }
 #pragma unroll
     for (int R = 0; R < 2; R++)
 #pragma unroll
@@ -2911,7 +2957,9 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
 #pragma unroll
         for (int v = 0; v < 4; v++) {
           const uint32_t off = (srow[R][v] | scol[C]) & kDrop ? kDrop : srow[R][v] + scol[C];
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, (double)z[R][C][v] + dout), ro, (int)off, 0, 0);
+          double x = z[R][C][v];
+          if constexpr (MIXED) x += __builtin_fma(R ? -g1 : g1, mid + v, at[C]);
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), ro, (int)off, 0, 0);
         }
   }
 }
