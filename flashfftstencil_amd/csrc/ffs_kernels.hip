@@ -3094,10 +3094,13 @@ hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, h
 // pad per 16 values (the column stride).
 // STEPS, the direct algorithm: its sums hold no values from beyond the stencil's reach, but the zeros around the band
 // turn an infinity or NaN anywhere in a group's window into NaN for the whole group.  A wave that has such a result takes
-// the launch's steps one by one in its LDS window, as k_direct1d does.  The test and the
-// path cost 1-4% of a launch (1D7P 2^24 x 100 351 -> 355 us, 5000 x 200 23.4 -> 24.5).
+// the launch's steps one by one in its LDS window, as k_direct1d does.  Its sums run in four chains, so that they round no
+// more than the steps did (l2 error against 80-bit sums over 120 random cases, relative to k_direct1d: geometric mean 0.86;
+// two chains, as in the transform algorithm, 1.07, and with the taps in plain doubles 1.42 and up to 22).  Both together:
+// 1D7P 2^24 x 100 351 -> 368 us, 5000 x 200 23.4 -> 24.6.
 template <bool STEPS>
 __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
+  constexpr int kChains = STEPS ? 4 : 2;
   extern __shared__ double lds[];
   const int kk = 16 * a.nb;                    // contraction length
   double* sT = lds;                            // g[-15 .. kk - 1], zeros outside the taps
@@ -3117,15 +3120,18 @@ __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
     } else {
       for (int i = lane; i < win; i += 64) sX[i + (i >> 4)] = a.src[wrap_near(base + i, a.n)];
     }
-    d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+    d4 acc[kChains];
+#pragma unroll
+    for (int c = 0; c < kChains; c++) acc[c] = d4{0.0, 0.0, 0.0, 0.0};
     for (int b = 0; b < a.nb; b++) {
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const int k = 16 * b + 4 * c + q;      // this lane's contraction index, in both operands
-        acc[c & 1] = FFS_MFMA64(sT[k - row + 15], sX[17 * (j + b) + 4 * c + q], acc[c & 1]);
+        acc[c % kChains] = FFS_MFMA64(sT[k - row + 15], sX[17 * (j + b) + 4 * c + q], acc[c % kChains]);
       }
     }
     d4 y = acc[0] + acc[1];
+    if (STEPS) y += acc[2] + acc[3];
     if (STEPS) {
       const bool finite = __builtin_isfinite(y[0]) & __builtin_isfinite(y[1]) & __builtin_isfinite(y[2]) & __builtin_isfinite(y[3]);
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite) != 0, 0)) {
@@ -3251,28 +3257,60 @@ __global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
 }
 
 // Taps of the t-fold 1D stencil in correlation order (ref: e = 2r - a; centred: e = a), by repeated squaring of the
-// tap polynomial in FP64; one workgroup of kLineMaxTaps threads, thread i forms coefficient i.
+// tap polynomial; one workgroup of kLineMaxTaps threads, thread i forms coefficient i.  A rounding error of a square doubles
+// with every later one, those of neighbouring coefficients are alike, and all outputs share them: in plain doubles the gain
+// of a launch of depth 61 (1D7P) was off by 4.7e-16, with only the last squares plain 2.2e-16, like this 4e-17.  Every sum is
+// compensated: it starts from `big`, which no product exceeds, so s - acc is exact and the second FMA is what the
+// addition lost (Dekker's fast two-sum with an FMA for the product).  Polynomials of up to kPairTaps coefficients also keep
+// their own rounding (high, low).
+constexpr int kPairTaps = 128;
 __global__ __launch_bounds__(kLineMaxTaps) void k_gen_line_taps(double* out, const double* taps, int32_t K,
                                                                 int32_t convention, int32_t t) {
-  __shared__ double one[kLineMaxTaps], cur[kLineMaxTaps];
+  __shared__ double2 one[kLineMaxTaps], cur[kLineMaxTaps];
   const int i = threadIdx.x;
-  one[i] = i < K ? taps[convention == 0 ? K - 1 - i : i] : 0.0;
+  one[i] = make_double2(i < K ? taps[convention == 0 ? K - 1 - i : i] : 0.0, 0.0);
   cur[i] = one[i];
   __syncthreads();
+  double step = 0.0;  // sum of the taps' sizes: bounds every coefficient of a power, raised to that power
+  for (int e = 0; e < K; e++) step += fabs(one[e].x);
+  double bound = step;
   int n = K;  // coefficients of cur
-  auto times = [&](const double* f, int m) {  // cur *= f (m coefficients)
-    double sum = 0.0;
-    for (int e = max(0, i - n + 1); e < m && e <= i; e++) sum = __builtin_fma(f[e], cur[i - e], sum);
+  auto times = [&](const double2* f, int m, double fbound) {  // cur *= f (m coefficients)
+#pragma clang fp contract(off)
+    const int first = max(0, i - n + 1), last = min(m - 1, i);
+    bound *= fbound;
+    const double big = 4.0 * bound;
+    double acc = big, low = 0.0;
+    const bool pairs = n + m - 1 <= kPairTaps;
+    auto add = [&](double2 a, double2 b) {
+      const double s = __builtin_fma(a.x, b.x, acc);
+      low += __builtin_fma(a.x, b.x, -(s - acc));
+      if (pairs) low = __builtin_fma(a.x, b.y, __builtin_fma(a.y, b.x, low));
+      acc = s;
+    };
+    int e = first;
+    for (; e + 7 <= last; e += 8) {  // eight at a time: the LDS reads of one group overlap
+      double2 a[8], b[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        a[k] = f[e + k];
+        b[k] = cur[i - e - k];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) add(a[k], b[k]);
+    }
+    for (; e <= last; e++) add(f[e], cur[i - e]);
     __syncthreads();
-    cur[i] = sum;
+    const double sum = acc - big, h = sum + low;
+    cur[i] = make_double2(h, low - (h - sum));
     n += m - 1;
     __syncthreads();
   };
   for (int bit = 30 - __builtin_clz(t); bit >= 0; bit--) {
-    times(cur, n);
-    if ((t >> bit) & 1) times(one, K);
+    times(cur, n, bound);
+    if ((t >> bit) & 1) times(one, K, step);
   }
-  out[i] = i < n ? cur[i] : 0.0;
+  out[i] = i < n ? cur[i].x : 0.0;
 }
 
 // Operands of k_line_bf16: [block b][term][lane] of 4 words; element e of lane (i + 16q) is T[i][32 b + 8q + e] =

@@ -206,3 +206,21 @@ def test_direct_1d_infinities_and_nan(ffs, torch_cuda, algorithm, convention, ra
         assert np.array_equal(got[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)]), taps
         # |out| <= max |in| < 1 in every step, each rounding K + 1 times
         assert np.abs(got[ok] - ref[ok]).max(initial=0.0) <= 2 ** -53 * (K + 1) * steps, taps
+
+
+@pytest.mark.parametrize("algorithm", ["direct", "fft"])
+@pytest.mark.parametrize("shape,steps", [("Heat-1D", 20), ("Heat-1D", 182), ("1D5P", 61), ("1D7P", 20), ("1D7P", 61), ("1D7P", 182)])
+def test_1d_gain_of_deep_launches(ffs, torch_cuda, algorithm, shape, steps):
+    # The mean of the grid is multiplied by (sum w)^T.  Roundings of single outputs average out over 11,556 points; what is
+    # left is the gain error of the t-fold taps, which every output shares: below half an ulp per launch.
+    torch = torch_cuda
+    _, r, w, _ = ffs.named_stencil(shape, seed=3)
+    x = torch.rand(11556, dtype=torch.float64, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    y = torch.empty_like(x)
+    with ffs.Plan(1, (11556,), w, r, steps, algorithm=algorithm) as plan:
+        plan.run(x, y)
+        torch.cuda.synchronize()
+        launches = plan.info["launches"]
+    want = x.cpu().numpy().astype(np.longdouble).mean() * np.asarray(w, dtype=np.longdouble).sum() ** steps
+    got = y.cpu().numpy().astype(np.longdouble).mean()
+    assert abs(got / want - 1) <= 2 ** -53 * launches, (float(got / want - 1), launches)
