@@ -38,6 +38,7 @@ PRECISIONS = {"fp64": 0, "bf16": 1, "mixed": 1, "f32": 2, "bf16x2": 3, "f16": 4}
 CONVENTIONS = {"ref": 0, "centred": 1, "centered": 1}
 ALGORITHMS = {"fft": 0, "direct": 1, "auto": 2}
 MAPPINGS = {"auto": 0, "xcd": 1, "linear": 2}
+RUN_KERNELS = {"blocks": 0, "wide": 1, "stream": 2, "line": 3}
 
 
 class FFSError(RuntimeError):
@@ -88,7 +89,8 @@ class PlanInfo(ctypes.Structure):
         ("bytes_per_block", ctypes.c_double),
         ("algorithm", ctypes.c_int32),
         ("mapping", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 2),
+        ("run_kernel", ctypes.c_int32),
+        ("run_depth", ctypes.c_int32),
     ]
 
     def as_dict(self) -> dict:

@@ -1268,6 +1268,8 @@ ffs_status ffs_plan_get_info(const ffs_plan* pl, ffs_plan_info* info) {
   info->convention = p.convention;
   info->algorithm = pl->direct ? FFS_ALGO_DIRECT : FFS_ALGO_FFT;
   info->mapping = linear_map(pl) ? FFS_MAP_LINEAR : FFS_MAP_XCD;
+  info->run_kernel = pl->line ? FFS_RUN_LINE : pl->stream ? FFS_RUN_STREAM : pl->wide ? FFS_RUN_WIDE : FFS_RUN_BLOCKS;
+  info->run_depth = (int32_t)(pl->line ? pl->line_t : pl->stream ? pl->stream_t : pl->wide ? 2 * pl->t : pl->t);
   if (pl->direct) {
     const ffsk::DirectArgs a = make_direct_args(pl, nullptr, nullptr, pl->t);
     const int r = p.radius, K = 2 * r + 1;

@@ -97,7 +97,8 @@ typedef enum ffs_mapping { FFS_MAP_AUTO = 0, FFS_MAP_XCD = 1, FFS_MAP_LINEAR = 2
 
 /* ffs_problem.flags bits.
  *   FULL_STAGES: on 32-point tiles whose valid region fits one 16 x 16 block (V <= 16), compute every
- *                output block of the two inverse stages instead of only the kept one.  The results are
+ *                output block of the two inverse stages instead of only the kept one (runs of the mixed forms that
+ *                launch 64-point windows have no such stages: there the flag acts on ffs_run_block).  The results are
  *                bitwise the same (the kept values come from the same operands in the same order); it
  *                exists to check exactly that, and costs ~1.4x the tile time.  No reference counterpart. */
 #define FFS_FLAG_FULL_STAGES 0x1
@@ -122,6 +123,14 @@ typedef struct ffs_problem {
   int32_t reserved;
 } ffs_problem;
 
+/* Kernels of a whole run. */
+typedef enum ffs_run_kernel {
+  FFS_RUN_BLOCKS = 0, /* the block kernel of ffs_run_block, once per block */
+  FFS_RUN_WIDE = 1,   /* mixed 2D forms: two blocks per launch on 64-point windows */
+  FFS_RUN_STREAM = 2, /* 3D FP64 and BF16: planes transformed, axis 0 direct */
+  FFS_RUN_LINE = 3    /* 1D FP64 and BF16: banded products */
+} ffs_run_kernel;
+
 /* What a plan chose. */
 typedef struct ffs_plan_info {
   int32_t dims, radius;
@@ -135,15 +144,17 @@ typedef struct ffs_plan_info {
   int64_t blocks;         /* fused blocks per run, tail included */
   int64_t tiles;          /* tiles per block */
   int64_t launches;       /* kernel launches per run: `blocks`; half of them (rounded up) where the mixed 2D
-                             forms take two blocks per launch on 64-point windows (V <= 16, blocks >= 2); in 3D
-                             (FP64, BF16) those of the streamed kernel, whose depth is its own, on grids where
-                             it is the faster one.  ffs_run_block always runs one block of depth `fuse`. */
+                             forms take two blocks per launch on 64-point windows (V <= 16, blocks >= 2); those of
+                             the streamed kernel in 3D (FP64, BF16) and of the banded products in 1D (FP64, BF16),
+                             whose depth is their own, where they are the faster ones.  ffs_run_block always runs one
+                             block of depth `fuse`. */
   double flops_per_block; /* flops one block executes: matrix-core flops (FFT; see the kernels' header
                              comment) or FP64 FMA flops including the halo recomputation (DIRECT) */
   double bytes_per_block; /* algorithmic HBM bytes of one block: 16 B per grid point */
   int32_t algorithm;      /* ffs_algorithm actually used (FFT or DIRECT) */
   int32_t mapping;        /* ffs_mapping used by the tile kernels (XCD or LINEAR) */
-  int32_t reserved[2];
+  int32_t run_kernel;     /* ffs_run_kernel: what a whole run launches */
+  int32_t run_depth;      /* steps per launch of a whole run (the last launch takes the rest) */
 } ffs_plan_info;
 
 typedef struct ffs_plan ffs_plan;

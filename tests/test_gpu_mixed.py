@@ -236,7 +236,8 @@ def test_bf16x2_form_withdrawn(ffs, torch_cuda):
 def test_out16_bitwise_equals_full_stages(ffs, oracle, torch_cuda, form, convention, radius, fuse, size):
     # 32-point tiles with V <= 16: the reduced inverse stages (only the kept output block, from the
     # shifted inverse operands) must give bitwise the values of the full stages at those positions.
-    # Steps 2 t + 1: a main block and a tail block of another shift.  (3, 2): V = 20 > 16, full both ways.
+    # Steps 2 t + 1: a main block and a tail block of another shift, compared one by one (a whole run of the mixed forms
+    # launches 64-point windows instead, which have no reduced stages).  (3, 2): V = 20 > 16, full both ways.
     torch = torch_cuda
     rng = np.random.default_rng(700 + 10 * radius + fuse)
     w = rng.random((2 * radius + 1) ** 2)
@@ -247,14 +248,20 @@ def test_out16_bitwise_equals_full_stages(ffs, oracle, torch_cuda, form, convent
     for full in (False, True):
         plan = ffs.Plan(2, size, w, radius, 2 * fuse + 1, precision=form, convention=convention, fuse=fuse, tile=32,
                         full_stages=full)
-        d = torch.empty_like(d_in)
-        plan.run(d_in, d)
+        d = [torch.empty_like(d_in) for _ in range(3)]
+        plan.run(d_in, d[0])
+        plan.run_block(d_in, d[1])
+        plan.run_block(d_in, d[2], tail=True)
         torch.cuda.synchronize()
         info = plan.info
         plan.close()
         outs.append(d)
-    assert info["valid"][0] == 32 - 2 * radius * fuse
-    assert torch.equal(outs[0], outs[1]), (form, convention, radius, fuse, float((outs[0] - outs[1]).abs().max()))
+    assert info["valid"][0] == 32 - 2 * radius * fuse and info["fuse_tail"] == 1
+    for k, (a, b) in enumerate(zip(*outs)):
+        assert torch.equal(a, b), (form, convention, radius, fuse, ("run", "main", "tail")[k], float((a - b).abs().max()))
+    for k, depth in ((1, fuse), (2, 1)):
+        ref = oracle.sweep(x, radius, w, depth, convention=0 if convention == "ref" else 1)
+        assert oracle.errors(outs[0][k].cpu().numpy(), ref)[1] <= (1e-12 if form == "fp64" else TOL_MIXED)
 
 
 @pytest.mark.parametrize("form", ["f16", "bf16"])

@@ -342,9 +342,9 @@ def test_3d_mappings_bitwise_equal(ffs, oracle, torch_cuda, precision):
                                                 (1, (260, 78, 84), 2), (2, (121, 113, 140), 3), (3, (90, 131, 157), 2),
                                                 (1, (129, 257, 65), 1)])
 def test_3d_streamed(ffs, oracle, torch_cuda, precision, tol, convention, radius, sizes, steps):
-    """3D grids large enough for the streamed kernel: every tap count (3, 5, 7), main and tail depths, planes one
-    past and one short of a multiple of the valid width, segments of unequal length, fewer planes than
-    the stencil reaches (3), signed taps."""
+    """3D grids around the size from which the streamed kernel is the faster one (which kernel runs is the planner's choice
+    here; test_3d_streamed_forms asserts it): planes one past and one short of a multiple of the valid width, segments of
+    unequal length, few planes, signed taps."""
     torch = torch_cuda
     rng = np.random.default_rng(40 * radius + steps)
     w = rng.standard_normal((2 * radius + 1) ** 3)
@@ -368,8 +368,8 @@ def test_3d_streamed(ffs, oracle, torch_cuda, precision, tol, convention, radius
                                             (2, 4099, 130), (1, 5000, 248), (12, 1500, 30), (40, 700, 2), (60, 2000, 9)])
 def test_1d_banded_product(ffs, oracle, torch_cuda, precision, tol, convention, radius, n, steps):
     """1D runs as banded products: grids around a tile of 256 outputs, smaller than the stencil's reach, numbers of
-    taps around a multiple of the contraction block (2rt + 16 = 16 b, 32 b and one past), up to the deepest launch and past it
-    (a tail of another depth), wide stencils, signed taps."""
+    taps around a multiple of the contraction block (2rt + 16 = 16 b, 32 b and one past), up to the deepest launch and past it,
+    wide stencils, signed taps."""
     torch = torch_cuda
     rng = np.random.default_rng(radius + steps)
     w = rng.standard_normal(2 * radius + 1)
@@ -438,3 +438,88 @@ def test_3d_streamed_smooth_fields_as_exact_as_blocks(ffs, oracle, torch_cuda, c
     run = oracle.errors(d_out.cpu().numpy(), ref)[2]
     blocks = oracle.errors(a.cpu().numpy(), ref)[2]
     assert run <= blocks, (run, blocks, info)
+
+
+def _signed_mean_one(radius, dims, seed):
+    rng = np.random.default_rng(seed)
+    w = rng.standard_normal((2 * radius + 1) ** dims)
+    w += 2.0 * np.abs(w).sum() / w.size
+    return w / w.sum()
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("precision,radius,sizes,steps,depth,launches", [
+    ("fp64", 1, (129, 257, 65), 1, 1, 1), ("fp64", 1, (2, 600, 610), 5, 1, 5), ("fp64", 1, (150, 131, 139), 7, 2, 4),
+    ("fp64", 1, (2, 900, 800), 4, 2, 2), ("fp64", 2, (121, 113, 140), 3, 1, 3), ("fp64", 2, (3, 700, 690), 2, 1, 2),
+    ("bf16", 1, (129, 257, 65), 1, 1, 1), ("bf16", 1, (3, 900, 900), 4, 1, 4), ("bf16", 1, (150, 131, 139), 7, 2, 4),
+    ("bf16", 1, (2, 600, 610), 5, 2, 3), ("bf16", 1, (5, 1000, 1000), 11, 3, 4), ("bf16", 2, (140, 150, 160), 3, 1, 3),
+    ("bf16", 3, (90, 131, 157), 2, 1, 2), ("bf16", 3, (5, 500, 500), 2, 1, 2)])
+def test_3d_streamed_forms(ffs, oracle, torch_cuda, convention, precision, radius, sizes, steps, depth, launches):
+    """The streamed kernel in every form: 3, 5 and 7 taps along axis 0 (FP64 3 and 5), a last launch of a smaller depth (padded
+    taps), fewer planes than taps, signed taps.  The route and its depth are asserted."""
+    torch = torch_cuda
+    w = _signed_mean_one(radius, 3, 40 * radius + steps)
+    x = oracle.uniform(300 + steps, sizes)
+    d_in = torch.from_numpy(x).cuda()
+    d_out = torch.empty_like(d_in)
+    with ffs.Plan(3, sizes, w, radius, steps, precision=precision, convention=convention) as plan:
+        plan.run(d_in, d_out)
+        torch.cuda.synchronize()
+        info = plan.info
+    assert (info["run_kernel"], info["run_depth"], info["launches"]) == (ffs.RUN_KERNELS["stream"], depth, launches), info
+    ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
+    assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= (1e-12 if precision == "fp64" else 1e-6), info
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("precision,radius,n,steps,depth,launches", [
+    ("fp64", 3, 900, 101, 51, 2), ("fp64", 60, 2000, 10, 4, 3), ("fp64", 3, 700, 83, 42, 2), ("fp64", 1, 3001, 249, 125, 2),
+    ("fp64", 100, 3000, 5, 2, 3), ("bf16", 3, 900, 101, 34, 3), ("bf16", 60, 2000, 9, 2, 5), ("bf16", 2, 500, 249, 63, 4),
+    ("bf16", 24, 400, 21, 6, 4)])
+def test_1d_banded_product_tails(ffs, oracle, torch_cuda, convention, precision, radius, n, steps, depth, launches):
+    """Banded products whose last launch has another depth (its own taps and, in the mixed form, operands), wide and narrow
+    stencils; the route and its depth are asserted."""
+    torch = torch_cuda
+    assert steps % depth != 0 and -(-steps // depth) == launches
+    w = _signed_mean_one(radius, 1, radius + steps)
+    x = oracle.uniform(70 + n, (n,))
+    d_in = torch.from_numpy(x).cuda()
+    d_out = torch.empty_like(d_in)
+    with ffs.Plan(1, (n,), w, radius, steps, precision=precision, convention=convention) as plan:
+        plan.run(d_in, d_out)
+        torch.cuda.synchronize()
+        info = plan.info
+    assert (info["run_kernel"], info["run_depth"], info["launches"]) == (ffs.RUN_KERNELS["line"], depth, launches), info
+    ref = oracle.sweep(x, radius, w, steps, convention=0 if convention == "ref" else 1)
+    assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= (1e-12 if precision == "fp64" else 1e-6), info
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("dims,sizes,radius,fuse,steps,precision,algorithm,kernel", [
+    (1, (2000,), 1, 50, 130, "fp64", "fft", "line"), (1, (2000,), 3, 20, 47, "fp64", "fft", "line"),
+    (1, (700,), 2, 30, 71, "bf16", "fft", "line"), (1, (241,), 3, 37, 75, "bf16", "fft", "line"),
+    (1, (5000,), 1, 40, 100, "fp64", "direct", "line"), (1, (3000,), 2, 17, 40, "fp64", "direct", "line"),
+    (1, (2500,), 3, 9, 22, "fp64", "direct", "line"),
+    (2, (75, 90), 2, 4, 11, "f16", "fft", "wide"), (2, (75, 90), 2, 4, 11, "bf16", "fft", "wide"),
+    (2, (33, 61), 1, 8, 21, "f16", "fft", "wide"), (2, (33, 61), 3, 3, 8, "bf16", "fft", "wide"),
+    (2, (64, 48), 1, 15, 40, "f16", "fft", "wide"),
+    (3, (150, 131, 139), 1, 2, 7, "fp64", "fft", "stream"), (3, (150, 131, 139), 1, 2, 7, "bf16", "fft", "stream")])
+def test_run_block_where_runs_launch_other_kernels(ffs, oracle, torch_cuda, convention, dims, sizes, radius, fuse, steps,
+                                                   precision, algorithm, kernel):
+    """ffs_run_block, main and tail, on plans whose whole runs launch other kernels: the 240-point windows, k_direct1d, the
+    32-point mixed tiles with V <= 16 and the 16^3 tiles."""
+    torch = torch_cuda
+    w = _signed_mean_one(radius, dims, 9 * radius + fuse)
+    x = oracle.uniform(11 + fuse, sizes)
+    d_in = torch.from_numpy(x).cuda()
+    with ffs.Plan(dims, sizes, w, radius, steps, precision=precision, convention=convention, fuse=fuse,
+                  algorithm=algorithm) as plan:
+        info = plan.info
+        assert info["run_kernel"] == ffs.RUN_KERNELS[kernel] and info["fuse"] == fuse and info["fuse_tail"] == steps % fuse
+        for tail in (False, True):
+            d_out = torch.empty_like(d_in)
+            plan.run_block(d_in, d_out, tail=tail)
+            torch.cuda.synchronize()
+            ref = oracle.sweep(x, radius, w, info["fuse_tail"] if tail else fuse, convention=0 if convention == "ref" else 1)
+            tol = 1e-12 if precision == "fp64" else 1e-6
+            assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= tol, (tail, info)
