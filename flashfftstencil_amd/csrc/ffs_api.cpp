@@ -225,11 +225,18 @@ bool depth_in_range(const ffs_plan* pl, int64_t depth) {
 // plus 6,000 for a wave's chain of load, product and store, plus the larger of the memory time (16 B per point at
 // 5.3 TB/s) and the products (FP64: 256 cycles per block of 16 and tile; BF16: 120 per block of 32 and tile, LDS reads
 // included, and 250 for the tile's split).
+// Direct runs of one shallow block on long lines keep k_direct1d, which streams 2048-point windows at 5.3 TB/s where the
+// 256-point ones reach 4.8, until its steps cost more than that: above 2^24 points up to t = 12 (radius 1: 18), product over
+// k_direct1d at 60,000,001 points Heat-1D t = 8 1.10, 18 1.03, 24 0.84; 1D5P 8 1.07, 12 0.99; 1D7P 8 1.10, 12 1.02, 16 0.90;
+// above 2^20 up to t = 6 (at 4,000,001 Heat-1D 4 1.08, 8 0.96; 1D7P 3 1.18, 6 1.04, 8 0.96; at 9,000,001 1D7P 6 1.08, 8 0.98).
 void choose_line(ffs_plan* pl) {
   const ffs_problem& p = pl->prob;
   const int64_t r = p.radius;
   const bool fp64 = p.precision == FFS_PREC_FP64;
   if (p.dims != 1 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
+  if (pl->direct && pl->nblocks == 1 && p.sizes[0] > ((int64_t)1 << 20) &&
+      pl->t <= (p.sizes[0] <= ((int64_t)1 << 24) ? 6 : r == 1 ? 18 : 12))
+    return;
   const int64_t block = fp64 ? 16 : 32, nbmax = fp64 ? ffsk::kLineMaxNb64 : ffsk::kLineMaxNbBF;
   const int64_t most = std::min<int64_t>(ffsk::kLineMaxTaps, block * nbmax - 15);
   double best = 1e300;

@@ -224,3 +224,27 @@ def test_1d_gain_of_deep_launches(ffs, torch_cuda, algorithm, shape, steps):
     want = x.cpu().numpy().astype(np.longdouble).mean() * np.asarray(w, dtype=np.longdouble).sum() ** steps
     got = y.cpu().numpy().astype(np.longdouble).mean()
     assert abs(got / want - 1) <= 2 ** -53 * launches, (float(got / want - 1), launches)
+
+
+@pytest.mark.parametrize("radius,n,steps,kernel", [
+    (1, 1 << 20, 3, "line"), (1, (1 << 20) + 1, 6, "blocks"), (2, (1 << 20) + 1, 7, "line"), (3, 1 << 24, 6, "blocks"),
+    (3, (1 << 24) + 1, 12, "blocks"), (3, (1 << 24) + 1, 13, "line"), (1, (1 << 24) + 1, 18, "blocks"),
+    (1, (1 << 24) + 1, 19, "line"), (2, (1 << 24) + 1, 13, "line")])
+def test_direct_1d_shallow_runs_on_long_lines(ffs, torch_cuda, radius, n, steps, kernel):
+    # Long lines and few steps keep the streaming kernel, which is the faster one there; both sides of the rule's edges against the
+    # transform algorithm (the banded product, itself held to the oracle).
+    torch = torch_cuda
+    rng = np.random.default_rng(radius + steps)
+    w = rng.random(2 * radius + 1)
+    w /= w.sum()
+    x = torch.rand(n, dtype=torch.float64, device="cuda", generator=torch.Generator(device="cuda").manual_seed(steps))
+    outs = []
+    for algorithm in ("direct", "fft"):
+        y = torch.empty_like(x)
+        with ffs.Plan(1, (n,), w, radius, steps, algorithm=algorithm) as plan:
+            plan.run(x, y)
+            torch.cuda.synchronize()
+            assert plan.info["run_kernel"] == ffs.RUN_KERNELS[kernel if algorithm == "direct" else "line"]
+        outs.append(y)
+    # values below 1, a rounding of each of the K multiply-adds of every step at most
+    assert float((outs[0] - outs[1]).abs().max()) <= 2 ** -53 * (2 * radius + 2) * steps
