@@ -266,20 +266,27 @@ void choose_line(ffs_plan* pl) {
 int64_t direct_segments(const ffs_problem& p, int num_cus, int64_t t, int64_t strips) {
   const int64_t n0 = p.sizes[0], fill = 2 * (int64_t)p.radius * t + t - 1;
   const int64_t resident = (int64_t)num_cus * (p.dims == 2 ? 2 : 1);
-  double best = 1e300;
-  int64_t best_seg = n0;
   int64_t most = std::min<int64_t>(n0, std::max<int64_t>(1, 8 * resident / strips + 1));
   const int64_t of16 = (n0 + 15) / 16;
   if (strips * of16 >= num_cus / 2) most = std::min(most, of16);
-  for (int64_t nseg = 1; nseg <= most; nseg++) {
-    const int64_t seg = (n0 + nseg - 1) / nseg, units = strips * ((n0 + seg - 1) / seg);
+  double best = 1e300;
+  int64_t best_seg = n0;
+  // For a number of rounds the shortest segment is the best one, and it belongs to the most segments that fit them: one
+  // candidate per round (plus the 2D launch of one workgroup per CU) instead of one per number of segments.
+  auto consider = [&](int64_t nseg) {
+    if (nseg < 1) return;
+    const int64_t seg = (n0 + std::min(nseg, most) - 1) / std::min(nseg, most), units = strips * ((n0 + seg - 1) / seg);
     const double rounds = p.dims == 2 && units <= num_cus ? 0.68 : (double)((units + resident - 1) / resident);
     const double cost = rounds * (double)(seg + fill);
     if (cost < best * (1 - 1e-9)) {
       best = cost;
       best_seg = seg;
     }
-  }
+  };
+  if (p.dims == 2) consider(num_cus / strips);
+  int64_t rounds = (strips + resident - 1) / resident;
+  for (; rounds * resident / strips < most; rounds++) consider(rounds * resident / strips);
+  consider(most);
   return best_seg;
 }
 
