@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -787,14 +788,14 @@ ffs_status plan_host(const ffs_problem* p, ffs_plan* pl) {
   return choose_config(pl);
 }
 
-// CU count of a device that is a gfx950, else 0 with the reason in `arch`.  Asked once per device (a query
-// takes longer than a small run's launches).
+// CU count and architecture of a device, asked once (a query takes longer than a small run's launches); a query that
+// fails is asked again by the next plan.
 struct DeviceFacts {
-  std::once_flag once;
-  hipError_t err = hipSuccess;
+  std::atomic<bool> known{false};
   int num_cus = 0;
   char arch[32] = {};
 };
+std::mutex g_devices_mu;
 constexpr int kMaxDevices = 256;
 DeviceFacts g_devices[kMaxDevices];
 
@@ -809,14 +810,16 @@ ffs_status plan_device(ffs_plan* pl) {
   pl->dev = pl->prob.device;
   if (hipSetDevice(pl->dev) != hipSuccess) return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
   DeviceFacts& f = g_devices[pl->dev];
-  std::call_once(f.once, [&] {
-    hipDeviceProp_t prop;
-    f.err = hipGetDeviceProperties(&prop, pl->dev);
-    if (f.err != hipSuccess) return;
-    std::snprintf(f.arch, sizeof f.arch, "%.*s", 31, prop.gcnArchName);
-    f.num_cus = prop.multiProcessorCount;
-  });
-  if (f.err != hipSuccess) return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
+  if (!f.known.load(std::memory_order_acquire)) {
+    std::lock_guard<std::mutex> lock(g_devices_mu);
+    if (!f.known.load(std::memory_order_relaxed)) {
+      hipDeviceProp_t prop;
+      if (hipGetDeviceProperties(&prop, pl->dev) != hipSuccess) return fail(FFS_ERR_HIP, "cannot query device %d", pl->dev);
+      std::snprintf(f.arch, sizeof f.arch, "%.*s", 31, prop.gcnArchName);
+      f.num_cus = prop.multiProcessorCount;
+      f.known.store(true, std::memory_order_release);
+    }
+  }
   if (std::strncmp(f.arch, "gfx950", 6) != 0)
     return fail(FFS_ERR_NO_DEVICE, "device %d is %s; this library is built for gfx950 only", pl->dev, f.arch);
   pl->num_cus = f.num_cus;

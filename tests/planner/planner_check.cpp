@@ -7,6 +7,29 @@
 #include <cstring>
 #include <random>
 
+// The device queries of the library's host source, answered here.
+static int props_calls = 0, props_failing = 0;
+static hipError_t fake_count(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+static hipError_t fake_set(int) { return hipSuccess; }
+static hipError_t fake_props(hipDeviceProp_t* prop, int) {
+  props_calls++;
+  if (props_failing > 0) {
+    props_failing--;
+    return hipErrorNotReady;
+  }
+  std::memset(prop, 0, sizeof *prop);
+  std::strcpy(prop->gcnArchName, "gfx950:sramecc+:xnack-");
+  prop->multiProcessorCount = 256;
+  return hipSuccess;
+}
+#undef hipGetDeviceProperties
+#define hipGetDeviceCount fake_count
+#define hipSetDevice fake_set
+#define hipGetDeviceProperties fake_props
+
 #include "../../flashfftstencil_amd/csrc/ffs_api.cpp"
 
 static int failures = 0;
@@ -75,7 +98,17 @@ static void segments_cost() {
   EXPECT(sum > 0 && best < 5e-6, "%g s per call", best);
 }
 
+// A device is asked once, but a query that failed is no answer: the next plan asks again.
+static void device_query() {
+  props_failing = 1;
+  ffs_plan pl;
+  EXPECT(plan_device(&pl) == FFS_ERR_HIP && props_calls == 1, "%d calls", props_calls);
+  EXPECT(plan_device(&pl) == FFS_OK && props_calls == 2 && pl.num_cus == 256, "%s, %d calls", g_err.c_str(), props_calls);
+  EXPECT(plan_device(&pl) == FFS_OK && props_calls == 2 && pl.num_cus == 256, "%s, %d calls", g_err.c_str(), props_calls);
+}
+
 int main() {
+  device_query();
   segments();
   segments_cost();
   if (failures) {
