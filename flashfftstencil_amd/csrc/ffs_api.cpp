@@ -235,14 +235,15 @@ void choose_line(ffs_plan* pl) {
   const int64_t r = p.radius;
   const bool fp64 = p.precision == FFS_PREC_FP64;
   if (p.dims != 1 || r < 1 || p.steps < 1 || (!fp64 && p.precision != FFS_PREC_MIXED_BF16)) return;
-  if (pl->direct && pl->nblocks == 1 && p.sizes[0] > ((int64_t)1 << 20) &&
+  if (pl->direct && (pl->nblocks == 1 || p.fuse > 0) && p.sizes[0] > ((int64_t)1 << 20) &&
       pl->t <= (p.sizes[0] <= ((int64_t)1 << 24) ? 6 : r == 1 ? 18 : 12))
     return;
   const int64_t block = fp64 ? 16 : 32, nbmax = fp64 ? ffsk::kLineMaxNb64 : ffsk::kLineMaxNbBF;
   const int64_t most = std::min<int64_t>(ffsk::kLineMaxTaps, block * nbmax - 15);
   double best = 1e300;
-  for (int64_t t = 1; 2 * r * t + 1 <= most && t <= p.steps; t++) {
-    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
+  for (int64_t t = p.fuse > 0 ? pl->t : 1; 2 * r * t + 1 <= most && t <= p.steps; t++) {
+    if (p.fuse > 0 && t > pl->t) break;  // a depth that the caller set is the depth of the launches
+    const int64_t nl = (p.steps + t - 1) / t, te = p.fuse > 0 ? t : (p.steps + nl - 1) / nl;
     const int64_t nb = (2 * r * te + 16 + block - 1) / block;
     const double n = (double)p.sizes[0];
     const double work = std::ceil(n / 256.0 / 1024.0) * (fp64 ? (double)nb * 256.0 : (double)nb * 120.0 + 250.0);
@@ -361,8 +362,9 @@ void choose_stream(ffs_plan* pl) {
   const double pairs = (double)pl->units;
   double best = (double)pl->nblocks *
                 (8000.0 + std::ceil(pairs / (fp64 ? 512.0 : 768.0)) * (fp64 ? 45000.0 : 36000.0) - (pairs <= 256.0 ? 10000.0 : 0.0));
-  for (int64_t t = 1; 2 * r * t + 1 <= emax; t++) {
-    const int64_t nl = (p.steps + t - 1) / t, te = (p.steps + nl - 1) / nl;
+  for (int64_t t = p.fuse > 0 ? pl->t : 1; 2 * r * t + 1 <= emax; t++) {
+    if (p.fuse > 0 && t > pl->t) break;  // a depth that the caller set is the depth of the launches
+    const int64_t nl = (p.steps + t - 1) / t, te = p.fuse > 0 ? t : (p.steps + nl - 1) / nl;
     if ((nl > 1 && pl->nblocks == 1) || !depth_in_range(pl, te)) continue;
     const int64_t V = 32 - 2 * r * te;
     const int64_t tiles = ((p.sizes[1] + V - 1) / V) * ((p.sizes[2] + V - 1) / V);
@@ -1579,14 +1581,14 @@ ffs_status ffs_autotune(ffs_problem* p, const char* cache_path, double* best_ms)
     std::memcpy(&bits, &p->weights[i], sizeof bits);
     for (int k = 0; k < 8; k++, bits >>= 8) wh = (wh ^ (bits & 0xff)) * 0x100000001b3ULL;
   }
+  // 1D and 3D keys carry a version: entries of the version before hold depths that runs did not use.
   char key[256];
-  std::snprintf(key, sizeof key, "d%d_r%d_p%d_c%d_a%d_n%lldx%lldx%lld_T%lld_w%016llx_f%d_%s", p->dims, p->radius,
+  std::snprintf(key, sizeof key, "d%d%s_r%d_p%d_c%d_a%d_n%lldx%lldx%lld_T%lld_w%016llx_f%d_%s", p->dims, p->dims == 2 ? "" : "v2", p->radius,
                 p->precision, p->convention, p->algorithm, (long long)p->sizes[0],
                 (long long)(p->dims > 1 ? p->sizes[1] : 1), (long long)(p->dims > 2 ? p->sizes[2] : 1),
                 (long long)p->steps, (unsigned long long)wh, p->flags, arch);
-  // host-only admissibility check of a configuration (the planner's own validation, no device work)
-  auto admissible = [&](int algo, int tile, int fuse, int mapping) {
-    ffs_plan probe;
+  // The planner's choice for a configuration (host only, no device work); false if it refuses it.
+  auto planned = [&](ffs_plan& probe, int algo, int tile, int fuse, int mapping) {
     probe.prob = *p;
     probe.prob.algorithm = algo;
     if (algo == FFS_ALGO_DIRECT) probe.prob.precision = FFS_PREC_FP64;
@@ -1597,6 +1599,10 @@ ffs_status ffs_autotune(ffs_problem* p, const char* cache_path, double* best_ms)
     probe.weights.assign(p->weights, p->weights + ntaps_key);
     probe.prob.weights = probe.weights.data();
     return choose_config(&probe) == FFS_OK;
+  };
+  auto admissible = [&](int algo, int tile, int fuse, int mapping) {
+    ffs_plan probe;
+    return planned(probe, algo, tile, fuse, mapping);
   };
   auto apply = [&](int algo, int tile, int fuse, int mapping) {
     p->algorithm = algo;
@@ -1652,7 +1658,11 @@ ffs_status ffs_autotune(ffs_problem* p, const char* cache_path, double* best_ms)
       const int64_t tmax = p->radius == 0 ? 1 : std::max<int64_t>(1, (tile - vmin) / (2 * p->radius));
       for (int64_t t = 1; t <= std::min(tmax, tcap); t++)
         if (pick(t, tmax))
-          for (int mp : {FFS_MAP_XCD, FFS_MAP_LINEAR}) cands.push_back({FFS_ALGO_FFT, tile, (int)t, mp});
+          for (int mp : {FFS_MAP_XCD, FFS_MAP_LINEAR}) {
+            ffs_plan probe;  // banded products take no mapping: one candidate per depth
+            if (mp == FFS_MAP_XCD && planned(probe, FFS_ALGO_FFT, tile, (int)t, mp) && probe.line) continue;
+            cands.push_back({FFS_ALGO_FFT, tile, (int)t, mp});
+          }
     }
   }
   if (p->algorithm != FFS_ALGO_FFT) {  // direct candidates (FP64), when the radius is offered
@@ -1664,6 +1674,17 @@ ffs_status ffs_autotune(ffs_problem* p, const char* cache_path, double* best_ms)
     const int64_t tmax = ffsk::direct_max_depth(p->dims, p->radius, star_support(&probe));
     for (int64_t t = 1; t <= std::min(tmax, tcap); t++)
       if (pick(t, tmax)) cands.push_back({FFS_ALGO_DIRECT, 0, (int)t, FFS_MAP_AUTO});
+  }
+  // 1D: the depth that the planner takes by itself, which may lie between the ones above or (as fuse = 0) beyond them.
+  for (int algo : {FFS_ALGO_FFT, FFS_ALGO_DIRECT}) {
+    ffs_plan probe;
+    const int tile = algo == FFS_ALGO_FFT ? 240 : 0, mp = algo == FFS_ALGO_FFT ? FFS_MAP_LINEAR : FFS_MAP_AUTO;
+    if (p->dims != 1 || (p->algorithm != FFS_ALGO_AUTO && p->algorithm != algo)) continue;
+    if (!planned(probe, algo, tile, 0, mp) || !probe.line) continue;
+    const int depth = admissible(algo, tile, (int)probe.line_t, mp) ? (int)probe.line_t : 0;
+    bool listed = false;
+    for (const Cand& c : cands) listed = listed || (c.algo == algo && c.fuse == depth);
+    if (!listed) cands.push_back({algo, tile, depth, mp});
   }
   double best = 1e300;
   Cand win{-1, 0, 0, 0};

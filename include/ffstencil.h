@@ -91,7 +91,7 @@ typedef enum ffs_algorithm { FFS_ALGO_FFT = 0, FFS_ALGO_DIRECT = 1, FFS_ALGO_AUT
  *   LINEAR:      hardware dispatch order (consecutive workgroups go to different XCDs);
  *   AUTO:        XCD for the 2D FP64 form on 32-point tiles (measured 4% faster on Box2D25P 8192^2),
  *                LINEAR otherwise (1-3% faster than XCD bands for the mixed 2D forms there).
- * The direct kernels ignore it.  No reference counterpart (the reference launches one warp per tile
+ * The direct kernels and the banded products of 1D runs ignore it.  No reference counterpart (the reference launches one warp per tile
  * pair in grid order). */
 typedef enum ffs_mapping { FFS_MAP_AUTO = 0, FFS_MAP_XCD = 1, FFS_MAP_LINEAR = 2 } ffs_mapping;
 
@@ -113,7 +113,8 @@ typedef struct ffs_problem {
   int32_t convention;    /* ffs_convention */
   int32_t tile;          /* DFT length per axis; 0 = automatic (1D: 240 = 16x15 prime-factor; 3D: 16; 2D: 32
                             for the FP16/BF16 forms, 16 or 32 for FP64 by the depth cost model, 16 for FP32) */
-  int32_t fuse;          /* fused depth t; 0 = automatic */
+  int32_t fuse;          /* fused depth t of a block; 0 = automatic.  When set, 1D and 3D runs launch that depth, and
+                            mixed 2D runs t or 2t (two blocks at once, see ffs_plan_info.launches) */
   int32_t use_graph;     /* 1 = replay the block loop from a hipGraph (chains of more than 4 launches;
                             shorter chains launch directly, which is cheaper), 0 = plain launches */
   int32_t device;        /* HIP device ordinal */
@@ -233,7 +234,7 @@ ffs_status ffs_run_block(ffs_plan* plan, const double* d_in, double* d_out, int3
 
 /* Autotuner: time the admissible (algorithm, tile, fused depth, wave-to-tile mapping) plans of `p` on
  * its device (full T-step runs on a scratch grid of p's sizes) and write the fastest into p->tile,
- * p->fuse, p->mapping and p->algorithm (FFS_ALGO_AUTO searches both algorithms; a DIRECT winner also
+ * p->fuse (0, automatic, where a 1D run is fastest at a depth beyond a block's), p->mapping and p->algorithm (FFS_ALGO_AUTO searches both algorithms; a DIRECT winner also
  * sets p->precision to FFS_PREC_FP64).  With a non-NULL `cache_path`, results are read from / appended to that JSON-lines
  * file keyed by (dims, radius, precision, convention, algorithm, sizes, T), so each configuration is
  * measured once.  best_ms (may be NULL) receives the winner's time per run.  No reference counterpart

@@ -68,3 +68,15 @@ def test_autotune_cache_keyed_by_weights(ffs, oracle, torch_cuda, tmp_path):
         got[shape] = fuse
     assert len(open(cache).readlines()) == 2
     assert got["Box2D25P"] <= 4
+
+
+@pytest.mark.parametrize("algorithm", ["fft", "auto"])
+def test_autotune_1d_depth_beyond_a_block(ffs, torch_cuda, tmp_path, algorithm):
+    # Heat-1D x 240 on a short line: one launch of the banded product at a depth no block has.  The planner's own depth is
+    # among the candidates, so the tuned plan is that or one about as fast.
+    _, r, w, _ = ffs.named_stencil("Heat-1D", seed=4)
+    algo, tile, fuse, mapping, ms = ffs.autotune_full(1, (5000,), w, r, 240, precision="fp64", algorithm=algorithm)
+    with ffs.Plan(1, (5000,), w, r, 240, precision="fp64", tile=tile, fuse=fuse, algorithm=algo, mapping=mapping) as tuned:
+        with ffs.Plan(1, (5000,), w, r, 240, precision="fp64") as own:
+            assert own.info["launches"] == 1
+            assert tuned.info["launches"] <= 2 * own.info["launches"], tuned.info

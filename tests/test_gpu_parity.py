@@ -523,3 +523,26 @@ def test_run_block_where_runs_launch_other_kernels(ffs, oracle, torch_cuda, conv
             ref = oracle.sweep(x, radius, w, info["fuse_tail"] if tail else fuse, convention=0 if convention == "ref" else 1)
             tol = 1e-12 if precision == "fp64" else 1e-6
             assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= tol, (tail, info)
+
+
+@pytest.mark.parametrize("dims,sizes,radius,precision,algorithm,fuses", [
+    (1, (3001,), 1, "fp64", "fft", (1, 7, 50, 100)), (1, (3001,), 2, "bf16", "fft", (1, 9, 50)),
+    (1, (3001,), 1, "fp64", "direct", (1, 7, 60)), (1, (3001,), 3, "fp64", "auto", (2, 9)),
+    (3, (150, 131, 139), 1, "fp64", "fft", (1, 2)), (3, (150, 131, 139), 1, "bf16", "fft", (1, 2, 3)),
+    (3, (150, 131, 139), 1, "fp64", "fft", (4,))])
+def test_forced_depth_is_the_launched_depth(ffs, oracle, torch_cuda, dims, sizes, radius, precision, algorithm, fuses):
+    """A depth that the caller sets is what 1D and 3D runs launch (4 in 3D: beyond the streamed kernel's, on the tiles)."""
+    torch = torch_cuda
+    w = _signed_mean_one(radius, dims, radius)
+    steps = 101 if dims == 1 else 7
+    x = oracle.uniform(5, sizes)
+    d_in = torch.from_numpy(x).cuda()
+    ref = oracle.sweep(x, radius, w, steps)
+    for fuse in fuses:
+        d_out = torch.empty_like(d_in)
+        with ffs.Plan(dims, sizes, w, radius, steps, precision=precision, algorithm=algorithm, fuse=fuse) as plan:
+            plan.run(d_in, d_out)
+            torch.cuda.synchronize()
+            info = plan.info
+        assert info["run_depth"] == fuse and info["launches"] == -(-steps // fuse), (fuse, info)
+        assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= (1e-12 if precision == "fp64" else 1e-6), (fuse, info)
