@@ -3120,6 +3120,7 @@ __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
     } else {
       for (int i = lane; i < win; i += 64) sX[i + (i >> 4)] = a.src[wrap_near(base + i, a.n)];
     }
+    lds_fence();  // the wave reads what its other lanes wrote
     d4 acc[kChains];
 #pragma unroll
     for (int c = 0; c < kChains; c++) acc[c] = d4{0.0, 0.0, 0.0, 0.0};
@@ -3150,6 +3151,7 @@ __global__ __launch_bounds__(256) void k_line_f64(LineArgs a) {
         for (int v = 0; v < 4; v++) y[v] = sX[17 * j + 4 * q + v];
       }
     }
+    lds_fence();  // before the next window overwrites it
     const int64_t p = p0 + 16 * j + 4 * q;
     if (p + 3 < a.n) {
       *reinterpret_cast<d2u*>(a.dst + p) = d2u{y[0], y[1]};
@@ -3239,6 +3241,7 @@ __global__ __launch_bounds__(256) void k_line_bf16(LineArgs a) {
         big[m] = FFS_MFMA_BF16(T[0], xh, big[m]);
       }
     }
+    lds_fence();  // before the next window overwrites it
     const double add = c * a.dc_gain;
 #pragma unroll
     for (int m = 0; m < M; m++) {
