@@ -1033,13 +1033,15 @@ hipError_t dft_tables(const ffs_plan* pl, hipStream_t s);
 hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
   const ffs_problem& p = pl->prob;
   const int K = 2 * p.radius + 1;
+  double big = 0.0;
+  for (double w : pl->weights) big += 4.0 * std::fabs(w);
   if (pl->wide) {
     float* H = reinterpret_cast<float*>(pl->d_wide + ffsk::kOpsWide);
     hipError_t e = ffsk::gen_operands_wide(pl->d_wide, p.precision == FFS_PREC_MIXED_F16, s);
-    if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, pl->norm_wide, s);
+    if (e == hipSuccess) e = ffsk::gen_spectrum_real(H, 64, pl->d_taps, K, p.convention, 2 * pl->t, pl->norm_wide, big, s);
     if (e == hipSuccess && pl->t_wide_tail > 0)
       e = ffsk::gen_spectrum_real(H + ffsk::kSpecWide, 64, pl->d_taps, K, p.convention, pl->t_wide_tail,
-                                  pl->norm_wide_tail, s);
+                                  pl->norm_wide_tail, big, s);
     if (e != hipSuccess) return e;
   }
   if (pl->stream) {
@@ -1068,9 +1070,9 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
   if (pl->direct || (run_only && (pl->wide || pl->stream || pl->line))) return hipSuccess;
   if (!real_tiles(pl)) return dft_tables(pl, s);
   hipError_t e = ffsk::gen_operands_real(pl->d_ops, s);
-  if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, 0, s);
+  if (e == hipSuccess) e = ffsk::gen_spectrum_real(pl->d_H, 32, pl->d_taps, K, p.convention, pl->t, 0, big, s);
   if (e == hipSuccess && pl->t_tail > 0)
-    e = ffsk::gen_spectrum_real(pl->d_H + ffsk::kSpecReal, 32, pl->d_taps, K, p.convention, pl->t_tail, 0, s);
+    e = ffsk::gen_spectrum_real(pl->d_H + ffsk::kSpecReal, 32, pl->d_taps, K, p.convention, pl->t_tail, 0, big, s);
   return e;
 }
 // The DFT tables of the plan's family (complex operands, spectrum of the cyclic DFT, inverse operands).

@@ -123,6 +123,7 @@ hipError_t gen_operands32_f64(double* ops, hipStream_t s);
 // Tables of the real half-sample transforms.  32-point FP64 kernels: kOpsReal operand doubles, and the filter
 // of one depth, 4 doubles per (k0, k1) in kernel order.  64-point mixed kernels: kOpsWide operand words (the
 // BF16 form's size; FP16 uses two thirds), and kSpecWide floats per depth, times 2^filter_exp.
+// big: 4 times the sum of the taps' sizes or more.
 constexpr int kOpsReal = 2 * 4 * kLanes;
 constexpr int kSpecReal = 4 * 16 * 16;
 constexpr int kOpsWide = 4 * 3 * 4 * kLanes;
@@ -131,7 +132,7 @@ constexpr int kWideScaleExp = 9;  // FP16 64-point windows: folded fluctuations 
 hipError_t gen_operands_real(double* ops, hipStream_t s);
 hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s);
 hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
-                             int32_t filter_exp, hipStream_t s);
+                             int32_t filter_exp, double big, hipStream_t s);
 // Inverse operands of an out16 block, output column j <- window column (j + shift) mod 32:
 //   mixed forms: u4 per lane, [arr: R, I, NI][term 0..2][lane] (the kOps32Words entries of block Kb = 0);
 //   FP64: [R][chunk v][arr: Fr, -(Fr + Fi), Fi - Fr][lane] doubles (the kOps32F64 entries of block Kb = 0).

@@ -2576,58 +2576,129 @@ __global__ void k_gen_operands_real(double* t) {
 // factor 2^filter_exp are folded in.
 // Entry order: FP64 32-point (P = 32, doubles), entry v * 64 + lane <-> (q + 4v, j); 64-point (P = 64, floats),
 // entry ((2 b0 + b1) * 4 + v) * 64 + lane <-> (2 (4q + v) + b0, 2j + b1).
-__device__ __forceinline__ void cpow_t(double& kr, double& ki, int64_t t) {
-  double pr = 1.0, pi = 0.0, br = kr, bi = ki;
+// The FP64 filter is formed in pairs of doubles: rounded as it went, a filter's low frequencies erred together (by the power
+// t), and with them every block by the same gain (Star2D9P, 25 blocks of t = 5: 3.3e-14 of the mean; in pairs 1.4e-15, which
+// is the transform matrices' rounding; complex transforms before 1.6e-14).  The 64-point filter is stored in FP32.
+struct Pair {  // h + l, |l| <= ulp(h) / 2; sums by Knuth's two-sum, products by FMA
+  double h, l;
+  __device__ Pair(double x = 0.0) : h(x), l(0.0) {}
+  __device__ Pair(double x, double y) : h(x), l(y) {}
+};
+__device__ __forceinline__ Pair operator+(Pair a, Pair b) {
+#pragma clang fp contract(off)
+  const double s = a.h + b.h, v = s - a.h, e = ((a.h - (s - v)) + (b.h - v)) + (a.l + b.l), h = s + e;
+  return Pair(h, e - (h - s));
+}
+__device__ __forceinline__ Pair operator-(Pair a) { return Pair(-a.h, -a.l); }
+__device__ __forceinline__ Pair operator-(Pair a, Pair b) { return a + -b; }
+__device__ __forceinline__ Pair operator*(Pair a, Pair b) {
+#pragma clang fp contract(off)
+  const double p = a.h * b.h, e = __builtin_fma(a.h, b.h, -p) + (a.h * b.l + a.l * b.h), h = p + e;
+  return Pair(h, e - (h - p));
+}
+__device__ __forceinline__ double to_double(Pair a) { return a.h; }
+__device__ __forceinline__ double to_double(double a) { return a; }
+// Sum of w x.  Pairs: started from `big`, which no product exceeds, so s - acc is exact and the second FMA is what the
+// addition lost.
+template <typename T>
+struct Sum;
+template <>
+struct Sum<double> {
+  double sum = 0.0;
+  __device__ Sum(double) {}
+  __device__ void add(double w, double x) { sum += w * x; }
+  __device__ double value() const { return sum; }
+};
+template <>
+struct Sum<Pair> {
+  double big, acc, low = 0.0;
+  __device__ Sum(double b) : big(b), acc(b) {}
+  __device__ void add(double w, Pair x) {
+#pragma clang fp contract(off)
+    const double s = __builtin_fma(w, x.h, acc);
+    low = __builtin_fma(w, x.l, low + __builtin_fma(w, x.h, -(s - acc)));
+    acc = s;
+  }
+  __device__ Pair value() const { return Pair(acc - big) + Pair(low); }
+};
+
+__constant__ double kCos32[17][2] = {  // cos(pi m / 32), high and low
+    {0x1.0000000000000p+0, 0x0.0p+0}, {0x1.fd88da3d12526p-1, -0x1.87df6378811c7p-55},
+    {0x1.f6297cff75cb0p-1, 0x1.562172a361fd3p-56}, {0x1.e9f4156c62ddap-1, 0x1.760b1e2e3f81ep-55},
+    {0x1.d906bcf328d46p-1, 0x1.457e610231ac2p-56}, {0x1.c38b2f180bdb1p-1, -0x1.6e0b1757c8d07p-56},
+    {0x1.a9b66290ea1a3p-1, 0x1.9f630e8b6dac8p-60}, {0x1.8bc806b151741p-1, -0x1.2c5e12ed1336dp-55},
+    {0x1.6a09e667f3bcdp-1, -0x1.bdd3413b26456p-55}, {0x1.44cf325091dd6p-1, 0x1.8076a2cfdc6b3p-57},
+    {0x1.1c73b39ae68c8p-1, 0x1.b25dd267f6600p-55}, {0x1.e2b5d3806f63bp-2, 0x1.e0d891d3c6841p-58},
+    {0x1.87de2a6aea963p-2, -0x1.72cedd3d5a610p-57}, {0x1.294062ed59f06p-2, -0x1.5d28da2c4612dp-56},
+    {0x1.8f8b83c69a60bp-3, -0x1.26d19b9ff8d82p-57}, {0x1.917a6bc29b42cp-4, -0x1.e2718d26ed688p-60},
+    {0x0.0p+0, 0x0.0p+0}};
+// exp(i pi m / P), 0 <= m < 2 P
+template <int P>
+__device__ __forceinline__ void unit_root(int m, double& c, double& s) {
+  sincospi((double)m / (double)P, &s, &c);
+}
+template <int P>
+__device__ __forceinline__ void unit_root(int m, Pair& c, Pair& s) {
+  static_assert(P == 32, "the table's angles");
+  auto cosine = [](int k) {
+    k &= 63;
+    if (k > 32) k = 64 - k;
+    const int i = k > 16 ? 32 - k : k;
+    const Pair x(kCos32[i][0], kCos32[i][1]);
+    return k > 16 ? -x : x;
+  };
+  c = cosine(m);
+  s = cosine(m - 16);
+}
+
+template <typename T>
+__device__ __forceinline__ void cpow_t(T& kr, T& ki, int64_t t) {
+  T pr = 1.0, pi = 0.0, br = kr, bi = ki;
   for (int64_t n = t; n > 0; n >>= 1) {
     if (n & 1) {
-      const double tr = pr * br - pi * bi;
+      const T tr = pr * br - pi * bi;
       pi = pr * bi + pi * br;
       pr = tr;
     }
-    const double tr = br * br - bi * bi;
-    bi = 2.0 * br * bi;
+    const T tr = br * br - bi * bi;
+    bi = T(2.0) * (br * bi);
     br = tr;
   }
   kr = pr;
   ki = pi;
 }
-__global__ void k_gen_spectrum_real(void* H, int32_t P, const double* taps, int32_t K, int32_t convention,
-                                    int64_t t, int32_t filter_exp) {
-  __shared__ double2 root[128];  // exp(i pi m / P), m < 2P <= 128
-  for (int m = threadIdx.x; m < 2 * P; m += blockDim.x) {
-    double s, c;
-    sincospi((double)m / (double)P, &s, &c);
-    root[m] = make_double2(c, s);
-  }
+template <int P, typename T, typename Out>
+__global__ void k_gen_spectrum_real(Out* H, const double* taps, int32_t K, int32_t convention, int64_t t,
+                                    int32_t filter_exp, double big) {
+  __shared__ double store[2 * P * 2 * sizeof(T) / sizeof(double)];
+  T* re = reinterpret_cast<T*>(store);
+  T* im = re + 2 * P;
+  for (int m = threadIdx.x; m < 2 * P; m += blockDim.x) unit_root<P>(m, re[m], im[m]);
   __syncthreads();
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= P * P / 4) return;
   const int lane = e % kLanes, v = (e / kLanes) % 4, b = e / (4 * kLanes);
   const int k0 = P == 32 ? (lane >> 4) + 4 * v : 2 * (4 * (lane >> 4) + v) + (b >> 1);
   const int k1 = P == 32 ? lane & 15 : 2 * (lane & 15) + (b & 1);
-  double L1r = 0.0, L1i = 0.0, L2r = 0.0, L2i = 0.0;
+  Sum<T> S1r(big), S1i(big), S2r(big), S2i(big);
   for (int a0 = 0; a0 < K; a0++)
     for (int a1 = 0; a1 < K; a1++) {
       const double w = taps[a0 * K + a1];
       if (w == 0.0) continue;
       const int e0 = convention == 0 ? K - 1 - a0 : a0, e1 = convention == 0 ? K - 1 - a1 : a1;
       const int x0 = (2 * k0 + 1) * e0, x1 = (2 * k1 + 1) * e1;
-      const double2 u1 = root[(x0 + x1) & (2 * P - 1)], u2 = root[(x0 - x1) & (2 * P - 1)];
-      L1r += w * u1.x;
-      L1i += w * u1.y;
-      L2r += w * u2.x;
-      L2i += w * u2.y;
+      const int m1 = (x0 + x1) & (2 * P - 1), m2 = (x0 - x1) & (2 * P - 1);
+      S1r.add(w, re[m1]);
+      S1i.add(w, im[m1]);
+      S2r.add(w, re[m2]);
+      S2i.add(w, im[m2]);
     }
+  T L1r = S1r.value(), L1i = S1i.value(), L2r = S2r.value(), L2i = S2i.value();
   cpow_t(L1r, L1i, t);
   cpow_t(L2r, L2i, t);
   const double norm = ldexp(0.5 * 4.0 / ((double)P * (double)P), filter_exp);
-  const double h[4] = {(L1r + L2r) * norm, (L2r - L1r) * norm, (L1i + L2i) * norm, (L1i - L2i) * norm};
-  for (int i = 0; i < 4; i++) {
-    if (P == 32)
-      static_cast<double*>(H)[4 * e + i] = h[i];
-    else
-      static_cast<float*>(H)[4 * e + i] = (float)h[i];
-  }
+  const double h[4] = {to_double(L1r + L2r), to_double(L2r - L1r), to_double(L1i + L2i), to_double(L1i - L2i)};
+  for (int i = 0; i < 4; i++) H[4 * e + i] = (Out)(h[i] * norm);
 }
 
 // Operands of the 64-point windows: [cos, sin][block b][term][lane] of 4 words; element e of lane (j + 16q) is
@@ -2674,9 +2745,14 @@ hipError_t gen_operands_wide(uint32_t* ops, bool f16, hipStream_t s) {
 }
 
 hipError_t gen_spectrum_real(void* H, int32_t P, const double* d_taps, int32_t K, int32_t convention, int64_t t,
-                             int32_t filter_exp, hipStream_t s) {
-  hipLaunchKernelGGL(k_gen_spectrum_real, dim3((unsigned)(P * P / 4 / 64)), dim3(64), 0, s, H, P, d_taps, K, convention, t,
-                     filter_exp);
+                             int32_t filter_exp, double big, hipStream_t s) {
+  const dim3 g((unsigned)(P * P / 4 / 64)), b(64);
+  if (P == 32)
+    hipLaunchKernelGGL((k_gen_spectrum_real<32, Pair, double>), g, b, 0, s, static_cast<double*>(H), d_taps, K, convention, t,
+                       filter_exp, big);
+  else
+    hipLaunchKernelGGL((k_gen_spectrum_real<64, double, float>), g, b, 0, s, static_cast<float*>(H), d_taps, K, convention, t,
+                       filter_exp, big);
   return hipGetLastError();
 }
 
