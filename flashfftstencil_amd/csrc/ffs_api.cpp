@@ -1050,10 +1050,10 @@ hipError_t plan_tables(const ffs_plan* pl, hipStream_t s, bool run_only) {
     char* H = base + stream_ops_bytes(pl);
     hipError_t e = mixed ? ffsk::gen_operands_fold(pl->d_wide, s) : ffsk::gen_operands_real(reinterpret_cast<double*>(base), s);
     if (e == hipSuccess)
-      e = ffsk::gen_stream3d(H, mixed, pl->stream_E, pl->d_taps, K, p.convention, (int32_t)pl->stream_t, s);
+      e = ffsk::gen_stream3d(H, mixed, pl->stream_E, pl->d_taps, K, p.convention, (int32_t)pl->stream_t, big, s);
     if (e == hipSuccess && pl->stream_tail > 0)
       e = ffsk::gen_stream3d(H + stream_spec_bytes(pl), mixed, pl->stream_E, pl->d_taps, K, p.convention,
-                             (int32_t)pl->stream_tail, s);
+                             (int32_t)pl->stream_tail, big, s);
     if (e != hipSuccess) return e;
   }
   if (pl->line) {

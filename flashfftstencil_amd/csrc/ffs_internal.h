@@ -190,7 +190,7 @@ struct Stream3Args {
 };
 constexpr int kOpsFold = 6 * kLanes * 4;
 hipError_t gen_stream3d(void* H, bool mixed, int32_t E, const double* d_taps, int32_t K, int32_t convention, int32_t t,
-                        hipStream_t s);
+                        double big, hipStream_t s);  // big: as for gen_spectrum_real
 hipError_t gen_operands_fold(uint32_t* ops, hipStream_t s);
 hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, hipStream_t s);
 // Two fused blocks of a 32-point mixed plan on 64-point windows (FP16, BF16), for one grid or a batch's items.

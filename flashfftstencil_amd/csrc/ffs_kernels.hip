@@ -3044,58 +3044,57 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
 // axis-0 tap e <= 2 r t (zero above), as k_gen_spectrum_real forms them from the coefficients of z^e of
 // (sum_e0 z^e0 sum g[e0][e1][e2] exp(i (w1 e1 + w2 e2)))^t and its mirror (w2 -> -w2).  FP64 order (row q + 4v) or
 // FP32 order (row 4q + v).  Then the operands: 16 x 16 cosine and sine matrices, FP64 chunks or BF16 pairings.
+// FP64 in pairs of doubles, as the 2D filter (Heat-3D over 26 steps: gain of the mean off by 1.9e-15 in plain doubles).
 constexpr int kStreamMaxE = 7;
-__global__ void k_gen_stream3d(void* H, int32_t mixed, int32_t E, const double* taps, int32_t K, int32_t convention,
-                               int32_t t) {
+template <typename T, typename Out>
+__global__ void k_gen_stream3d(Out* H, int32_t E, const double* taps, int32_t K, int32_t convention, int32_t t, double big) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= 4 * kLanes) return;
+  constexpr bool mixed = sizeof(Out) == sizeof(float);
   const int lane = x % kLanes, v = x / kLanes;
   const int k1 = mixed ? 4 * (lane >> 4) + v : (lane >> 4) + 4 * v, k2 = lane & 15;
-  double L[2][2][kStreamMaxE];  // [w2, -w2][re, im][tap]
+  T L[2][2][kStreamMaxE];  // [w2, -w2][re, im][tap]
   for (int sgn = 0; sgn < 2; sgn++) {
-    double one[2][kStreamMaxE] = {}, pw[2][kStreamMaxE] = {};
-    for (int a0 = 0; a0 < K; a0++)
+    T one[2][kStreamMaxE] = {};
+    T (&pw)[2][kStreamMaxE] = L[sgn];
+    for (int a0 = 0; a0 < K; a0++) {
+      Sum<T> re(big), im(big);
       for (int a1 = 0; a1 < K; a1++)
         for (int a2 = 0; a2 < K; a2++) {
           const double w = taps[(a0 * K + a1) * K + a2];
           if (w == 0.0) continue;
-          const int e0 = convention == 0 ? K - 1 - a0 : a0, e1 = convention == 0 ? K - 1 - a1 : a1;
-          const int e2 = convention == 0 ? K - 1 - a2 : a2;
-          int m = (2 * k1 + 1) * e1 + (sgn ? -1 : 1) * (2 * k2 + 1) * e2;
-          m = ((m % 64) + 64) % 64;
-          double s, c;
-          sincospi((double)m / 32.0, &s, &c);
-          one[0][e0] += w * c;
-          one[1][e0] += w * s;
+          const int e1 = convention == 0 ? K - 1 - a1 : a1, e2 = convention == 0 ? K - 1 - a2 : a2;
+          T c, s;
+          unit_root<32>(((2 * k1 + 1) * e1 + (sgn ? -1 : 1) * (2 * k2 + 1) * e2) & 63, c, s);
+          re.add(w, c);
+          im.add(w, s);
         }
-    pw[0][0] = 1.0;
-    for (int n = 0; n < t; n++) {  // pw *= one (degree n (K - 1) before)
-      double nr[kStreamMaxE] = {}, ni[kStreamMaxE] = {};
+      const int e0 = convention == 0 ? K - 1 - a0 : a0;
+      one[0][e0] = re.value();
+      one[1][e0] = im.value();
+    }
+    for (int i = 0; i < kStreamMaxE; i++) {
+      pw[0][i] = one[0][i];
+      pw[1][i] = one[1][i];
+    }
+    for (int n = 1; n < t; n++) {  // pw *= one (degree n (K - 1) before)
+      T nr[kStreamMaxE] = {}, ni[kStreamMaxE] = {};
       for (int i = 0; i <= n * (K - 1); i++)
         for (int e = 0; e < K && i + e < kStreamMaxE; e++) {
-          nr[i + e] += pw[0][i] * one[0][e] - pw[1][i] * one[1][e];
-          ni[i + e] += pw[0][i] * one[1][e] + pw[1][i] * one[0][e];
+          nr[i + e] = nr[i + e] + (pw[0][i] * one[0][e] - pw[1][i] * one[1][e]);
+          ni[i + e] = ni[i + e] + (pw[0][i] * one[1][e] + pw[1][i] * one[0][e]);
         }
       for (int i = 0; i < kStreamMaxE; i++) {
         pw[0][i] = nr[i];
         pw[1][i] = ni[i];
       }
     }
-    for (int i = 0; i < kStreamMaxE; i++) {
-      L[sgn][0][i] = pw[0][i];
-      L[sgn][1][i] = pw[1][i];
-    }
   }
   const double norm = 0.5 / 256.0;
   for (int e = 0; e < E; e++) {
-    const double h[4] = {(L[0][0][e] + L[1][0][e]) * norm, (L[1][0][e] - L[0][0][e]) * norm,
-                         (L[0][1][e] + L[1][1][e]) * norm, (L[0][1][e] - L[1][1][e]) * norm};
-    for (int i = 0; i < 4; i++) {
-      if (mixed)
-        static_cast<float*>(H)[(e * 4 * kLanes + x) * 4 + i] = (float)h[i];
-      else
-        static_cast<double*>(H)[(e * 4 * kLanes + x) * 4 + i] = h[i];
-    }
+    const double h[4] = {to_double(L[0][0][e] + L[1][0][e]), to_double(L[1][0][e] - L[0][0][e]),
+                         to_double(L[0][1][e] + L[1][1][e]), to_double(L[0][1][e] - L[1][1][e])};
+    for (int i = 0; i < 4; i++) H[(e * 4 * kLanes + x) * 4 + i] = (Out)(h[i] * norm);
   }
 }
 
@@ -3122,8 +3121,13 @@ __global__ void k_gen_operands_fold(uint32_t* t) {
 }
 
 hipError_t gen_stream3d(void* H, bool mixed, int32_t E, const double* d_taps, int32_t K, int32_t convention, int32_t t,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_gen_stream3d, dim3(4), dim3(64), 0, s, H, (int32_t)mixed, E, d_taps, K, convention, t);
+                        double big, hipStream_t s) {
+  if (mixed)
+    hipLaunchKernelGGL((k_gen_stream3d<double, float>), dim3(4), dim3(64), 0, s, static_cast<float*>(H), E, d_taps, K, convention,
+                       t, big);
+  else
+    hipLaunchKernelGGL((k_gen_stream3d<Pair, double>), dim3(4), dim3(64), 0, s, static_cast<double*>(H), E, d_taps, K, convention,
+                       t, big);
   return hipGetLastError();
 }
 hipError_t gen_operands_fold(uint32_t* ops, hipStream_t s) {

@@ -546,3 +546,22 @@ def test_forced_depth_is_the_launched_depth(ffs, oracle, torch_cuda, dims, sizes
             info = plan.info
         assert info["run_depth"] == fuse and info["launches"] == -(-steps // fuse), (fuse, info)
         assert oracle.errors(d_out.cpu().numpy(), ref)[1] <= (1e-12 if precision == "fp64" else 1e-6), (fuse, info)
+
+
+@pytest.mark.parametrize("shape,steps", [("Heat-3D", 26), ("Box3D27P", 31)])
+def test_3d_streamed_fp64_gain(ffs, torch_cuda, shape, steps):
+    """The mean of the grid is multiplied by (sum w)^T.  Roundings of single outputs average out over 3.4 million points; what
+    is left is the gain error that every launch shares, from the rounding of the transform matrices and the filters: below half
+    an ulp a launch."""
+    torch = torch_cuda
+    _, r, w, _ = ffs.named_stencil(shape, seed=0x5EED0002)
+    x = torch.rand((140, 150, 160), dtype=torch.float64, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    y = torch.empty_like(x)
+    with ffs.Plan(3, x.shape, w, r, steps) as plan:
+        plan.run(x, y)
+        torch.cuda.synchronize()
+        info = plan.info
+    assert info["run_kernel"] == ffs.RUN_KERNELS["stream"]
+    want = x.cpu().numpy().astype(np.longdouble).mean() * np.asarray(w, dtype=np.longdouble).sum() ** steps
+    got = y.cpu().numpy().astype(np.longdouble).mean()
+    assert abs(got / want - 1) <= 2 ** -53 * info["launches"], (float(got / want - 1), info)
