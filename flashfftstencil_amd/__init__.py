@@ -273,7 +273,8 @@ class Plan:
         return inf.as_dict()
 
     def read_table(self, which: int) -> bytes:
-        """Raw bytes of one of the plan's device tables (0 ops, 1 mixed ops, 2 spectrum, 3 out16 inverse)."""
+        """Raw bytes of one of the plan's device tables (0 ops, 1 mixed ops, 2 spectrum, 3 out16 inverse,
+        4 operands and 5 filters of the kernel that whole runs launch)."""
         lib = load_library()
         n = ctypes.c_int64()
         _check(lib.ffs_plan_read_table(self._h, which, None, 0, ctypes.byref(n)))

@@ -1379,13 +1379,35 @@ ffs_status ffs_plan_get_info(const ffs_plan* pl, ffs_plan_info* info) {
 ffs_status ffs_plan_read_table(const ffs_plan* pl, int32_t which, void* host_out, int64_t capacity,
                                int64_t* bytes) {
   if (!pl) return fail(FFS_ERR_INVALID_ARG, "plan is NULL");
-  if (pl->direct) return fail(FFS_ERR_UNSUPPORTED, "the direct algorithm has no transform tables");
+  const bool run_table = which == FFS_TABLE_RUN_OPS || which == FFS_TABLE_RUN_FILTER;
+  if (pl->direct && !(run_table && pl->line))
+    return fail(FFS_ERR_UNSUPPORTED, "the direct algorithm has no transform tables");
   const TableSizes ts = dft_table_sizes(pl);
   const void* src = nullptr;
   size_t n = 0;
   // Real half-sample plans keep other tables: theirs is generated into temporary memory below.
-  const bool own = !real_tiles(pl);
+  const bool own = !real_tiles(pl) || run_table;
+  const bool ops = which == FFS_TABLE_RUN_OPS;
+  if (run_table && pl->line) {
+    const char* taps = reinterpret_cast<const char*>(pl->d_wide);
+    const size_t per = ops ? line_ops_bytes(pl) : sizeof(double) * ffsk::kLineMaxTaps;
+    src = ops ? taps + 2 * sizeof(double) * ffsk::kLineMaxTaps : taps;
+    n = per * (pl->line_tail > 0 ? 2 : 1);
+  } else if (run_table && pl->stream) {
+    const char* base = reinterpret_cast<const char*>(pl->d_wide);
+    src = ops ? base : base + stream_ops_bytes(pl);
+    n = ops ? stream_ops_bytes(pl) : stream_spec_bytes(pl) * (pl->stream_tail > 0 ? 2 : 1);
+  } else if (run_table && pl->wide) {
+    src = ops ? pl->d_wide : pl->d_wide + ffsk::kOpsWide;
+    n = ops ? sizeof(uint32_t) * (size_t)(pl->prob.precision == FFS_PREC_MIXED_F16 ? ffsk::kOpsWide / 3 * 2 : ffsk::kOpsWide)
+            : sizeof(float) * ffsk::kSpecWide * (pl->t_wide_tail > 0 ? 2 : 1);
+  } else if (run_table && real_tiles(pl)) {
+    src = ops ? pl->d_ops : pl->d_H;
+    n = sizeof(double) * (ops ? (size_t)ffsk::kOpsReal : (size_t)ffsk::kSpecReal * (pl->t_tail > 0 ? 2 : 1));
+  }
   switch (which) {
+    case FFS_TABLE_RUN_OPS:
+    case FFS_TABLE_RUN_FILTER: break;
     case FFS_TABLE_OPS: src = pl->d_ops; n = ts.ops; break;
     case FFS_TABLE_OPS_MIXED: src = pl->d_opsm; n = ts.opsm; break;
     case FFS_TABLE_SPECTRUM: src = pl->d_H; n = ts.H; break;

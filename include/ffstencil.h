@@ -191,14 +191,20 @@ ffs_status ffs_plan_get_info(const ffs_plan* plan, ffs_plan_info* info);
  *   OPS_MIXED:  split operands of the mixed forms (BF16/FP16 words, FP32 chunks)
  *   SPECTRUM:   [main | tail] x [re plane | im plane] of K^t / prod(P), in the tile family's order
  *   INVERSE16:  out16 inverse operands of the main and the tail depth
- * The 32-point FP64 kernels run real half-sample transforms on tables of their own; for those plans the DFT
- * tables above are generated at the call.
+ *   RUN_OPS:    operands of the kernel that a whole run launches, where it is not the block kernel, and of the 32-point FP64
+ *               kernels: cosine and sine matrices of the real half-sample transforms (FP64 doubles or split words),
+ *               BF16 line: split Toeplitz operands of the main and the tail depth
+ *   RUN_FILTER: their filters (lines: the taps of the t-fold stencil), main depth, then the tail's where there is one
+ * The 32-point FP64 kernels read RUN_OPS and RUN_FILTER only; the complex DFT tables above are generated at the call for
+ * those plans (what a cyclic transform of the same window would use).
  * No reference counterpart (the reference's tables live in __constant__ memory, src/2D/create_fft_pfa_plan.cu:25-107). */
 typedef enum ffs_table {
   FFS_TABLE_OPS = 0,
   FFS_TABLE_OPS_MIXED = 1,
   FFS_TABLE_SPECTRUM = 2,
-  FFS_TABLE_INVERSE16 = 3
+  FFS_TABLE_INVERSE16 = 3,
+  FFS_TABLE_RUN_OPS = 4,
+  FFS_TABLE_RUN_FILTER = 5
 } ffs_table;
 ffs_status ffs_plan_read_table(const ffs_plan* plan, int32_t which, void* host_out, int64_t capacity,
                                int64_t* bytes);

@@ -75,7 +75,8 @@ def test_dft_operands_1d_prime_factor(ffs, torch_cuda):
 
 
 def test_dft_operands_32_fp64(ffs, torch_cuda):
-    # [R][chunk v][column block Kb][arr][lane], lane (n + 16k) = entry (16 R + 4 v + k, 16 Kb + n)
+    # What ffs_plan_read_table answers for a plan of 32-point FP64 tiles; its kernels read the real half-sample tables
+    # (test_real_tables_32_fp64).  [R][chunk v][column block Kb][arr][lane], lane (n + 16k) = entry (16 R + 4 v + k, 16 Kb + n)
     _, r, w, _ = ffs.named_stencil("Box2D25P", seed=2)
     plan = ffs.Plan(2, (256, 256), w, r, 8, precision="fp64", tile=32)
     assert plan.info["tile"][0] == 32
@@ -254,3 +255,198 @@ def test_read_table_errors(ffs, torch_cuda):
     with pytest.raises(ffs.FFSError, match="UNSUPPORTED"):
         direct.read_table(0)
     direct.close()
+
+
+# ---- tables of the kernels that runs launch ----
+LD = np.longdouble
+PI = 4 * np.arctan(LD(1))
+
+
+def trig(n, P):
+    """cos and sin of pi (2a + 1)(2b + 1) / (2 P), a, b < n, in extended precision (exact angle reduction)."""
+    k = 2 * np.arange(n) + 1
+    th = PI * (np.outer(k, k) % (4 * P)).astype(LD) / (2 * P)
+    return np.cos(th), np.sin(th)
+
+
+def real_filter(L1, L2, P):
+    """(alpha, beta, gamma, delta) of the window's filter from L(w0, w1) and L(w0, -w1), with the transforms' 4 / P^2."""
+    s = LD(2) / (P * P)
+    return np.stack([(L1.real + L2.real) * s, (L2.real - L1.real) * s, (L1.imag + L2.imag) * s, (L1.imag - L2.imag) * s], -1)
+
+
+def half_sample_gain(w, K, convention, k0, k1, P, t):
+    """(sum g[e] exp(i (w0 e0 + w1 e1)))^t and the same at -w1, w = pi (2k + 1) / P, correlation taps g."""
+    g = np.asarray(w, dtype=LD).reshape(K, K)
+    if convention == "ref":
+        g = g[::-1, ::-1]
+    e = np.arange(K)
+    out = []
+    for sign in (1, -1):
+        L = np.zeros(k0.shape, dtype=np.clongdouble)
+        for a in range(K):
+            for b in range(K):
+                m = ((2 * k0 + 1) * e[a] + sign * (2 * k1 + 1) * e[b]) % (2 * P)
+                th = PI * m.astype(LD) / P
+                L = L + g[a, b] * (np.cos(th) + 1j * np.sin(th))
+        p = np.ones_like(L)
+        for _ in range(t):
+            p = p * L
+        out.append(p)
+    return out
+
+
+def halves(words, f16):
+    """The two 16-bit values of each 32-bit word, low half first, as numbers."""
+    w = np.stack([words & 0xFFFF, words >> 16], -1).astype(np.uint32)
+    return w.astype(np.uint16).view(np.float16).astype(LD) if f16 else (w << 16).view(np.float32).astype(LD)
+
+
+LANES = np.arange(64)
+Q, J = LANES // 16, LANES % 16
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("radius,fuse,tail", [(2, 4, 1), (1, 8, 5), (7, 1, 0)])
+def test_real_tables_32_fp64(ffs, torch_cuda, convention, radius, fuse, tail):
+    rng = np.random.default_rng(radius)
+    K = 2 * radius + 1
+    w = rng.standard_normal(K * K)
+    w /= np.abs(w).sum()
+    with ffs.Plan(2, (200, 200), w, radius, 2 * fuse + tail, fuse=fuse, tile=32, convention=convention) as plan:
+        ops, filt = table(plan, 4, np.float64).reshape(2, 4, 64), table(plan, 5, np.float64)
+    for got, want in zip(ops, trig(16, 32)):
+        for v in range(4):  # lane (j + 16 k): entry (4 v + k, j)
+            assert np.abs(got[v] - want[4 * v + Q, J]).max() <= 2.0 ** -53
+    depths = [fuse] + ([tail] if tail else [])
+    assert filt.size == 1024 * len(depths)
+    for got, t in zip(filt.reshape(-1, 4, 64, 4), depths):
+        for v in range(4):  # entry v * 64 + lane: (k0, k1) = (q + 4 v, j)
+            want = real_filter(*half_sample_gain(w, K, convention, Q + 4 * v, J, 32, t), 32)
+            assert np.abs(got[v] - want).max() <= 2.0 ** -53 * np.abs(want).max()  # |entries| <= 2^-8 or so, rounded once
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("form", ["f16", "bf16"])
+@pytest.mark.parametrize("radius,fuse,tail,gain", [(2, 4, 3, 1.0), (1, 8, 1, 0.25), (3, 3, 0, 1.7), (15, 1, 1, 0.5)])
+def test_wide_tables(ffs, torch_cuda, convention, form, radius, fuse, tail, gain):
+    rng = np.random.default_rng(radius)
+    K = 2 * radius + 1
+    w = rng.standard_normal(K * K)
+    L = half_sample_gain(w, K, convention, *np.meshgrid(np.arange(32), np.arange(32), indexing="ij"), 64, 1)
+    w *= gain / float(max(np.abs(x).max() for x in L))
+    steps = 4 * fuse + tail
+    with ffs.Plan(2, (100, 120), w, radius, steps, fuse=fuse, precision=form, convention=convention) as plan:
+        assert plan.info["run_kernel"] == ffs.RUN_KERNELS["wide"]
+        words, filt = table(plan, 4, np.uint32), table(plan, 5, np.float32).astype(LD)
+    nt = 2 if form == "f16" else 3
+    terms = halves(words.reshape(2, 2, nt, 64, 4), form == "f16").reshape(2, 2, nt, 64, 8).sum(axis=2)
+    for got, want in zip(terms, trig(32, 64)):
+        for b in range(2):
+            for e in range(8):  # element e of lane (j + 16 q): entry (2 (4q + (e & 3)) + (e >> 2), 2j + b)
+                err = np.abs(got[b, :, e] - want[2 * (4 * Q + (e & 3)) + (e >> 2), 2 * J + b]).max()
+                assert err <= (2.0 ** -22 if form == "f16" else 2.0 ** -24)
+    depths = [2 * fuse] + ([tail] if tail else [])
+    assert filt.size == 4096 * len(depths)
+    for got, t in zip(filt.reshape(-1, 4, 4, 64, 4), depths):
+        scale = 1.0
+        if form == "f16":  # normalised: |K|^t times a power of two in (1/2, 1] at its largest over the window's frequencies
+            scale = 2.0 ** -np.ceil(t * np.log2(gain) - 1e-9)
+            assert 0.5 < gain ** t * scale <= 1.0 + 1e-6
+        for b in range(4):
+            for v in range(4):  # entry (b * 4 + v) * 64 + lane: (2 (4q + v) + b0, 2j + b1)
+                want = scale * real_filter(*half_sample_gain(w, K, convention, 2 * (4 * Q + v) + (b >> 1), 2 * J + (b & 1), 64, t), 64)
+                assert np.abs(got[b, v] - want).max() <= 2.0 ** -23 * gain ** t * scale / 1024
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("form,radius,sizes,steps", [("fp64", 1, (150, 131, 139), 7), ("bf16", 1, (150, 131, 139), 7),
+                                                     ("fp64", 2, (121, 113, 140), 3), ("bf16", 3, (90, 131, 157), 2)])
+def test_stream_tables(ffs, torch_cuda, convention, form, radius, sizes, steps):
+    K = 2 * radius + 1
+    rng = np.random.default_rng(radius)
+    w = rng.random(K ** 3)
+    w /= w.sum()
+    with ffs.Plan(3, sizes, w, radius, steps, precision=form, convention=convention) as plan:
+        info = plan.info
+        assert info["run_kernel"] == ffs.RUN_KERNELS["stream"]
+        raw, filt = plan.read_table(4), table(plan, 5, np.float64 if form == "fp64" else np.float32).astype(LD)
+    if form == "fp64":
+        ops = np.frombuffer(raw, np.float64).reshape(2, 4, 64)
+        for got, want in zip(ops, trig(16, 32)):
+            for v in range(4):
+                assert np.abs(got[v] - want[4 * v + Q, J]).max() <= 2.0 ** -53
+    else:  # pairings (h|h), (m|m), (l|h): elements 0..3 of the three hold the terms, 4..7 their partners
+        ops = halves(np.frombuffer(raw, np.uint32).reshape(2, 3, 64, 4), False).reshape(2, 3, 64, 8)
+        for got, want in zip(ops, trig(16, 32)):
+            for e in range(4):
+                assert np.abs(got[:, :, e].sum(axis=0) - want[4 * Q + e, J]).max() <= 2.0 ** -24
+                assert np.array_equal(got[:, :, e + 4], got[[0, 1, 0], :, e])
+    depths = [info["run_depth"]] + ([steps % info["run_depth"]] if steps % info["run_depth"] else [])
+    E = 2 * radius * info["run_depth"] + 1
+    g = np.asarray(w, dtype=LD).reshape(K, K, K)
+    if convention == "ref":
+        g = g[::-1, ::-1, ::-1]
+    for got, t in zip(filt.reshape(len(depths), E, 4, 64, 4), depths):
+        for v in range(4):
+            k1 = 4 * Q + v if form == "bf16" else Q + 4 * v
+            poly = [np.zeros((E, 64), dtype=np.clongdouble) for _ in range(2)]
+            for p in poly:
+                p[0] = 1
+            one = [np.zeros((K, 64), dtype=np.clongdouble) for _ in range(2)]
+            for s, sign in enumerate((1, -1)):
+                for a in range(K):
+                    for b in range(K):
+                        for c in range(K):
+                            th = PI * (((2 * k1 + 1) * b + sign * (2 * J + 1) * c) % 64).astype(LD) / 32
+                            one[s][a] += g[a, b, c] * (np.cos(th) + 1j * np.sin(th))
+                for _ in range(t):
+                    nxt = np.zeros_like(poly[s])
+                    for i in range(E):
+                        for a in range(K):
+                            if i + a < E:
+                                nxt[i + a] += poly[s][i] * one[s][a]
+                    poly[s] = nxt
+            for e in range(E):
+                want = real_filter(poly[0][e], poly[1][e], 32)
+                assert np.abs(got[e, v] - want).max() <= (2.0 ** -52 if form == "fp64" else 2.0 ** -24) * np.abs(want).max() + 1e-300
+
+
+@pytest.mark.parametrize("convention", ["ref", "centred"])
+@pytest.mark.parametrize("form,algorithm,radius,n,steps", [("fp64", "fft", 3, 900, 101), ("fp64", "direct", 1, 5000, 248),
+                                                           ("bf16", "fft", 3, 900, 101), ("bf16", "fft", 60, 2000, 9)])
+def test_line_tables(ffs, torch_cuda, convention, form, algorithm, radius, n, steps):
+    K = 2 * radius + 1
+    rng = np.random.default_rng(radius)
+    w = rng.standard_normal(K)
+    w /= np.abs(w).sum()
+    with ffs.Plan(1, (n,), w, radius, steps, precision=form, algorithm=algorithm, convention=convention) as plan:
+        info = plan.info
+        assert info["run_kernel"] == ffs.RUN_KERNELS["line"]
+        taps = table(plan, 5, np.float64).reshape(-1, 512)
+        words = table(plan, 4, np.uint32) if form == "bf16" else None
+    depths = [info["run_depth"]] + ([steps % info["run_depth"]] if steps % info["run_depth"] else [])
+    assert len(taps) == len(depths)
+    for d, (got, t) in enumerate(zip(taps, depths)):
+        one = np.asarray(w, dtype=LD)[::-1 if convention == "ref" else 1]
+        powers = [np.array([1], dtype=LD)]
+        for _ in range(t):
+            powers.append(np.convolve(powers[-1], one))
+        g, h = powers[t], np.abs(powers[t // 2])
+        # rounded once, and for more than 128 taps the two halves of the last square (and the odd step's factor) before it
+        halves_of = np.convolve(h, h) if t % 2 == 0 else np.convolve(np.convolve(h, h), np.abs(one))
+        bound = 2.0 ** -53 * (np.abs(g) + (3 * halves_of if g.size > 128 else 0)).max()
+        assert np.abs(got[:g.size] - g).max() <= bound * (1 + 1e-9) and not got[g.size:].any()
+        if words is None:
+            continue
+        T = halves(words.reshape(len(depths), -1, 3, 64, 4)[d], False).reshape(-1, 3, 64, 8).sum(axis=1)
+        pad = np.concatenate([np.zeros(16, LD), g, np.zeros(32 * len(T) + 16, LD)])
+        for b in range(len(T)):
+            for e in range(8):  # element e of lane (i + 16 q): T[i][32 b + 8 q + e] = g[32 b + 8 q + e - i]
+                k = 32 * b + 8 * Q + e - J
+                want = np.where(k >= 0, pad[np.maximum(k, 0) + 16], 0)
+                assert np.abs(T[b, :, e] - want).max() <= 2.0 ** -24 * np.abs(g).max()
+    if form == "fp64":
+        with ffs.Plan(1, (n,), w, radius, steps, precision=form, algorithm=algorithm, convention=convention) as plan:
+            with pytest.raises(ffs.FFSError, match="UNSUPPORTED"):
+                plan.read_table(4)  # the FP64 product reads the taps themselves
