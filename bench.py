@@ -14,24 +14,24 @@ Workloads (seed 0x5EED0000 + index, SplitMix64; weights uniform[0,1) normalised 
      planner's depths are timed beside it)
 
 `value` is C3's mixed FP16 form (the metric's headline comparison); every workload's record sits under
-`configs` with its forms' GStencils/s, the dominant kernel's roofline, max-rel / rel-L2 against the FP64
+`configs` with its forms' GStencils/s, the run's roofline, max-rel / rel-L2 against the FP64
 form (full T) and against the FP64 direct sweep (the oracle, on a bounded sample), and the oracle's CPU
 time on the host's cores.
 
-Roofline of one fused block (ffs_run_block: one launch of the plan's block kernel), algorithmic counts only:
-  flops  = the real GEMMs the kernel's formulation needs, each counted once (FP64 2D: the folded real
-           transforms; elsewhere the complex products, Gauss form in FP64; the inverse stages cut to the kept
-           output block; never the split products of the mixed forms: executed MFMA flops / products
-           per real GEMM, 1 FP64/FP32 (2 for the compensated FP32 form in 3D), 3 FP16, 6 BF16),
+Roofline of one launch of the timed run (run time / launches, whatever kernel it launches), algorithmic counts only:
+  flops  = the real GEMMs the kernel's formulation needs, each counted once (FP64 2D, 64-point windows and the
+           streamed planes: the folded real transforms; 1D: the banded product; elsewhere the complex products,
+           Gauss form in FP64; the inverse stages cut to the kept output blocks; never the split products of the
+           mixed forms: executed MFMA flops / products per real GEMM, 1 FP64/FP32 (2 for the compensated FP32
+           form in 3D), 3 FP16, 6 BF16; never the planes that fill the stream's segments),
            against the matrix peak of the form's arithmetic (FP64 78.6 TF, FP32 157.3 TF, FP16/BF16
-           2.5 PF); direct kernel: 2 |S| t per point against the FP64 vector peak;
-  bytes  = 16 x points (FP64 state read once and written once per block) against 8 TB/s;
+           2.5 PF); direct kernels: 2 |S| t per point against the FP64 vector peak;
+  bytes  = 16 x points (FP64 state read once and written once per launch) against 8 TB/s;
   frac   = the larger of the two fractions, `bound` names which.
-`run` beside it: what a whole run launches (the mixed 2D forms two blocks at once, 3D and 1D kernels of
-their own): launches, ms per launch, and the same 16 x points per launch against 8 TB/s.
+`block` beside it, where the run launches other kernels: the same for one fused block of the plan (ffs_run_block).
 Also: `matrix_frac_dense`, the dense count tiles x 8 d P^(d+1) per real tile (per-axis complex DFT
-GEMMs with real-pair packing; 1D prime-factor window 240 = 15 x 16: 8 x 240 x (15 + 16)), and
-`executed_mfma_tflops` (split products included).
+GEMMs with real-pair packing; 1D prime-factor window 240 = 15 x 16: 8 x 240 x (15 + 16); none for the banded
+product), and `executed_mfma_tflops` (split products included).
 
 Printed: one JSON line.  --gpus N > 1 exits: the library runs on one GPU.
 """
@@ -123,9 +123,15 @@ def roofline(info, kernel_s, form, radius, taps):
         flops = info["flops_per_block"] / products(form, info)
         dense = tile_flops(info) * info["tiles"]
         peak, unit_peak = MATRIX_PEAK[form], f"{form} matrix"
+    return fractions(flops, bytes_alg, kernel_s, peak, unit_peak, "mfma" if form != "direct" else "valu", dense,
+                     info["flops_per_block"] if form != "direct" else None)
+
+
+def fractions(flops, bytes_alg, kernel_s, peak, unit_peak, unit, dense, executed):
+    """Roofline object of a launch of kernel_s seconds; frac is the larger of the compute and the HBM fraction."""
     f_frac = flops / kernel_s / peak
     b_frac = bytes_alg / kernel_s / HBM_PEAK
-    out = {"executed_mfma_tflops": info["flops_per_block"] / kernel_s / 1e12 if form != "direct" else None,
+    out = {"executed_mfma_tflops": executed / kernel_s / 1e12 if executed else None,
            "flops_per_launch": flops, "dense_flops_per_launch": dense, "bytes_per_launch": bytes_alg,
            "kernel_ms": kernel_s * 1e3, "matrix_frac": f_frac,
            "matrix_frac_dense": dense / kernel_s / peak if dense else None, "hbm_frac": b_frac,
@@ -133,13 +139,49 @@ def roofline(info, kernel_s, form, radius, taps):
     if b_frac >= f_frac:
         out.update(bound="hbm", achieved=bytes_alg / kernel_s / 1e9, peak=HBM_PEAK / 1e9, unit="GB/s", frac=b_frac)
     else:
-        out.update(bound="mfma" if form != "direct" else "valu", achieved=flops / kernel_s / 1e12,
-                   peak=peak / 1e12, unit="TFLOP/s", frac=f_frac)
+        out.update(bound=unit, achieved=flops / kernel_s / 1e12, peak=peak / 1e12, unit="TFLOP/s", frac=f_frac)
+    return out
+
+
+RUN_KERNEL_NAMES = {0: "blocks", 1: "64-point windows", 2: "streamed planes", 3: "banded product"}
+
+
+def run_counts(info, form, radius):
+    """(flops with every real GEMM once, executed MFMA flops, dense flops or None) of one launch of a run that launches
+    a kernel of its own (info["run_kernel"] 1, 2 or 3), at the main depth."""
+    kind, depth, n = info["run_kernel"], info["run_depth"], info["sizes"]
+    if kind == 1:  # 16 + 16 + 16 + 8 products of 16 x 16 x 32 per 64-point window
+        v = 64 - 2 * radius * depth
+        windows = -(-n[0] // v) * -(-n[1] // v)
+        flops = windows * 56 * 2.0 * 16 * 16 * 32
+        dense = windows * 8.0 * 2 * 64 ** 3
+    elif kind == 2:  # 8 + 8 products of 16 x 16 x 16 per plane of a 32 x 32 window
+        v = 32 - 2 * radius * depth
+        windows = n[0] * -(-n[1] // v) * -(-n[2] // v)
+        flops = windows * 16 * 2.0 * 16 ** 3
+        dense = windows * 8.0 * 2 * 32 ** 3
+    else:  # 16 x k x 16 per 256 points, k = taps + 15 (executed: rounded up to blocks of 16 or 32)
+        tiles, k, block = -(-n[0] // 256), 2 * radius * depth + 16, 16 if form in ("fp64", "direct") else 32
+        flops = tiles * 2.0 * 256 * k
+        return flops, flops / k * (-(-k // block) * block) * PRODUCTS.get(form, 1), None
+    return flops, flops * PRODUCTS[form], dense
+
+
+def run_roofline(info, launch_s, form, radius, taps):
+    """Roofline object of one launch of the timed run (launch_s: run time / launches)."""
+    if info.get("run_kernel", 0) == 0:
+        out = roofline(info, launch_s, form, radius, taps)
+    else:
+        flops, executed, dense = run_counts(info, form, radius)
+        out = fractions(flops, 16.0 * float(np.prod(info["sizes"][:info["dims"]])), launch_s,
+                        MATRIX_PEAK["fp64" if form == "direct" else form], ("fp64" if form == "direct" else form) + " matrix",
+                        "mfma", dense, executed)
+    out.update(kernel=RUN_KERNEL_NAMES[info.get("run_kernel", 0)], launches=info["launches"])
     return out
 
 
 def traffic(workload, form):
-    """HBM bytes per launch of the dominant kernel from the committed rocprofv3 --pmc summary, if any."""
+    """HBM bytes per launch of the run's kernel from the committed rocprofv3 --pmc summary, if any."""
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
             return json.load(f).get(f"{workload}/{form}")
@@ -304,22 +346,21 @@ def bench_grid(name, args, torch, ffs, forms=None):
 
         kms, _ = timed(torch, one_block, 1, args.kernel_reps, stream, min_ms=5.0)
         del d_a, d_b
-        rl = roofline(info, kms * 1e-3, form, radius, taps)
+        rl = run_roofline(info, ms * 1e-3 / max(info["launches"], 1), form, radius, taps)
         rl["traffic"] = traffic(name, form)
         if rl["traffic"] is not None:
             rl["traffic_from"] = "profiles/traffic.json (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, copy-calibrated)"
-        launch_ms = ms / max(info["launches"], 1)
-        rl["run"] = {"launches": info["launches"], "launch_ms": launch_ms,
-                     "hbm_frac": 16.0 * npts / (launch_ms * 1e-3) / HBM_PEAK}
+        if info["run_kernel"] != 0:
+            rl["block"] = roofline(info, kms * 1e-3, form, radius, taps)
         gst = npts * T / (ms * 1e-3) / 1e9
         res[form] = dict(value=gst, ms_per_step=ms, timed_runs=reps, wall_s=wall, roofline=rl,
                          plan={k: info[k] for k in ("tile", "valid", "fuse", "fuse_tail", "blocks", "algorithm",
-                                                    "mapping")})
+                                                    "mapping", "run_kernel", "run_depth")})
         outputs[form] = d_out
-        log(f"{name} {form}: {gst:.1f} GStencil/s, {ms:.3f} ms/run, block {kms:.3f} ms, roofline {rl['bound']} "
-            f"{rl['frac']:.1%} (matrix {rl['matrix_frac']:.1%}, hbm {rl['hbm_frac']:.1%}), P={info['tile']} "
-            f"t={info['fuse']} V={info['valid']} blocks={info['blocks']}; run: {info['launches']} launches of "
-            f"{launch_ms:.3f} ms, hbm {rl['run']['hbm_frac']:.1%}")
+        log(f"{name} {form}: {gst:.1f} GStencil/s, {ms:.3f} ms/run, {info['launches']} launches ({rl['kernel']}, depth "
+            f"{info['run_depth']}) of {rl['kernel_ms']:.3f} ms, roofline {rl['bound']} {rl['frac']:.1%} (matrix "
+            f"{rl['matrix_frac']:.1%}, hbm {rl['hbm_frac']:.1%}); block {kms:.3f} ms, P={info['tile']} t={info['fuse']} "
+            f"V={info['valid']} blocks={info['blocks']}")
         plan.close()
     if "fp64" in outputs:
         ref64 = outputs["fp64"]
@@ -426,11 +467,14 @@ def bench_batch(args, torch, ffs, forms=None):
         for i in range(len(specs)):
             inf = batch.info(i)
             rounds = max(rounds, inf["launches"])
-            flops += inf["flops_per_block"] / products(form, inf) * inf["blocks"]
+            if inf["run_kernel"]:
+                flops += run_counts(inf, form, inf["radius"])[0] * inf["launches"]
+            else:
+                flops += inf["flops_per_block"] / products(form, inf) * inf["blocks"]
             bytes_alg += 16.0 * inf["sizes"][0] * inf["sizes"][1] * inf["launches"]
         s = ms * 1e-3
         f_frac, b_frac = flops / s / MATRIX_PEAK[form], bytes_alg / s / HBM_PEAK
-        rl = {"scope": f"whole run ({rounds} rounds); flops as of the blocks it stands for", "flops_per_run": flops,
+        rl = {"scope": f"whole run ({rounds} rounds)", "flops_per_run": flops,
               "bytes_per_run": bytes_alg, "matrix_frac": f_frac, "hbm_frac": b_frac, "traffic": None}
         if b_frac >= f_frac:
             rl.update(bound="hbm", achieved=bytes_alg / s / 1e9, peak=HBM_PEAK / 1e9, unit="GB/s", frac=b_frac)

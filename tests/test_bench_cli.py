@@ -71,3 +71,28 @@ def test_roofline_follows_algorithmic_counts():
     assert bench.roofline(info1, 20e-6, "fp64", 1, 3)["dense_flops_per_launch"] == 8 * 240 * 31 * 9363
     rld = bench.roofline(info, 0.36e-3, "direct", 2, 25)
     assert rld["flops_per_launch"] == 2 * 25 * 8192 * 8192 * 4 and rld["executed_mfma_tflops"] is None
+
+
+def test_run_roofline_counts_the_kernel_that_runs_launch():
+    sys.path.insert(0, ROOT)
+    import bench
+
+    # Box2D25P 8192^2, FP16, 64-point windows of depth 8 (V = 32): 65,536 windows of 56 products of 16 x 16 x 32
+    info = dict(dims=2, sizes=[8192, 8192, 1], tile=[32, 32, 1], tiles=512 * 512, fuse=4, flops_per_block=0.0, run_kernel=1,
+                run_depth=8, launches=32)
+    rl = bench.run_roofline(info, 0.336e-3, "f16", 2, 25)
+    assert rl["flops_per_launch"] == 65536 * 56 * 16384 and rl["kernel"] == "64-point windows" and rl["launches"] == 32
+    assert abs(rl["executed_mfma_tflops"] - 3 * 65536 * 56 * 16384 / 0.336e-3 / 1e12) < 1e-6
+    assert rl["bound"] == "hbm" and abs(rl["frac"] - 2 ** 30 / 0.336e-3 / 8e12) < 1e-6
+    # Box3D27P 512^3, FP64, streamed planes of depth 2 (V = 28): 16 products of 16^3 per plane and window
+    info3 = dict(info, dims=3, sizes=[512, 512, 512], run_kernel=2, run_depth=2, launches=16)
+    rl3 = bench.run_roofline(info3, 0.75e-3, "fp64", 1, 27)
+    assert rl3["flops_per_launch"] == 512 * 19 * 19 * 16 * 8192 and rl3["bound"] == "mfma"
+    # Heat-1D 2^20, depth 64: 4,096 tiles of a 16 x 144 x 16 product; the direct algorithm runs the same one
+    info1 = dict(info, dims=1, sizes=[1 << 20, 1, 1], run_kernel=3, run_depth=64, launches=1)
+    for form in ("fp64", "direct"):
+        rl1 = bench.run_roofline(info1, 9.0e-6, form, 1, 3)
+        assert rl1["flops_per_launch"] == 4096 * 2 * 256 * 144 and rl1["dense_flops_per_launch"] is None
+    # a run of blocks: as the block's roofline
+    blocks = dict(info, run_kernel=0, flops_per_block=2162688.0 * 131072, launches=64)
+    assert bench.run_roofline(blocks, 0.3657e-3, "f16", 2, 25)["frac"] == bench.roofline(blocks, 0.3657e-3, "f16", 2, 25)["frac"]
