@@ -2577,8 +2577,8 @@ __global__ void k_gen_operands_real(double* t) {
 // Entry order: FP64 32-point (P = 32, doubles), entry v * 64 + lane <-> (q + 4v, j); 64-point (P = 64, floats),
 // entry ((2 b0 + b1) * 4 + v) * 64 + lane <-> (2 (4q + v) + b0, 2j + b1).
 // The FP64 filter is formed in pairs of doubles: rounded as it went, a filter's low frequencies erred together (by the power
-// t), and with them every block by the same gain (Star2D9P, 25 blocks of t = 5: 3.3e-14 of the mean; in pairs 1.4e-15, which
-// is the transform matrices' rounding; complex transforms before 1.6e-14).  The 64-point filter is stored in FP32.
+// t), and with them every block by the same gain (Star2D9P, 25 blocks of t = 5: 3.3e-14 of the mean; in pairs and without the
+// matrices' own gain (kRealGain) 1e-15 and less).  The 64-point filter is stored in FP32.
 struct Pair {  // h + l, |l| <= ulp(h) / 2; sums by Knuth's two-sum, products by FMA
   double h, l;
   __device__ Pair(double x = 0.0) : h(x), l(0.0) {}
@@ -2596,8 +2596,12 @@ __device__ __forceinline__ Pair operator*(Pair a, Pair b) {
   const double p = a.h * b.h, e = __builtin_fma(a.h, b.h, -p) + (a.h * b.l + a.l * b.h), h = p + e;
   return Pair(h, e - (h - p));
 }
-__device__ __forceinline__ double to_double(Pair a) { return a.h; }
-__device__ __forceinline__ double to_double(double a) { return a; }
+// Filter values as they are stored.  FP64: the gain that the transforms' matrices have from their own rounding to doubles is
+// taken out (the constant field through the four stages in extended precision, mean over the valid region: 1.0e-16 to
+// 1.13e-16 for every stencil and depth).
+constexpr double kRealGain = 1.1e-16;
+__device__ __forceinline__ double stored(Pair a) { return (a * Pair(1.0, -kRealGain)).h; }
+__device__ __forceinline__ double stored(double a) { return a; }
 // Sum of w x.  Pairs: started from `big`, which no product exceeds, so s - acc is exact and the second FMA is what the
 // addition lost.
 template <typename T>
@@ -2697,7 +2701,7 @@ __global__ void k_gen_spectrum_real(Out* H, const double* taps, int32_t K, int32
   cpow_t(L1r, L1i, t);
   cpow_t(L2r, L2i, t);
   const double norm = ldexp(0.5 * 4.0 / ((double)P * (double)P), filter_exp);
-  const double h[4] = {to_double(L1r + L2r), to_double(L2r - L1r), to_double(L1i + L2i), to_double(L1i - L2i)};
+  const double h[4] = {stored(L1r + L2r), stored(L2r - L1r), stored(L1i + L2i), stored(L1i - L2i)};
   for (int i = 0; i < 4; i++) H[4 * e + i] = (Out)(h[i] * norm);
 }
 
@@ -3044,7 +3048,7 @@ __global__ __launch_bounds__(256, PREC == 0 ? 1 : 2) void k_stream3d(Stream3Args
 // axis-0 tap e <= 2 r t (zero above), as k_gen_spectrum_real forms them from the coefficients of z^e of
 // (sum_e0 z^e0 sum g[e0][e1][e2] exp(i (w1 e1 + w2 e2)))^t and its mirror (w2 -> -w2).  FP64 order (row q + 4v) or
 // FP32 order (row 4q + v).  Then the operands: 16 x 16 cosine and sine matrices, FP64 chunks or BF16 pairings.
-// FP64 in pairs of doubles, as the 2D filter (Heat-3D over 26 steps: gain of the mean off by 1.9e-15 in plain doubles).
+// FP64 in pairs of doubles, as the 2D filter (Heat-3D over 26 steps: mean off by 1.9e-15 in plain doubles, so 5e-16).
 constexpr int kStreamMaxE = 7;
 template <typename T, typename Out>
 __global__ void k_gen_stream3d(Out* H, int32_t E, const double* taps, int32_t K, int32_t convention, int32_t t, double big) {
@@ -3092,8 +3096,8 @@ __global__ void k_gen_stream3d(Out* H, int32_t E, const double* taps, int32_t K,
   }
   const double norm = 0.5 / 256.0;
   for (int e = 0; e < E; e++) {
-    const double h[4] = {to_double(L[0][0][e] + L[1][0][e]), to_double(L[1][0][e] - L[0][0][e]),
-                         to_double(L[0][1][e] + L[1][1][e]), to_double(L[0][1][e] - L[1][1][e])};
+    const double h[4] = {stored(L[0][0][e] + L[1][0][e]), stored(L[1][0][e] - L[0][0][e]),
+                         stored(L[0][1][e] + L[1][1][e]), stored(L[0][1][e] - L[1][1][e])};
     for (int i = 0; i < 4; i++) H[(e * 4 * kLanes + x) * 4 + i] = (Out)(h[i] * norm);
   }
 }

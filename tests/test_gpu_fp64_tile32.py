@@ -105,7 +105,8 @@ def test_2d_fp64_tile32_edges(ffs, oracle, torch_cuda, convention, radius, fuse,
 @pytest.mark.parametrize("shape,steps", [("Heat-2D", 82), ("Star2D9P", 5), ("Star2D9P", 125), ("Box2D9P", 64), ("Box2D25P", 125)])
 def test_2d_fp64_tile32_gain(ffs, torch_cuda, shape, steps):
     # The mean of the grid is multiplied by (sum w)^T.  Roundings of single outputs average out over 207,000 points; what is left
-    # is the gain error that every block shares, from the rounding of the transform matrices and the filter: below one ulp a block.
+    # is the gain error that every block shares, from the rounding of the transform matrices and the filter: below half an ulp a
+    # block.
     torch = torch_cuda
     _, r, w, _ = ffs.named_stencil(shape, seed=3)
     x = torch.rand((450, 460), dtype=torch.float64, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
@@ -116,4 +117,4 @@ def test_2d_fp64_tile32_gain(ffs, torch_cuda, shape, steps):
         launches = plan.info["launches"]
     want = x.cpu().numpy().astype(np.longdouble).mean() * np.asarray(w, dtype=np.longdouble).sum() ** steps
     got = y.cpu().numpy().astype(np.longdouble).mean()
-    assert abs(got / want - 1) <= 2 ** -52 * launches, (float(got / want - 1), launches)
+    assert abs(got / want - 1) <= 2 ** -53 * launches, (float(got / want - 1), launches)

@@ -302,6 +302,16 @@ def halves(words, f16):
     return w.astype(np.uint16).view(np.float16).astype(LD) if f16 else (w << 16).view(np.float32).astype(LD)
 
 
+def _matrix_gain():
+    """The FP64 filters take out the gain of the matrices' rounding to doubles: a constant window through the rounded
+    sine matrix and back, mean over the near half, both axes; the kernels' constant is 1.1e-16."""
+    sine = trig(16, 32)[1].astype(np.float64).astype(LD)
+    gain = float((sine.T @ (sine @ np.full(16, LD(2))) / 16).mean() - 1)
+    assert abs(2 * gain - 1.1e-16) < 2e-17, gain
+    return 1 - LD(1.1e-16)
+
+
+MATRIX_GAIN = _matrix_gain()
 LANES = np.arange(64)
 Q, J = LANES // 16, LANES % 16
 
@@ -322,7 +332,7 @@ def test_real_tables_32_fp64(ffs, torch_cuda, convention, radius, fuse, tail):
     assert filt.size == 1024 * len(depths)
     for got, t in zip(filt.reshape(-1, 4, 64, 4), depths):
         for v in range(4):  # entry v * 64 + lane: (k0, k1) = (q + 4 v, j)
-            want = real_filter(*half_sample_gain(w, K, convention, Q + 4 * v, J, 32, t), 32)
+            want = MATRIX_GAIN * real_filter(*half_sample_gain(w, K, convention, Q + 4 * v, J, 32, t), 32)
             assert np.abs(got[v] - want).max() <= 2.0 ** -53 * np.abs(want).max()  # |entries| <= 2^-8 or so, rounded once
 
 
@@ -408,7 +418,7 @@ def test_stream_tables(ffs, torch_cuda, convention, form, radius, sizes, steps):
                                 nxt[i + a] += poly[s][i] * one[s][a]
                     poly[s] = nxt
             for e in range(E):
-                want = real_filter(poly[0][e], poly[1][e], 32)
+                want = real_filter(poly[0][e], poly[1][e], 32) * (MATRIX_GAIN if form == "fp64" else 1)
                 assert np.abs(got[e, v] - want).max() <= (2.0 ** -52 if form == "fp64" else 2.0 ** -24) * np.abs(want).max() + 1e-300
 
 
