@@ -1727,21 +1727,23 @@ struct Plane64 {
 };
 
 // Folded window relative to its plane: z[b][C] = rows near - far, z[2 + b][C] = near + far, differences taken in FP64.
-// The plane is read off 8 rows spread over the window (0, 8, 16, 24, 39, 47, 55, 63): their mean, and the slopes that the
-// means of the near and the far halves differ by (39 rows and 32 columns apart; symmetrical about the centre, so a
-// plane is recovered exactly).  A constant left in the window is one term of a cyclic transform but a whole series of a
-// negacyclic one, each term of which rounds (with the centre sample, as in the 32-point kernels, the FP16 form's
-// relative error on Box2D25P 8192^2 x 32 was 3.7e-8 instead of 5.9e-9), and a slope left in it is twice as large as in a
+// The plane is read off 16 rows spread over the window (0, 4, .. 28 and 35, 39, .. 63): their mean, and the slopes that the
+// means of the near and the far halves differ by (35 rows and 32 columns apart; symmetrical about the centre, so a
+// plane is recovered exactly; 8 rows gave noise fields 5 to 10% more error for 0.5% of the time).  A constant left in the
+// window is one term of a cyclic transform but a whole series of a negacyclic one, each term of which rounds (with the
+// centre sample, as in the 32-point kernels, the FP16 form's relative error on Box2D25P 8192^2 x 32 was 3.7e-8 instead of
+// 5.9e-9 with a mean, now 2.7e-9 at x 256), and a slope left in it is twice as large as in a
 // 32-point window: on waves of 200 to 1500 points the l2 error was 1.2 to 1.5 times that of the two 32-point blocks
 // with the mean alone, 0.7 to 0.9 times with the plane (geometric means, 120 random cases).  It costs 48 FP64 operations
-// and 16 of the reduction per lane and window: 332 -> 344 us (FP16), 451 -> 458 us (BF16) per launch on Box2D25P 8192^2.
+// and some 30 of the reduction per lane and window: 332 -> 346 us (FP16), 451 -> 460 us (BF16) per launch on Box2D25P 8192^2.
 __device__ __forceinline__ Plane64 fold64(const Raw64& r, Tile16& z) {
-  const d2u nn = r.g[0][0], nf = r.g[0][1], fn = r.g[0][2], ff = r.g[0][3];  // [row half][column half]
+  // [row half][column half]
+  const d2u nn = r.g[0][0] + r.g[2][0], nf = r.g[0][1] + r.g[2][1], fn = r.g[0][2] + r.g[2][2], ff = r.g[0][3] + r.g[2][3];
   const double sn = nn[0] + nn[1], snf = nf[0] + nf[1], sfn = fn[0] + fn[1], sff = ff[0] + ff[1];
   const double near = sn + snf, far = sfn + sff;
   const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
   double all = near + far, rows = far - near, cols = (snf + sff) - (sn + sfn);
-  wave_sum3(all, rows, cols, 1.0 / 512, 1.0 / (256 * 39), 1.0 / (256 * 32), lane);
+  wave_sum3(all, rows, cols, 1.0 / 1024, 1.0 / (512 * 35), 1.0 / (512 * 32), lane);
   const Plane64 p = {all, rows, cols};
   const double two = p.c + p.c, e0 = p.s1 * (double)(4 * j - 63), e1 = e0 + (p.s1 + p.s1);
   const double sum[4] = {two + e0, two + e1, two - e0, two - e1};  // columns 2j, 2j + 1, 63 - 2j, 62 - 2j
