@@ -529,7 +529,7 @@ ffs_status choose_config(ffs_plan* pl) {
   }
   // Two blocks per launch on 64-point windows wherever the valid region of the doubled tile still fits the
   // near half of the window (2V <= 32; beyond it the inverse stages would need both halves) and there are
-  // two blocks to take: Box2D25P 8192^2, two t = 4 blocks 684 us, one 64-point launch 337 us (FP16; BF16 1000 and 445).
+  // two blocks to take: Box2D25P 8192^2, two t = 4 blocks 684 us, one 64-point launch 346 us (FP16; BF16 1000 and 460).
   pl->wide = pl->kind == ffsk::KIND_2D32 && p.precision != FFS_PREC_FP64 && pl->V[0] <= 16 && pl->nblocks >= 2 &&
              depth_in_range(pl, 2 * pl->t);
   if (pl->wide) pl->t_wide_tail = p.steps % (2 * pl->t);

@@ -1117,7 +1117,9 @@ __device__ __forceinline__ void store16(const TileArgs& a, const PairCoord& pc, 
 
 // One tile pair of the 32-point family.  The spectrum comes from LDS (single-grid launch) or from the
 // grid's FP64 table in global memory (batch launch, where every grid has its own stencil and depth).
-template <int NTERMS, bool H_FROM_LDS, bool OUT16, int IKBS = 1>  // IKBS as for tile32_pair_f64
+// IKBS: column blocks per chunk of the inverse-operand table sG (1: the shifted one-block table; 2: the forward operands,
+// read through a shifted_view whose lane is `ilane`).
+template <int NTERMS, bool H_FROM_LDS, bool OUT16, int IKBS = 1>
 __device__ __forceinline__ void tile32_pair(const TileArgs& a, int64_t tp, const u4* __restrict__ sF,
                                             const f2* __restrict__ sH, const u4* __restrict__ sG, int lane, int q,
                                             int j, int ilane = -1) {
@@ -1304,7 +1306,7 @@ __device__ __forceinline__ void stage32_f16(const Blk4& zr, const Blk4& zi, cons
   }
 }
 
-template <bool H_FROM_LDS, bool OUT16, int IKBS = 1>  // IKBS as for tile32_pair_f64
+template <bool H_FROM_LDS, bool OUT16, int IKBS = 1>  // IKBS as for tile32_pair
 __device__ __forceinline__ void tile32_pair_f16(const TileArgs& a, int64_t tp, const u4* __restrict__ sF,
                                                 const f2* __restrict__ sH, const u4* __restrict__ sG, int lane,
                                                 int q, int j, int ilane = -1) {
@@ -1642,9 +1644,9 @@ __device__ __forceinline__ double dpp_shl1(double x) {
   return __builtin_bit_cast(double, (uint64_t)a | ((uint64_t)b << 32));
 }
 
-// kx, ky, kz times the sums of x, y and z over the wave, as wave-uniform values (scalar registers).  The three share the lanes from the first exchange on (lane 4k carries
-// x, 4k + 1 y, 4k + 2 z), so they cost five exchanges inside the rows and two across them instead of three times four
-// and three times three row sums.
+// kx, ky, kz times the sums of x, y and z over the wave, as wave-uniform values (scalar registers).  The three share the
+// lanes from the first exchange on (lane 4k carries x, 4k + 1 y, 4k + 2 z), so they cost five exchanges inside the rows
+// and two across them instead of three times four and three times three row sums.
 template <int CTRL>
 __device__ __forceinline__ double dpp_get(double x) {
   const uint64_t w = __builtin_bit_cast(uint64_t, x);
@@ -1798,8 +1800,9 @@ __device__ __forceinline__ void store64(const TileArgs& a, const TilePos& p, int
 //
 // What bounds it (Box2D25P 8192^2, depth 8, one launch): gather and store alone take 264 us (1.07 GB, 200 us at
 // the copy rate), the stages and the store alone 226 us; without the requests ahead the two followed each
-// other (450 us at 2 waves per SIMD), with them the launch takes 337 us (FP16; BF16 451), against 684 (1000)
-// for the two 32-point blocks it replaces.  232 VGPRs, 2 waves per SIMD; at 3 the raw window spills (711 us).
+// other (450 us at 2 waves per SIMD), with them the launch takes 337 us (FP16; BF16 451; with the fitted plane 346 and
+// 460), against 684 (1000) for the two 32-point blocks it replaces.  242 VGPRs, 2 waves per SIMD; at 3 the raw window
+// spills (711 us).
 template <int PREC>
 __device__ __forceinline__ void tile64(const TileArgs& a, const TilePos& p, const u4* __restrict__ sW,
                                        const f4* __restrict__ H, int lane, int q, int j, const Win64& cur, Raw64& raw,
@@ -3173,8 +3176,8 @@ hipError_t launch_stream3d(const Stream3Args& a, int32_t precision, int32_t E, h
 // ordered so that a lane ends with 4 consecutive outputs.
 //
 // FP64 is bound by the matrix pipe (64 cycles per chunk; two tiles per wave, which halve the LDS reads, were 2%
-// slower), BF16 by HBM at the depths it takes (2rt up to 304) with LDS reads close behind.  Heat-1D 2^20 x 64
-// FP64 14.7 -> 10 us, 2^24 x 256 787 -> 320; 1D7P 2^24 x 100 FP64 954 -> 369, BF16 770 -> 184 us.
+// slower), BF16 by HBM at the depths it takes (2rt up to 304) with LDS reads close behind.  Against the 240-point windows:
+// Heat-1D 2^20 x 64 FP64 14.7 -> 9.4 us, 2^24 x 256 787 -> 320; 1D7P 2^24 x 100 FP64 954 -> 351, BF16 781 -> 147 us.
 // ---------------------------------------------------------------------------------------------
 // FP64: taps in LDS (zero-padded on both sides), operands of both sides read per K = 4 chunk; the window with one
 // pad per 16 values (the column stride).
@@ -3447,8 +3450,8 @@ hipError_t launch_line(const LineArgs& a, int32_t precision, hipStream_t s, int 
     else
       hipLaunchKernelGGL(k_line_f64<false>, g, b, lds, s, a);
   } else if (a.n > 4096 * (int64_t)num_cus * 4) {
-    // Two tiles per wave share the operand reads (1D7P 2^24 x 100, before the requests ahead: 184 us, one tile 207, four 209) once every SIMD
-    // has eight such waves; below that one tile per wave keeps its chain short (2,000,000 x 64: 39.8 against 40.6).
+    // Two tiles per wave share the operand reads (1D7P 2^24 x 100, before the requests ahead: 184 us, one tile 207,
+    // four 209) once every SIMD has eight such waves; below that one tile per wave keeps its chain short (2,000,000 x 64: 39.8 against 40.6).
     launch_line_bf16<2>(a, s, num_cus);
   } else {
     launch_line_bf16<1>(a, s, num_cus);
